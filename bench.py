@@ -431,7 +431,7 @@ def main():
                     help="steps of the one-thread CPU oracle sample (0 = skip)")
     ap.add_argument("--no-graph", action="store_true")
     ap.add_argument("--layout", type=int, default=-1,
-                    help="stage-kernel layout of the main workload (-1: the autotuner picks)")
+                    help="stage-kernel layout of the main workload (-1: the default)")
     ap.add_argument("--batched-steps", type=int, default=50,
                     help="steps of the batched-cavity speedup measurement (0 = skip)")
     ap.add_argument("--batched-only", action="store_true")
@@ -485,7 +485,7 @@ def main():
     solver.step(dt, args.warmup)
     solver.sync()
     layout = solver.layout()
-    print(f"[bench] stage layout (autotuned) {layout}", file=sys.stderr, flush=True)
+    print(f"[bench] stage layout {layout}", file=sys.stderr, flush=True)
     timer = StreamTimer(solver.stream())
     solver.sync()
     w0 = time.perf_counter()
@@ -574,7 +574,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": traffic_src,
-                     "kernel": "nkc::stage_kernel (fused stage)",
+                     "kernel": "nkc::box_kernel (fused stage)",
                      "avg_launch_us": avg_launch_s * 1e6,
                      "alg_bytes_per_launch": alg_bytes, "alg_bytes_per_unit": B_ALG,
                      "moved_bytes_per_unit": B_MOVED, "achieved_moved": moved,

@@ -386,30 +386,20 @@ int32_t nkc_info(nkc_handle *h, int64_t out[8]);
 /* Enable (1, default) or disable (0) hipGraph replay in nkc_step. */
 int32_t nkc_set_graph(nkc_handle *h, int32_t enable);
 
-/* Stage-kernel layout (no counterpart in the reference).  Layouts 0..3
- * take one element per workgroup.  Bit 0: the four lane roles of an
- * element get whole waves each (0) or their (N+1)^2 lanes packed back to
- * back in fewer waves (1).  Bit 1: the register allocator is left free (0)
- * or held to 128 VGPRs for 4 waves per SIMD (1).  Layouts 4 and 5 take two
- * elements per workgroup, packed, with the free / 128-VGPR register budget;
- * they are built for N <= 5 only.  Layouts 6 and 7 split an element six
- * ways (the two update groups x three runs of levels, packed; every lane
- * forms one face flux), with the free / occupancy-bound register budget;
- * they are built for N >= 7 and carry sources, Drude and Lorentz regions
- * but no PML, incident field or graphene sheet (nkc_set_layout refuses
- * them on such a handle with NKC_ERR_UNSUPPORTED, and the tuner does not
- * time them there).  The first nkc_step times the layouts on
- * the handle's mesh and keeps the fastest (an autotuner; a packed
- * one-element layout with the same workgroup as the unpacked one, and a
- * layout not built for the order, are not timed).  nkc_set_layout forces
- * 0..NKC_NLAYOUT-1 (one built for the order), or -1 to tune again at the
- * next step; nkc_tune tunes now: out[NKC_NLAYOUT + 1] = {us per stage for
- * each layout (NaN: not timed), chosen layout} (out may be NULL).  All
- * layouts compute the same arithmetic: results are bit-identical. */
+/* Stage-kernel layouts (no counterpart in the reference): numbers a caller
+ * may name.  0..3 are accepted at every order, 4 and 5 at N <= 5, 6 and 7 at
+ * N >= 7 (there not with a PML, an incident field or a graphene sheet:
+ * NKC_ERR_UNSUPPORTED); a number not accepted at the order is NKC_ERR_ARG.
+ * Every order has one stage kernel, whose shape suits it, and every accepted
+ * number names it: results do not depend on the layout, and stepping needs
+ * no tuning.  nkc_set_layout names 0..NKC_NLAYOUT-1, or -1 (the next step
+ * takes 0); nkc_tune times the stage on the handle's mesh:
+ * out[NKC_NLAYOUT + 1] = {us per stage for each layout accepted (NaN: not
+ * accepted), chosen layout} (out may be NULL). */
 #define NKC_NLAYOUT 8
 int32_t nkc_set_layout(nkc_handle *h, int32_t layout);
 int32_t nkc_tune(nkc_handle *h, double *out);
-/* The current layout and the last tuner times without tuning:
+/* The current layout and the last times of nkc_tune without timing:
  * out[NKC_NLAYOUT + 1] as for nkc_tune (layout -1 before the first step). */
 int32_t nkc_get_layout(nkc_handle *h, double *out);
 
@@ -436,7 +426,7 @@ int32_t nkc_batch_stream(nkc_batch *b, void **stream);
 /* out[0] = total points, out[1] = cavities, out[2] = polynomial orders
  * (launches per stage), out[3] = total elements. */
 int32_t nkc_batch_info(nkc_batch *b, int64_t out[8]);
-/* Per polynomial order of the batch (tuned at its first step, -1 before):
+/* Per polynomial order of the batch (-1 before its first step):
  * out[2 i] = N, out[2 i + 1] = stage-kernel layout; cap = ints in out. */
 int32_t nkc_batch_layout(nkc_batch *b, int32_t *out, int64_t cap);
 

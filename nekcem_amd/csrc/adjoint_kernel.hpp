@@ -1,6 +1,6 @@
 // adjoint_kernel.hpp -- one reversed RK stage of the discrete adjoint.
 //
-// Forward stage i (stage_kernel.hpp): r = P B(u) + P s, k <- a_i k + dt r,
+// Forward stage i (box_kernel.hpp): r = P B(u) + P s, k <- a_i k + dt r,
 // u <- u + b_i k, with P = diag(1/mu, 1/eps) per node, B the strong-form DG
 // operator (volume curl + lifted upwind/central flux) and s the source.
 // Reversing it, with lambda the adjoint of u and kappa the adjoint of k:
@@ -16,9 +16,31 @@
 // flux of its face: its own flux and the neighbour's flux on the shared face,
 // so every output has a single owner (no atomics).
 #pragma once
-#include "stage_kernel.hpp"
+#include "stage_args.hpp"
 
 namespace nkc {
+
+// Whether the reversed stage's outputs and residual stream past L2: at N = 7 a
+// role's level is 64 doubles, whole cache lines from one wave; at the other
+// orders a level straddles lines and the plain forms are faster.
+template <int N1>
+constexpr bool nt_streams() { return N1 == 8; }
+
+// Four roles of (N+1)^2 lanes padded to whole waves: role & 1 selects the
+// update group (0: H, 1: E), role >> 1 the half of the levels; LDS as
+// u(i,j,k) of field f at f*N3 + idx, XOR-swizzled for power-of-two N1.
+template <int N1>
+struct Shape {
+    static constexpr int N2 = N1 * N1, N3 = N2 * N1;
+    static constexpr int ROLES = 4;
+    static constexpr int LANES = ((N2 + 63) / 64) * 64;
+    static constexpr int BS = LANES * ROLES;
+    static constexpr int KH = (N1 + 1) / 2;           // levels in the lower half
+    static constexpr bool SWZ = (N1 & (N1 - 1)) == 0;
+    __device__ static __forceinline__ int idx(int i, int j, int k) {
+        return (SWZ ? (i ^ j) : i) + N1 * j + N2 * k;
+    }
+};
 
 struct AdjArgs {
     const double *__restrict__ lam_in;  // 6 fields, stride fs

@@ -1,7 +1,7 @@
 // geo_kernel.hpp -- the RK stage on general hexahedra (curved, rotated,
 // sheared elements; any conforming face pairing), for gfx950.
 //
-// The same stage as stage_kernel.hpp (cem_maxwell_op + rk_maxwell_ab,
+// The same stage as box_kernel.hpp (cem_maxwell_op + rk_maxwell_ab,
 // src/cem_maxwell.F:484-508, 1906-1968), with the geometry per node instead
 // of per element: maxwell_wght_curl's full cofactor combine
 // (src/cem_maxwell.F:1464-1495) in strong form, curl u = sum_a G_a x du/dr_a
@@ -21,7 +21,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "stage_kernel.hpp"
+#include "stage_args.hpp"
 
 namespace nkc {
 

@@ -35,7 +35,7 @@
 
 namespace nkc {
 
-// FaceType codes live in stage_kernel.hpp: -1 PEC, -2 no partner.
+// FaceType codes live in stage_args.hpp: -1 PEC, -2 no partner.
 constexpr int32_t HOST_FACE_PEC = -1;
 constexpr int32_t HOST_FACE_NONE = -2;
 

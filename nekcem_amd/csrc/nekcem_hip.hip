@@ -28,7 +28,6 @@
 #include "mesh_tables.hpp"
 #include "order_launch.hpp"
 #include "restart_io.hpp"
-#include "stage_kernel.hpp"
 
 using namespace nkc;
 
@@ -105,7 +104,8 @@ struct DevMesh {
     double *D = nullptr, *geo = nullptr, *fco = nullptr, *ieps = nullptr, *imu = nullptr;
     double *dt_e = nullptr;       // per-element dt (batches), or null
     int32_t *nbr = nullptr;
-    int layout = -1;              // stage-kernel layout (PACK | OCC << 1); -1: not tuned yet
+    int layout = -1;              // stage-kernel layout named by the caller or the tuner; -1: none yet
+    bool nt = false;              // k and the outputs past the caches (stage_nt)
     std::vector<int32_t> xcd_lo;  // 9 element bounds of equal-work XCD ranges, or empty
     std::vector<double> jac, w;   // host copies (source weights)
     // general hexahedra (geo_kernel.hpp): per-node metric quotients and
@@ -115,12 +115,21 @@ struct DevMesh {
     int32_t *fnb = nullptr;
 };
 
+// Whether a stage streams k and its outputs past the caches (non-temporal):
+// once u, k and the output no longer fit the 256 MB Infinity Cache together.
+// Per stage, plain / non-temporal: N = 5 at 18^3 (181 MB) 39.1 / 47.2 us, at
+// 25^3 (486 MB) 137.7 / 121.6; N = 7 at 12^3 (127 MB) 32.2 / 33.8, at 18^3
+// (430 MB) 109.4 / 103.4; N = 8 at 12^3 (181 MB) 45.2 / 49.9, at 16^3 (430
+// MB) 116.9 / 110.0.
+bool stage_nt(int64_t npts) { return 18.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
+
 int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     dm.n1 = m.n1;
     dm.mat = m.mat ? MAT_NODE : MAT_ELEM;
     dm.nelt = m.nelt;
     dm.npts = m.nelt * m.n1 * m.n1 * m.n1;
     dm.fs = (dm.npts + 31) / 32 * 32;
+    dm.nt = stage_nt(dm.npts);
     dm.jac = m.jac;
     dm.w = m.w;
     const size_t ub = sizeof(double) * 6 * (size_t)dm.fs;
@@ -156,12 +165,8 @@ void dev_mesh_free(DevMesh &dm) {
     dm = DevMesh();
 }
 
-// Stage-kernel layouts: 0..3 one element per workgroup, bit 0 = PACK (lane
-// roles packed), bit 1 = OCC (4 waves/SIMD register budget); 4, 5 two
-// elements per workgroup, packed, without / with the OCC budget (N <= 5
-// only); 6, 7 the six-role kernel without / with the budget of its
-// LDS-bound occupancy (N >= 7 only; no PML, incident field or graphene
-// sheet).  The residual test entry uses layout 0.
+// Stage-kernel layouts: numbers a caller may name, per order; all of them
+// are the one kernel of that order (box_kernel.hpp).
 constexpr int NLAYOUT = NKC_NLAYOUT;
 
 // Work of a Drude element's stage relative to a plain one, for the XCD split
@@ -169,28 +174,30 @@ constexpr int NLAYOUT = NKC_NLAYOUT;
 // N = 9, 24^3, a workgroup's life ~1.6 times the others').
 constexpr double DRUDE_WORK = 1.6;
 
-// Elements per workgroup of a layout.
-int layout_epw(int layout) { return (layout == 4 || layout == 5) ? 2 : 1; }
-
-// Whether a layout is built for this order.
+// Whether a layout number names a kernel at this order.
 bool layout_built(int n1, int layout) {
     if (layout < 4) return true;
-    if (layout < 6) return n1 <= EPW_MAX_N1;
-    return n1 >= S6_MIN_N1;
+    if (layout < 6) return n1 <= 6;
+    return n1 >= 8;
 }
 
-// Whether a built layout carries the physics of these stage arguments (the
-// six-role kernel has no PML, incident field or graphene sheet).
+// Whether a layout may be named with the physics of these stage arguments
+// (6 and 7: no PML, incident field or graphene sheet).
 bool layout_runs(int n1, int layout, const StageArgs &a) {
     return layout_built(n1, layout) && !(layout >= 6 && (a.pml_off || a.inc_mask || a.gr_off));
 }
 
-// Lanes a workgroup of the given layout has.
-int stage_block(int n1, int layout) {
-    const int n2 = n1 * n1;
-    if (layout >= 6) return (6 * n2 + 63) / 64 * 64;
-    const int one = (layout & 1) ? (4 * n2 + 63) / 64 * 64 : 4 * ((n2 + 63) / 64 * 64);
-    return one * layout_epw(layout);
+// Lanes of a stage workgroup, and its LDS.
+int stage_block(int n1) {
+    switch (n1) {
+    case 4: return BoxShape<4>::BS;
+    case 5: return BoxShape<5>::BS;
+    case 6: return BoxShape<6>::BS;
+    case 7: return BoxShape<7>::BS;
+    case 8: return BoxShape<8>::BS;
+    case 9: return BoxShape<9>::BS;
+    default: return BoxShape<10>::BS;
+    }
 }
 
 }  // namespace
@@ -230,20 +237,15 @@ int32_t launch_geo_stage(const DevMesh &dm, const StageArgs &a, int gmode, hipSt
     return NKC_OK;
 }
 
-int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_t s, int layout = -2) {
+int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_t s) {
     if (dm.general) return launch_geo_stage(dm, a, mode == MODE_RK ? GMODE_RK : GMODE_RESIDUAL, s);
-    const int pk0 = layout == -2 ? (dm.layout < 0 ? 0 : dm.layout) : layout;
-    // the residual entry and orders without the layout run layout 0
-    const int pk = (mode == MODE_RK && layout_runs(dm.n1, pk0, a)) ? pk0 : 0;
-    const int64_t nwg = (dm.nelt + layout_epw(pk) - 1) / layout_epw(pk);
-    const int per_xcd = (int)((nwg + 7) / 8);
     StageArgs b = a;
-    b.per_xcd = per_xcd;
-    int grid = 8 * per_xcd;
+    b.per_xcd = (int)((dm.nelt + 7) / 8);
+    int grid = 8 * b.per_xcd;
     b.xcd_bal = 0;
     // the equal-work ranges: instances with in-stage physics only (a Drude
-    // region sets them), one element per workgroup
-    if (dm.xcd_lo.size() == 9 && layout_epw(pk) == 1 && (a.src_off || a.drude_off || a.lor_off || a.pml_off || a.inc_mask || a.gr_off)) {
+    // region sets them)
+    if (dm.xcd_lo.size() == 9 && (a.src_off || a.drude_off || a.lor_off || a.pml_off || a.inc_mask || a.gr_off)) {
         int len = 0;
         for (int x = 0; x < 8; ++x) {
             b.xcd_lo[x] = dm.xcd_lo[x];
@@ -254,13 +256,13 @@ int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_
         grid = 8 * std::max(len, 1);
     }
     switch (dm.n1) {
-    case 4: launch_stage_n4(b, dm.mat, mode, pk, grid, s); break;
-    case 5: launch_stage_n5(b, dm.mat, mode, pk, grid, s); break;
-    case 6: launch_stage_n6(b, dm.mat, mode, pk, grid, s); break;
-    case 7: launch_stage_n7(b, dm.mat, mode, pk, grid, s); break;
-    case 8: launch_stage_n8(b, dm.mat, mode, pk, grid, s); break;
-    case 9: launch_stage_n9(b, dm.mat, mode, pk, grid, s); break;
-    case 10: launch_stage_n10(b, dm.mat, mode, pk, grid, s); break;
+    case 4: launch_stage_n4(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 5: launch_stage_n5(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 6: launch_stage_n6(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 7: launch_stage_n7(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 8: launch_stage_n8(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 9: launch_stage_n9(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 10: launch_stage_n10(b, dm.mat, mode, dm.nt, grid, s); break;
     default: return fail(NKC_ERR_UNSUPPORTED, "polynomial order N=%d not built", dm.n1 - 1);
     }
     HIPCHK(hipGetLastError());
@@ -288,15 +290,15 @@ int32_t stage_kflags(int s) {
     return (s == 0 ? 0 : 1) | (s == 4 ? 0 : 2);
 }
 
-// Autotuner over the stage kernel's layouts (lane packing x register
-// budget): time each on this mesh, alternating, best of three rounds of
-// four launches, and keep the fastest.  It writes only a scratch output and
-// a scratch RK register, and with the handle's source, Drude, Lorentz, PML,
-// incident-field and graphene-sheet set-up (feat, may be null) it times the kernel
-// instance the step runs, the auxiliary fields and their registers
-// redirected to scratch: the state is untouched.  A packed layout whose
-// workgroup equals the unpacked one is not timed.  jsz, lsz, psz, gsz:
-// doubles of the Drude / Lorentz / PML / graphene-sheet state blocks.
+// Time of a stage on this mesh: best of three rounds of four launches.  It
+// writes only a scratch output and a scratch RK register, and with the
+// handle's source, Drude, Lorentz, PML, incident-field and graphene-sheet
+// set-up (feat, may be null) it times the kernel instance the step runs, the
+// auxiliary fields and their registers redirected to scratch: the state is
+// untouched.  Every layout number the order accepts with this physics names
+// that kernel: us holds its time for each of them (NaN for the others).
+// jsz, lsz, psz, gsz: doubles of the Drude / Lorentz / PML / graphene-sheet
+// state blocks.
 int32_t tune_stage(DevMesh &dm, const StageArgs *feat, size_t jsz, size_t lsz, size_t psz, size_t gsz,
                    const double *uin, hipStream_t s, double us[NLAYOUT]) {
     for (int l = 0; l < NLAYOUT; ++l) us[l] = NAN;
@@ -304,12 +306,6 @@ int32_t tune_stage(DevMesh &dm, const StageArgs *feat, size_t jsz, size_t lsz, s
         dm.layout = 0;            // the general kernel has one layout
         return NKC_OK;
     }
-    // not timed: a layout not built for this order, and a packed one-element
-    // layout whose workgroup equals its unpacked twin
-    auto skip = [&](int p) {
-        return !layout_built(dm.n1, p) || (p < 4 && (p & 1) && stage_block(dm.n1, p) == stage_block(dm.n1, p - 1)) ||
-               (p >= 6 && feat && (feat->pml_off || feat->inc_mask || feat->gr_off));
-    };
     const size_t blk = 6 * (size_t)dm.fs;
     const size_t jx = (feat && feat->drude_off) ? jsz : 0;
     const size_t lx = (feat && feat->lor_off) ? lsz : 0;
@@ -320,15 +316,10 @@ int32_t tune_stage(DevMesh &dm, const StageArgs *feat, size_t jsz, size_t lsz, s
     if (rc) return rc;
     StageArgs a = mesh_args(dm);
     if (feat) {
-        a.tdev = feat->tdev;
+        a.tst = feat->tst;
         a.src_off = feat->src_off;
         a.src_amp = feat->src_amp;
         for (int c = 0; c < 3; ++c) a.src_dir[c] = feat->src_dir[c];
-        a.src_t0 = feat->src_t0;
-        a.src_tw = feat->src_tw;
-        a.src_kind = feat->src_kind;
-        a.src_om = feat->src_om;
-        a.src_ph = feat->src_ph;
         a.inc_mask = feat->inc_mask;
         a.xyz = feat->xyz;
         for (int c = 0; c < 3; ++c) {
@@ -370,42 +361,69 @@ int32_t tune_stage(DevMesh &dm, const StageArgs *feat, size_t jsz, size_t lsz, s
     a.rkb = RK4B[0];
     a.dt = 1e-3;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    float best[NLAYOUT];
-    for (int l = 0; l < NLAYOUT; ++l) best[l] = INFINITY;
+    float best = INFINITY;
     rc = NKC_OK;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) rc = fail(NKC_ERR_HIP, "hipEventCreate");
-    for (int round = 0; round < 3 && rc == NKC_OK; ++round)
-        for (int p = 0; p < NLAYOUT && rc == NKC_OK; ++p) {
-            if (skip(p)) continue;
-            if ((rc = launch_stage(dm, a, MODE_RK, s, p))) break;
-            if (hipEventRecord(e0, s) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipEventRecord"); break; }
-            for (int r = 0; r < 4 && rc == NKC_OK; ++r) rc = launch_stage(dm, a, MODE_RK, s, p);
-            if (rc) break;
-            float ms = 0.0f;
-            if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = fail(NKC_ERR_HIP, "tuner timing");
-                break;
-            }
-            best[p] = std::min(best[p], ms / 4.0f);
+    for (int round = 0; round < 3 && rc == NKC_OK; ++round) {
+        if ((rc = launch_stage(dm, a, MODE_RK, s))) break;
+        if (hipEventRecord(e0, s) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipEventRecord"); break; }
+        for (int r = 0; r < 4 && rc == NKC_OK; ++r) rc = launch_stage(dm, a, MODE_RK, s);
+        if (rc) break;
+        float ms = 0.0f;
+        if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+            hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
+            rc = fail(NKC_ERR_HIP, "tuner timing");
+            break;
         }
+        best = std::min(best, ms / 4.0f);
+    }
     (void)hipStreamSynchronize(s);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     (void)hipFree(scr);
     if (rc) return rc;
-    int pick = 0;
-    for (int l = 0; l < NLAYOUT; ++l) {
-        if (std::isfinite(best[l])) us[l] = 1e3 * best[l];
-        if (best[l] < best[pick]) pick = l;
-    }
-    dm.layout = pick;
+    for (int l = 0; l < NLAYOUT; ++l)
+        if (layout_runs(dm.n1, l, a)) us[l] = 1e3 * best;
+    dm.layout = 0;
     return NKC_OK;
 }
 
-// time = time + dt at the end of a step (src/cem_drive.F:639), on the device
-// so a replayed graph sees the right stage times.
-__global__ void advance_time(double *t, double dt) { t[0] = t[0] + dt; }
+// The source's time factor: g(t) = exp(-((t-t0)/tw)^2) (kind 0) or
+// sin(om t + ph) (kind 1).
+struct SrcTime {
+    int32_t kind;
+    double t0, tw, om, ph;
+};
+__device__ double src_factor(const SrcTime &s, double t) {
+    if (s.kind == 1) return sin(s.om * t + s.ph);
+    const double tt = (t - s.t0) / s.tw;
+    return exp(-tt * tt);
+}
+
+// Start of a step whose stages need the time: t[2 + 2 s], t[3 + 2 s] = time
+// and source factor of stage s, then time = time + dt (src/cem_drive.F:639)
+// on the device, so a replayed graph sees the right stage times.  One small
+// launch a step instead of an exp or sin in every lane of every stage (N =
+// 8, 22^3, source: 308 -> 290 us per stage).
+struct StageC {
+    double c[5];
+};
+__global__ void stage_times(double *t, double dt, StageC rkc, SrcTime src) {
+    const double t0 = t[0];
+    __syncthreads();
+    if (threadIdx.x < 5) {
+        const double ts = t0 + rkc.c[threadIdx.x] * dt;
+        t[2 + 2 * threadIdx.x] = ts;
+        t[3 + 2 * threadIdx.x] = src_factor(src, ts);
+    }
+    if (threadIdx.x == 0) t[0] = t0 + dt;
+}
+// The pair of one given time, for nkc_residual.
+__global__ void stage_time(double *t, double time, SrcTime src) {
+    t[12] = time;
+    t[13] = src_factor(src, time);
+}
+__global__ void put_time(double *t, double time) { t[0] = time; }
 
 __global__ void maxabs_kernel(const double *__restrict__ u, int64_t fs, int64_t npts,
                               unsigned long long *out) {
@@ -450,9 +468,12 @@ struct nkc_handle {
     bool keep_k = false;                  // last stage writes the RK register (nkc_set_keep_k)
     double graph_dt = NAN;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
-    // tdev[0] = time at the start of the next step, tdev[1] = stage time for
-    // nkc_residual
+    // t_host: time at the start of the next step.  tdev (14 doubles): [0] the
+    // same on the device, kept when a source or an incident field needs it
+    // (tdev_ok: it is current); [2 + 2 s], [3 + 2 s] the time and source
+    // factor of stage s; [12], [13] those of nkc_residual.
     double *tdev = nullptr;
+    bool tdev_ok = false;
     double t_host = 0.0;
     // source
     int32_t *src_off = nullptr;
@@ -571,12 +592,10 @@ size_t sheet_size(const nkc_handle *h) {
 
 StageArgs base_args(nkc_handle *h) {
     StageArgs a = mesh_args(h->m);
-    a.tdev = h->tdev;
+    a.tst = h->tdev + 2;
     a.src_off = h->src_off;
     a.src_amp = h->src_amp;
     for (int c = 0; c < 3; ++c) a.src_dir[c] = h->src_dir[c];
-    a.src_t0 = h->src_t0;
-    a.src_tw = h->src_tw;
     a.drude_off = h->drude_off;
     a.dJ = h->dJ;
     a.dkJ = h->dkJ;
@@ -587,9 +606,6 @@ StageArgs base_args(nkc_handle *h) {
     a.lkL = h->lkL;
     a.lpar = h->lpar;
     a.lresL = h->lresL;
-    a.src_kind = h->src_kind;
-    a.src_om = h->src_om;
-    a.src_ph = h->src_ph;
     a.pml_off = h->pml_off;
     a.psig = h->psig;
     a.pP = h->pP;
@@ -617,8 +633,40 @@ int32_t handle_kflags(const nkc_handle *h, int s) {
     return stage_kflags(s) | ((h->keep_k && s == 4) ? 2 : 0);
 }
 
+// Whether the stages read the time.
+bool uses_time(const nkc_handle *h) { return h->src_off || h->inc_mask; }
+
+SrcTime src_time(const nkc_handle *h) { return SrcTime{h->src_kind, h->src_t0, h->src_tw, h->src_om, h->src_ph}; }
+
+// The stage times of a step about to be queued, and the time after it.
+int32_t queue_times(nkc_handle *h, double dt) {
+    if (!uses_time(h)) return NKC_OK;
+    StageC c;
+    for (int s = 0; s < 5; ++s) c.c[s] = RK4C[s];
+    hipLaunchKernelGGL(stage_times, dim3(1), dim3(64), 0, h->stream, h->tdev, dt, c, src_time(h));
+    HIPCHK(hipGetLastError());
+    return NKC_OK;
+}
+
+// The device's time brought up to t_host, when the stages will read it.
+int32_t current_time(nkc_handle *h) {
+    if (!uses_time(h) || h->tdev_ok) return NKC_OK;
+    hipLaunchKernelGGL(put_time, dim3(1), dim3(1), 0, h->stream, h->tdev, h->t_host);
+    HIPCHK(hipGetLastError());
+    h->tdev_ok = true;
+    return NKC_OK;
+}
+
+// t_host after a queued step (the device's sum when it keeps one).
+void time_passed(nkc_handle *h, double dt) {
+    h->t_host = h->t_host + dt;
+    if (!uses_time(h)) h->tdev_ok = false;
+}
+
 // Queue one RK step starting from buffer `from` (ends in 1-from).
 int32_t queue_step(nkc_handle *h, int from, double dt) {
+    const int32_t rt = queue_times(h, dt);
+    if (rt) return rt;
     for (int s = 0; s < 5; ++s) {
         StageArgs a = base_args(h);
         const int src = (from + s) & 1;
@@ -630,13 +678,11 @@ int32_t queue_step(nkc_handle *h, int from, double dt) {
         a.rka = RK4A[s];
         a.kflags = handle_kflags(h, s);
         a.rkb = RK4B[s];
-        a.rkc = RK4C[s];
+        a.tst = h->tdev + 2 + 2 * s;
         a.dt = dt;
         const int32_t rc = launch_stage(h->m, a, MODE_RK, h->stream);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(advance_time, dim3(1), dim3(1), 0, h->stream, h->tdev, dt);
-    HIPCHK(hipGetLastError());
     return NKC_OK;
 }
 
@@ -774,8 +820,9 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
         // element Jacobians and GLL weights of bm1 for the diagnostics
         if ((rc = upload(&h->djac, hm.jac)) || (rc = upload(&h->dw, hm.w))) break;
         if (hipMalloc((void **)&h->red, 8) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc"); break; }
-        if (hipMalloc((void **)&h->tdev, 2 * sizeof(double)) != hipSuccess ||
-            hipMemset(h->tdev, 0, 2 * sizeof(double)) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc time"); break; }
+        if (hipMalloc((void **)&h->tdev, 14 * sizeof(double)) != hipSuccess ||
+            hipMemset(h->tdev, 0, 14 * sizeof(double)) != hipSuccess ||
+            hipStreamSynchronize(nullptr) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc time"); break; }
     } while (0);
     if (rc) {
         free_handle(h);
@@ -788,7 +835,9 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
 
 // copy 6 fields between the caller's arrays (3 + 3 components at stride
 // ld, in host or device memory: hipMemcpyDefault tells them apart) and the
-// library's device blocks
+// library's device blocks.  A copy between device arrays, like a memset,
+// returns before it is done, and the handle's stream does not wait for the
+// null stream: finished here.
 int32_t copy_fields_h2d(double *dst, int64_t fs, int64_t dst_off, const double *hn, const double *en,
                         int64_t n, int64_t ld) {
     const size_t nb = sizeof(double) * n;
@@ -796,6 +845,7 @@ int32_t copy_fields_h2d(double *dst, int64_t fs, int64_t dst_off, const double *
         HIPCHK(hipMemcpy(dst + c * fs + dst_off, hn + c * ld, nb, hipMemcpyDefault));
         HIPCHK(hipMemcpy(dst + (3 + c) * fs + dst_off, en + c * ld, nb, hipMemcpyDefault));
     }
+    HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
 }
 
@@ -806,6 +856,7 @@ int32_t copy_fields_d2h(const double *src, int64_t fs, int64_t src_off, double *
         HIPCHK(hipMemcpy(hn + c * ld, src + c * fs + src_off, nb, hipMemcpyDefault));
         HIPCHK(hipMemcpy(en + c * ld, src + (3 + c) * fs + src_off, nb, hipMemcpyDefault));
     }
+    HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
 }
 
@@ -854,6 +905,8 @@ int32_t queue_step_store(nkc_handle *h, double dt, int64_t slot) {
     auto &A = h->adj;
     double *su = A.st_u + (int64_t)A.cur_slot * (5 * A.S + 1) * blk;
     double *sr = A.st_r ? A.st_r + (int64_t)A.cur_slot * 5 * A.S * blk : nullptr;
+    const int32_t rt = queue_times(h, dt);
+    if (rt) return rt;
     double *sj = h->ndrude ? A.stJ + (int64_t)A.cur_slot * 5 * A.S * (int64_t)drude_size(h) : nullptr;
     for (int s = 0; s < 5; ++s) {
         StageArgs a = base_args(h);
@@ -863,15 +916,13 @@ int32_t queue_step_store(nkc_handle *h, double dt, int64_t slot) {
         a.rka = RK4A[s];
         a.kflags = handle_kflags(h, s);
         a.rkb = RK4B[s];
-        a.rkc = RK4C[s];
+        a.tst = h->tdev + 2 + 2 * s;
         a.dt = dt;
         a.st_r = sr ? sr + (slot * 5 + s) * blk : nullptr;
         if (h->ndrude) a.st_J = sj + (slot * 5 + s) * (int64_t)drude_size(h);
         const int32_t rc = launch_stage(h->m, a, MODE_RK, h->stream);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(advance_time, dim3(1), dim3(1), 0, h->stream, h->tdev, dt);
-    HIPCHK(hipGetLastError());
     return NKC_OK;
 }
 
@@ -925,7 +976,6 @@ int32_t batch_queue_step(nkc_batch *b, int from) {
             a.rka = RK4A[s];
             a.kflags = stage_kflags(s);
             a.rkb = RK4B[s];
-            a.rkc = RK4C[s];
             a.dt = 0.0;              // per element from dt_e
             const int32_t rc = launch_stage(dm, a, MODE_RK, b->streams[i]);
             if (rc) return rc;
@@ -1047,8 +1097,6 @@ int32_t nkc_set_state(nkc_handle *h, const double *hn, const double *en, const d
     const DevMesh &m = h->m;
     if (ld < m.npts) return fail(NKC_ERR_ARG, "ld=%lld < npts=%lld", (long long)ld, (long long)m.npts);
     HIPCHK(hipStreamSynchronize(h->stream));
-    int32_t rc = copy_fields_h2d(m.u[h->cur], m.fs, 0, hn, en, m.npts, ld);
-    if (rc) return rc;
     const size_t nb = sizeof(double) * m.npts;
     for (int c = 0; c < 3; ++c) {
         if (khn) HIPCHK(hipMemcpy(m.k + c * m.fs, khn + c * ld, nb, hipMemcpyDefault));
@@ -1056,7 +1104,8 @@ int32_t nkc_set_state(nkc_handle *h, const double *hn, const double *en, const d
         if (ken) HIPCHK(hipMemcpy(m.k + (3 + c) * m.fs, ken + c * ld, nb, hipMemcpyDefault));
         else HIPCHK(hipMemset(m.k + (3 + c) * m.fs, 0, nb));
     }
-    return NKC_OK;
+    // last, as it also waits for the copies and fills of k
+    return copy_fields_h2d(m.u[h->cur], m.fs, 0, hn, en, m.npts, ld);
 }
 
 int32_t nkc_get_state(nkc_handle *h, double *hn, double *en, double *khn, double *ken, int64_t ld) {
@@ -1081,16 +1130,12 @@ int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps) {
     if (nsteps == 0) return NKC_OK;
     const double t0 = time ? *time : h->t_host;
     if (!(t0 == h->t_host)) {
-        HIPCHK(hipStreamSynchronize(h->stream));
-        HIPCHK(hipMemcpy(h->tdev, &t0, sizeof(double), hipMemcpyHostToDevice));
         h->t_host = t0;
+        h->tdev_ok = false;
     }
-    if (h->m.layout < 0) {
-        const StageArgs f = base_args(h);
-        const int32_t rc = tune_stage(h->m, &f, drude_size(h), lorentz_size(h), pml_size(h), sheet_size(h), h->m.u[h->cur], h->stream,
-                       h->tune_us);
-        if (rc) return rc;
-    }
+    if (h->m.layout < 0) h->m.layout = 0;
+    const int32_t rt = current_time(h);
+    if (rt) return rt;
     if (h->use_graph) {
         if (!(h->graph_dt == dt)) {
             const int32_t rc = capture(h, dt);
@@ -1107,7 +1152,7 @@ int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps) {
             h->cur ^= 1;
         }
     }
-    for (int64_t s = 0; s < nsteps; ++s) h->t_host = h->t_host + dt;   // same sums as the device
+    for (int64_t s = 0; s < nsteps; ++s) time_passed(h, dt);   // same sums as the device
     if (time) *time = h->t_host;
     return NKC_OK;
 }
@@ -1118,10 +1163,12 @@ int32_t nkc_residual(nkc_handle *h, double rktime, double *reshn, double *resen,
     if (ld < m.npts) return fail(NKC_ERR_ARG, "ld < npts");
     if (!h->res) HIPCHK(hipMalloc((void **)&h->res, sizeof(double) * 6 * m.fs));
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(h->tdev + 1, &rktime, sizeof(double), hipMemcpyHostToDevice));
+    if (uses_time(h)) {
+        hipLaunchKernelGGL(stage_time, dim3(1), dim3(1), 0, h->stream, h->tdev, rktime, src_time(h));
+        HIPCHK(hipGetLastError());
+    }
     StageArgs a = base_args(h);
-    a.tdev = h->tdev + 1;
-    a.rkc = 0.0;
+    a.tst = h->tdev + 12;
     a.uin = m.u[h->cur];
     a.res = h->res;
     const int32_t rc = launch_stage(m, a, MODE_RESIDUAL, h->stream);
@@ -1169,7 +1216,7 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     if (h->m.general && (amp != nullptr)) return general_refuses(h, "a source");
     HIPCHK(hipStreamSynchronize(h->stream));
     free_adjoint(h);                      // the stored trajectory has the old source
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->src_off); h->src_off = nullptr;
     (void)hipFree(h->src_amp); h->src_amp = nullptr;
     int32_t rc = drop_graphs(h);
@@ -1260,7 +1307,7 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     (void)hipFree(h->dpar); h->dpar = nullptr;
     (void)hipFree(h->dresJ); h->dresJ = nullptr;
     free_adjoint(h);                      // the stored trajectory has the old region
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     h->ndrude = 0;
     h->ndelem = 0;
     h->drude_slot.clear();
@@ -1475,7 +1522,7 @@ int32_t nkc_set_lorentz(nkc_handle *h, int64_t nlor, const int32_t *lindex, cons
     if (h->m.general && (nlor > 0)) return general_refuses(h, "a Lorentz region");
     HIPCHK(hipStreamSynchronize(h->stream));
     free_adjoint(h);
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->lor_off); h->lor_off = nullptr;
     (void)hipFree(h->lL); h->lL = nullptr;
     (void)hipFree(h->lkL); h->lkL = nullptr;
@@ -1570,7 +1617,7 @@ int32_t install_pml(nkc_handle *h, const std::vector<int64_t> &elems, const std:
 int32_t reset_pml(nkc_handle *h) {
     HIPCHK(hipStreamSynchronize(h->stream));
     free_adjoint(h);
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     free_pml(h);
     return drop_graphs(h);
 }
@@ -1717,7 +1764,7 @@ int32_t nkc_set_graphene(nkc_handle *h, int64_t ngraph, const int32_t *graphinde
     if (h->m.general && (ngraph > 0)) return general_refuses(h, "a graphene sheet");
     HIPCHK(hipStreamSynchronize(h->stream));
     free_adjoint(h);
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     free_sheet(h);
     int32_t rc = drop_graphs(h);
     if (rc || ngraph == 0) return rc;
@@ -1807,7 +1854,7 @@ int32_t nkc_set_incident(nkc_handle *h, int64_t nface, const int32_t *faces, con
     if (h->m.general && (nface > 0)) return general_refuses(h, "an incident field");
     HIPCHK(hipStreamSynchronize(h->stream));
     free_adjoint(h);
-    h->m.layout = -1;                     // the step's kernel instance may change: tune again
+    h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->inc_mask); h->inc_mask = nullptr;
     h->ninc = 0;
     int32_t rc = drop_graphs(h);
@@ -1873,8 +1920,9 @@ int32_t nkc_restart_read(nkc_handle *h, const char *path, int32_t *istep, int32_
     if ((rc = restart_read(path, m.n1, m.nelt, hd, u.data() + 3 * m.fs, u.data(), m.fs, err)))
         return fail(rc, "%s", err.c_str());
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(m.u[h->cur], u.data(), sizeof(double) * u.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(m.k, 0, sizeof(double) * u.size()));
+    HIPCHK(hipMemcpy(m.u[h->cur], u.data(), sizeof(double) * u.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipStreamSynchronize(nullptr));
     if (istep) *istep = hd.istep;
     if (dumpno) *dumpno = hd.dumpno;
     if (time) *time = hd.time;
@@ -1916,7 +1964,7 @@ int32_t nkc_info(nkc_handle *h, int64_t out[8]) {
     out[0] = h->m.npts;
     out[1] = h->m.mat;
     out[2] = 1;
-    out[3] = h->m.general ? GEO_BS : stage_block(n1, h->m.layout < 0 ? 0 : h->m.layout);
+    out[3] = h->m.general ? GEO_BS : stage_block(n1);
     out[4] = h->m.general ? (int64_t)sizeof(double) * (6 * n1 * n1 * n1 + 37 * n1 * n1)
                           : (int64_t)sizeof(double) * (6 * n1 * n1 * n1 + 25 * n1 * n1);
     out[5] = h->use_graph ? 1 : 0;
@@ -2115,8 +2163,8 @@ double step_time(const nkc_handle *h, int64_t step) {
 
 int32_t set_time(nkc_handle *h, double t) {
     HIPCHK(hipStreamSynchronize(h->stream));
-    HIPCHK(hipMemcpy(h->tdev, &t, sizeof(double), hipMemcpyHostToDevice));
     h->t_host = t;
+    h->tdev_ok = false;
     return NKC_OK;
 }
 
@@ -2139,9 +2187,10 @@ double *slot_u(nkc_handle *h, int k) {
 int32_t store_window(nkc_handle *h, int64_t seg, int64_t q) {
     int32_t rc;
     const int64_t n = win_steps(h, seg, q);
+    if ((rc = current_time(h))) return rc;
     for (int64_t s = 0; s < n; ++s) {
         if ((rc = queue_step_store(h, h->adj.dt, s))) return rc;
-        h->t_host = h->t_host + h->adj.dt;
+        time_passed(h, h->adj.dt);
     }
     h->adj.slot_id[h->adj.cur_slot] = seg * h->adj.nsub_max + q;
     return NKC_OK;
@@ -2383,6 +2432,7 @@ int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *la
     A.have_grad = true;
     if (geps) HIPCHK(hipMemcpy(geps, A.geps, sizeof(double) * m.npts, hipMemcpyDefault));
     if (gmu) HIPCHK(hipMemcpy(gmu, A.gmu, sizeof(double) * m.npts, hipMemcpyDefault));
+    HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
 }
 
@@ -2507,6 +2557,10 @@ int32_t nkc_batch_create(int32_t ncav, const nkc_box_desc *d, nkc_batch **out) {
         if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) { rc = fail(NKC_ERR_HIP, "stream"); break; }
         b->streams.push_back(s);
     }
+    // the orders step side by side: one working set
+    int64_t npts = 0;
+    for (const auto &dm : b->bins) npts += dm.npts;
+    for (auto &dm : b->bins) dm.nt = stage_nt(npts);
     if (!rc) {
         b->ev.resize(b->bins.size() + 1);
         for (auto &e : b->ev)
@@ -2538,10 +2592,9 @@ int32_t nkc_batch_set_state(nkc_batch *b, int32_t cav, const double *hn, const d
     const int64_t n3 = (int64_t)dm.n1 * dm.n1 * dm.n1, n = c.nelt * n3;
     if (ld < n) return fail(NKC_ERR_ARG, "ld < npts of cavity");
     HIPCHK(hipStreamSynchronize(b->main));
-    int32_t rc = copy_fields_h2d(dm.u[b->cur], dm.fs, c.off * n3, hn, en, n, ld);
-    if (rc) return rc;
     for (int f = 0; f < 6; ++f) HIPCHK(hipMemset(dm.k + f * dm.fs + c.off * n3, 0, sizeof(double) * n));
-    return NKC_OK;
+    // last, as it also waits for the fills of k
+    return copy_fields_h2d(dm.u[b->cur], dm.fs, c.off * n3, hn, en, n, ld);
 }
 
 int32_t nkc_batch_get_state(nkc_batch *b, int32_t cav, double *hn, double *en, int64_t ld) {
@@ -2574,11 +2627,7 @@ int32_t nkc_batch_step(nkc_batch *b, const double *dt, double *times, int64_t ns
         for (int c = 0; c < ncav; ++c) b->cav[c].dt = dt[c];
     }
     for (auto &dm : b->bins)
-        if (dm.layout < 0) {
-            double us[NLAYOUT];
-            const int32_t rc = tune_stage(dm, nullptr, 0, 0, 0, 0, dm.u[b->cur], b->main, us);
-            if (rc) return rc;
-        }
+        if (dm.layout < 0) dm.layout = 0;
     if (!b->graph_ok) {
         const int32_t rc = batch_capture(b);
         if (rc) return rc;

@@ -9,70 +9,37 @@
 namespace nkc {
 namespace {
 
-// Kernel instance by feature set: FEAT = 2 with a PML, an incident field or
-// a graphene sheet; 1 with a source, Drude or Lorentz region; 0 otherwise.
-template <int N1, int MAT, int MODE, int PACK, int OCC, int EPW>
-void launch_t(const StageArgs &a, int grid, hipStream_t s) {
-    const dim3 bs(Shape<N1, PACK>::BS * EPW);
-    if (a.pml_off || a.inc_mask || a.gr_off)
-        hipLaunchKernelGGL((stage_kernel<N1, MAT, MODE, PACK, OCC, 2, EPW>), dim3(grid), bs, 0, s, a);
-    else if (a.src_off || a.drude_off || a.lor_off)
-        hipLaunchKernelGGL((stage_kernel<N1, MAT, MODE, PACK, OCC, 1, EPW>), dim3(grid), bs, 0, s, a);
+template <int N1, int MAT, int MODE, int FEAT>
+void launch_f(const StageArgs &a, bool nt, int grid, hipStream_t s) {
+    constexpr int OCC = box_waves(N1, FEAT);
+    const dim3 bs(BoxShape<N1>::BS);
+    if (MODE != MODE_RESIDUAL && nt)
+        hipLaunchKernelGGL((box_kernel<N1, MAT, MODE, FEAT, MODE != MODE_RESIDUAL, OCC>), dim3(grid), bs, 0, s, a);
     else
-        hipLaunchKernelGGL((stage_kernel<N1, MAT, MODE, PACK, OCC, 0, EPW>), dim3(grid), bs, 0, s, a);
+        hipLaunchKernelGGL((box_kernel<N1, MAT, MODE, FEAT, false, OCC>), dim3(grid), bs, 0, s, a);
 }
 
-// The residual test entry always runs layout 0.
-template <int N1, int MAT, int PACK, int OCC, int EPW>
-void launch_m(const StageArgs &a, int mode, int grid, hipStream_t s) {
-    if (mode == MODE_RK) launch_t<N1, MAT, MODE_RK, PACK, OCC, EPW>(a, grid, s);
-    else launch_t<N1, MAT, MODE_RESIDUAL, 0, 0, 1>(a, grid, s);
-}
-
-template <int N1, int PACK, int OCC, int EPW>
-void launch_p(const StageArgs &a, int mat, int mode, int grid, hipStream_t s) {
-    if (mat == MAT_ELEM) launch_m<N1, MAT_ELEM, PACK, OCC, EPW>(a, mode, grid, s);
-    else launch_m<N1, MAT_NODE, PACK, OCC, EPW>(a, mode, grid, s);
-}
-
-// The six-role kernel (layouts 6, 7): RK stages with at most a source,
-// Drude or Lorentz region; anything else runs layout 0.
-template <int N1, int OCC>
-void launch_s6(const StageArgs &a, int mat, int mode, int grid, hipStream_t s) {
-    if (mode != MODE_RK || a.pml_off || a.inc_mask || a.gr_off) {
-        launch_p<N1, 0, 0, 1>(a, mat, mode, grid, s);
-        return;
-    }
-    const dim3 bs(Shape6<N1>::BS);
-    const bool feat = a.src_off || a.drude_off || a.lor_off;
-    if (mat == MAT_ELEM) {
-        if (feat) hipLaunchKernelGGL((stage6_kernel<N1, MAT_ELEM, MODE_RK, OCC, 1>), dim3(grid), bs, 0, s, a);
-        else hipLaunchKernelGGL((stage6_kernel<N1, MAT_ELEM, MODE_RK, OCC, 0>), dim3(grid), bs, 0, s, a);
+// Kernel instance by feature set: FEAT = 3 with a graphene sheet, 2 with a
+// PML or an incident field, 1 with a source, Drude or Lorentz region, 0
+// otherwise.  The residual test entry has the plain and the full instance.
+template <int N1, int MAT>
+void launch_m(const StageArgs &a, int mode, bool nt, int grid, hipStream_t s) {
+    const int feat = a.gr_off ? 3 : (a.pml_off || a.inc_mask) ? 2 : (a.src_off || a.drude_off || a.lor_off) ? 1 : 0;
+    if (mode == MODE_RESIDUAL) {
+        if (feat) launch_f<N1, MAT, MODE_RESIDUAL, 3>(a, false, grid, s);
+        else launch_f<N1, MAT, MODE_RESIDUAL, 0>(a, false, grid, s);
+    } else if (a.st_r || a.st_J) {
+        // the adjoint's recompute: sources and Drude regions only
+        if (feat) launch_f<N1, MAT, MODE_RK_STORE, 1>(a, nt, grid, s);
+        else launch_f<N1, MAT, MODE_RK_STORE, 0>(a, nt, grid, s);
+    } else if (feat == 3) {
+        launch_f<N1, MAT, MODE_RK, 3>(a, nt, grid, s);
+    } else if (feat == 2) {
+        launch_f<N1, MAT, MODE_RK, 2>(a, nt, grid, s);
+    } else if (feat == 1) {
+        launch_f<N1, MAT, MODE_RK, 1>(a, nt, grid, s);
     } else {
-        if (feat) hipLaunchKernelGGL((stage6_kernel<N1, MAT_NODE, MODE_RK, OCC, 1>), dim3(grid), bs, 0, s, a);
-        else hipLaunchKernelGGL((stage6_kernel<N1, MAT_NODE, MODE_RK, OCC, 0>), dim3(grid), bs, 0, s, a);
-    }
-}
-
-template <int N1>
-void launch_n(const StageArgs &a, int mat, int mode, int layout, int grid, hipStream_t s) {
-    switch (layout) {
-    case 1: launch_p<N1, 1, 0, 1>(a, mat, mode, grid, s); break;
-    case 2: launch_p<N1, 0, 1, 1>(a, mat, mode, grid, s); break;
-    case 3: launch_p<N1, 1, 1, 1>(a, mat, mode, grid, s); break;
-    case 4:
-        if constexpr (N1 <= EPW_MAX_N1) launch_p<N1, 1, 0, 2>(a, mat, mode, grid, s);
-        break;
-    case 5:
-        if constexpr (N1 <= EPW_MAX_N1) launch_p<N1, 1, 1, 2>(a, mat, mode, grid, s);
-        break;
-    case 6:
-        if constexpr (N1 >= S6_MIN_N1) launch_s6<N1, 0>(a, mat, mode, grid, s);
-        break;
-    case 7:
-        if constexpr (N1 >= S6_MIN_N1) launch_s6<N1, 1>(a, mat, mode, grid, s);
-        break;
-    default: launch_p<N1, 0, 0, 1>(a, mat, mode, grid, s); break;
+        launch_f<N1, MAT, MODE_RK, 0>(a, nt, grid, s);
     }
 }
 
@@ -89,8 +56,9 @@ void launch_adj_t(const AdjArgs &a, int grid, hipStream_t s) {
 #define NKC_CAT2(a, b) a##b
 #define NKC_CAT(a, b) NKC_CAT2(a, b)
 
-void NKC_CAT(launch_stage_n, NKC_N1)(const StageArgs &a, int mat, int mode, int layout, int grid, hipStream_t s) {
-    launch_n<NKC_N1>(a, mat, mode, layout, grid, s);
+void NKC_CAT(launch_stage_n, NKC_N1)(const StageArgs &a, int mat, int mode, bool nt, int grid, hipStream_t s) {
+    if (mat == MAT_ELEM) launch_m<NKC_N1, MAT_ELEM>(a, mode, nt, grid, s);
+    else launch_m<NKC_N1, MAT_NODE>(a, mode, nt, grid, s);
 }
 
 void NKC_CAT(launch_adjoint_n, NKC_N1)(const AdjArgs &a, int mat, int grid, hipStream_t s) {

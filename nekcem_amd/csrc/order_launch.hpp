@@ -8,18 +8,20 @@
 #include <hip/hip_runtime.h>
 
 #include "adjoint_kernel.hpp"
-#include "stage6_kernel.hpp"
-#include "stage_kernel.hpp"
+#include "box_kernel.hpp"
 
 namespace nkc {
 
-// Orders that have the two-element-per-workgroup layouts 4 and 5.
-constexpr int EPW_MAX_N1 = 6;
-// Orders that have the six-role layouts 6 and 7.
-constexpr int S6_MIN_N1 = 8;
+// Waves per SIMD the register allocator of the stage kernel keeps to (0:
+// free): 128 VGPRs from N = 6 on, where the 8-wave workgroups of N = 8, 9
+// then fit twice on a CU and the 4-wave ones of N = 6, 7 four times; 168 at
+// N = 7 with a PML, an incident field or a sheet, which would spill at 128 (its swizzled LDS
+// addresses take a register each).
+constexpr int box_waves(int n1, int feat) { return n1 < 7 ? 0 : (n1 == 8 && feat >= 2) ? 3 : 4; }
 
+// nt: k and the outputs past the caches (see stage_nt)
 #define NKC_DECL_ORDER(n)                                                                          \
-    void launch_stage_n##n(const StageArgs &a, int mat, int mode, int layout, int grid, hipStream_t s); \
+    void launch_stage_n##n(const StageArgs &a, int mat, int mode, bool nt, int grid, hipStream_t s); \
     void launch_adjoint_n##n(const AdjArgs &a, int mat, int grid, hipStream_t s);
 NKC_DECL_ORDER(4)
 NKC_DECL_ORDER(5)

@@ -551,18 +551,18 @@ class MaxwellSolver:
         return dict(istep=istep.value, dumpno=dumpno.value, time=t.value, dt=dt.value)
 
     def set_layout(self, layout):
-        """Force the stage-kernel layout (0..NLAYOUT-1), or -1 to re-tune."""
+        """Name the stage-kernel layout (0..NLAYOUT-1), or -1 for the default."""
         _lib.check(self._L.nkc_set_layout(self._h, int(layout)))
 
     def layout(self):
-        """dict(us=(tuner times per layout, NaN: not timed), layout) without
-        tuning."""
+        """dict(us=(times of tune() per layout, NaN: none), layout) without
+        timing."""
         out = np.empty(NLAYOUT + 1)
         _lib.check(self._L.nkc_get_layout(self._h, _d(out)))
         return dict(us=tuple(float(v) for v in out[:NLAYOUT]), layout=int(out[NLAYOUT]))
 
     def tune(self):
-        """Run the layout autotuner now: dict(us=(per layout), layout)."""
+        """Time the stage on this mesh: dict(us=(per layout), layout)."""
         out = np.empty(NLAYOUT + 1)
         _lib.check(self._L.nkc_tune(self._h, _d(out)))
         return dict(us=tuple(float(v) for v in out[:NLAYOUT]), layout=int(out[NLAYOUT]))
@@ -735,7 +735,7 @@ class BatchSolver:
         return dict(npts=out[0], ncav=out[1], norders=out[2], nelt=out[3])
 
     def layout(self):
-        """{N: stage-kernel layout} per polynomial order (-1 before tuning)."""
+        """{N: stage-kernel layout} per polynomial order (-1 before the first step)."""
         nb = self.info()["norders"]
         out = (C.c_int32 * (2 * nb))()
         _lib.check(self._L.nkc_batch_layout(self._b, out, 2 * nb))
