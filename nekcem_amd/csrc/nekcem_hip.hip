@@ -425,16 +425,25 @@ __global__ void stage_time(double *t, double time, SrcTime src) {
 }
 __global__ void put_time(double *t, double time) { t[0] = time; }
 
+// Largest |u| of a workgroup's share of the six fields, as the value's bits,
+// into out[blockIdx.x] (pinned host memory: no fill, no atomics, no copy back
+// -- the host takes the largest after one wait; a step and a check at 4^3,
+// N = 7: 86 -> 60 us).
+constexpr int CHECK_BLOCKS = 1024;
 __global__ void maxabs_kernel(const double *__restrict__ u, int64_t fs, int64_t npts,
                               unsigned long long *out) {
     unsigned long long m = 0;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int f = 0; f < 6; ++f)
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < npts; i += stride) {
-            const double v = fabs(u[f * fs + i]);
-            const unsigned long long b = __double_as_longlong(v);   // monotone for v >= 0, NaN on top
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < npts; i += stride) {
+        double v[6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) v[f] = u[f * fs + i];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            const unsigned long long b = __double_as_longlong(fabs(v[f]));   // monotone for v >= 0, NaN on top
             m = b > m ? b : m;
         }
+    }
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_down(m, off);
         m = o > m ? o : m;
@@ -446,11 +455,21 @@ __global__ void maxabs_kernel(const double *__restrict__ u, int64_t fs, int64_t 
     if (threadIdx.x == 0) {
         unsigned long long r = 0;
         for (int q = 0; q < (int)(blockDim.x >> 6); ++q) r = sm[q] > r ? sm[q] : r;
-        atomicMax(out, r);
+        out[blockIdx.x] = r;
     }
 }
 
-__global__ void zero_u64(unsigned long long *p) { *p = 0ull; }
+// Six fields between two device blocks: a caller's (three components from h
+// and three from e at stride ld) and the library's (stride fs), in one launch.
+template <bool IN>
+__global__ void copy_fields_kernel(double *h, double *e, int64_t ld, double *blk, int64_t fs, int64_t n) {
+    const int c = blockIdx.y;
+    double *u = (c < 3 ? h + c * ld : e + (c - 3) * ld), *b = blk + c * fs;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        if (IN) b[i] = u[i];
+        else u[i] = b[i];
+    }
+}
 
 }  // namespace
 
@@ -462,7 +481,7 @@ struct nkc_handle {
     int device = 0;
     hipStream_t stream = nullptr;
     double *res = nullptr;
-    unsigned long long *red = nullptr;   // check_finite result
+    unsigned long long *red = nullptr;   // check_finite results per workgroup (pinned host), made by the first check
     int cur = 0;                          // which u buffer holds the state
     bool use_graph = true;
     bool keep_k = false;                  // last stage writes the RK register (nkc_set_keep_k)
@@ -746,7 +765,8 @@ void free_handle(nkc_handle *h) {
     (void)hipFree(h->yz);
     h->yz = nullptr;
     dev_mesh_free(h->m);
-    (void)hipFree(h->res); (void)hipFree(h->red); (void)hipFree(h->tdev);
+    (void)hipFree(h->res); (void)hipFree(h->tdev);
+    if (h->red) (void)hipHostFree(h->red);
     (void)hipFree(h->src_off); (void)hipFree(h->src_amp);
     (void)hipFree(h->drude_off); (void)hipFree(h->dJ); (void)hipFree(h->dkJ);
     (void)hipFree(h->dpar); (void)hipFree(h->dresJ);
@@ -819,7 +839,6 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
         if ((rc = dev_mesh_upload(hm, h->m))) break;
         // element Jacobians and GLL weights of bm1 for the diagnostics
         if ((rc = upload(&h->djac, hm.jac)) || (rc = upload(&h->dw, hm.w))) break;
-        if (hipMalloc((void **)&h->red, 8) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc"); break; }
         if (hipMalloc((void **)&h->tdev, 14 * sizeof(double)) != hipSuccess ||
             hipMemset(h->tdev, 0, 14 * sizeof(double)) != hipSuccess ||
             hipStreamSynchronize(nullptr) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc time"); break; }
@@ -833,31 +852,53 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
     return NKC_OK;
 }
 
-// copy 6 fields between the caller's arrays (3 + 3 components at stride
-// ld, in host or device memory: hipMemcpyDefault tells them apart) and the
-// library's device blocks.  A copy between device arrays, like a memset,
-// returns before it is done, and the handle's stream does not wait for the
-// null stream: finished here.
-int32_t copy_fields_h2d(double *dst, int64_t fs, int64_t dst_off, const double *hn, const double *en,
-                        int64_t n, int64_t ld) {
-    const size_t nb = sizeof(double) * n;
-    for (int c = 0; c < 3; ++c) {
-        HIPCHK(hipMemcpy(dst + c * fs + dst_off, hn + c * ld, nb, hipMemcpyDefault));
-        HIPCHK(hipMemcpy(dst + (3 + c) * fs + dst_off, en + c * ld, nb, hipMemcpyDefault));
+// Whether both arrays are memory of the current device.
+bool on_device(const double *p, const double *q) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    for (const double *x : {p, q}) {
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, x) != hipSuccess) {
+            (void)hipGetLastError();   // plain host memory
+            return false;
+        }
+        if (at.type != hipMemoryTypeDevice || at.device != dev) return false;
+    }
+    return true;
+}
+
+// Copy 6 fields between the caller's arrays (3 + 3 components at stride ld,
+// in host or device memory) and the library's device blocks.  Device arrays
+// go in one launch on the null stream, where it follows the caller's work as
+// a hipMemcpy would; anything else by hipMemcpyDefault.  A copy between
+// device arrays, like a memset, returns before it is done, and the handle's
+// stream does not wait for the null stream: finished here.
+template <bool IN>
+int32_t copy_fields(double *blk, int64_t fs, double *hn, double *en, int64_t n, int64_t ld) {
+    if (on_device(hn, en)) {
+        const int nb = (int)std::min<int64_t>(2048, (n + 255) / 256);
+        hipLaunchKernelGGL(copy_fields_kernel<IN>, dim3(nb, 6), dim3(256), 0, nullptr, hn, en, ld, blk, fs, n);
+        HIPCHK(hipGetLastError());
+    } else {
+        const size_t nb = sizeof(double) * n;
+        for (int c = 0; c < 6; ++c) {
+            double *u = c < 3 ? hn + c * ld : en + (c - 3) * ld;
+            if (IN) HIPCHK(hipMemcpy(blk + c * fs, u, nb, hipMemcpyDefault));
+            else HIPCHK(hipMemcpy(u, blk + c * fs, nb, hipMemcpyDefault));
+        }
     }
     HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
 }
 
+int32_t copy_fields_h2d(double *dst, int64_t fs, int64_t dst_off, const double *hn, const double *en,
+                        int64_t n, int64_t ld) {
+    return copy_fields<true>(dst + dst_off, fs, const_cast<double *>(hn), const_cast<double *>(en), n, ld);
+}
+
 int32_t copy_fields_d2h(const double *src, int64_t fs, int64_t src_off, double *hn, double *en,
                         int64_t n, int64_t ld) {
-    const size_t nb = sizeof(double) * n;
-    for (int c = 0; c < 3; ++c) {
-        HIPCHK(hipMemcpy(hn + c * ld, src + c * fs + src_off, nb, hipMemcpyDefault));
-        HIPCHK(hipMemcpy(en + c * ld, src + (3 + c) * fs + src_off, nb, hipMemcpyDefault));
-    }
-    HIPCHK(hipStreamSynchronize(nullptr));
-    return NKC_OK;
+    return copy_fields<false>(const_cast<double *>(src) + src_off, fs, hn, en, n, ld);
 }
 
 // A caller's array (host or device memory) as a host vector, for the entry
@@ -1098,7 +1139,8 @@ int32_t nkc_set_state(nkc_handle *h, const double *hn, const double *en, const d
     if (ld < m.npts) return fail(NKC_ERR_ARG, "ld=%lld < npts=%lld", (long long)ld, (long long)m.npts);
     HIPCHK(hipStreamSynchronize(h->stream));
     const size_t nb = sizeof(double) * m.npts;
-    for (int c = 0; c < 3; ++c) {
+    if (!khn && !ken) HIPCHK(hipMemset(m.k, 0, sizeof(double) * 6 * m.fs));
+    else for (int c = 0; c < 3; ++c) {
         if (khn) HIPCHK(hipMemcpy(m.k + c * m.fs, khn + c * ld, nb, hipMemcpyDefault));
         else HIPCHK(hipMemset(m.k + c * m.fs, 0, nb));
         if (ken) HIPCHK(hipMemcpy(m.k + (3 + c) * m.fs, ken + c * ld, nb, hipMemcpyDefault));
@@ -1932,13 +1974,13 @@ int32_t nkc_restart_read(nkc_handle *h, const char *path, int32_t *istep, int32_
 
 int32_t nkc_check_finite(nkc_handle *h, double *maxabs) {
     if (!h) return fail(NKC_ERR_ARG, "null handle");
-    hipLaunchKernelGGL(zero_u64, dim3(1), dim3(1), 0, h->stream, h->red);
-    hipLaunchKernelGGL(maxabs_kernel, dim3(1024), dim3(256), 0, h->stream, h->m.u[h->cur], h->m.fs,
-                       h->m.npts, h->red);
+    if (!h->red) HIPCHK(hipHostMalloc((void **)&h->red, sizeof(unsigned long long) * CHECK_BLOCKS, hipHostMallocDefault));
+    const int nb = (int)std::min<int64_t>(CHECK_BLOCKS, (h->m.npts + 255) / 256);
+    hipLaunchKernelGGL(maxabs_kernel, dim3(nb), dim3(256), 0, h->stream, h->m.u[h->cur], h->m.fs, h->m.npts, h->red);
     HIPCHK(hipGetLastError());
-    unsigned long long bits = 0;
-    HIPCHK(hipMemcpyAsync(&bits, h->red, 8, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    unsigned long long bits = 0;
+    for (int i = 0; i < nb; ++i) bits = std::max(bits, h->red[i]);
     double mx;
     std::memcpy(&mx, &bits, 8);
     if (maxabs) *maxabs = mx;
