@@ -379,7 +379,8 @@ int32_t nkc_stream(nkc_handle *h, void **stream);
 
 /* Facts about the compiled handle: out[0] = npts, out[1] = material mode
  * (0 per element, 1 per node), out[2] = elements per workgroup,
- * out[3] = threads per workgroup, out[4] = LDS bytes per workgroup,
+ * out[3] = threads per workgroup (general handles: 256, whatever their kernel
+ * takes), out[4] = LDS bytes per workgroup,
  * out[5] = graph capture enabled (1/0). */
 int32_t nkc_info(nkc_handle *h, int64_t out[8]);
 

@@ -10,13 +10,23 @@
 // in-face orientation), the lift area/(J w3) of add_flux_to_res and
 // invqmass (:654-756, 1833-1904).
 //
-// Mapping: one workgroup of 256 lanes per element; the element's six fields
-// are staged in LDS; phase 1 forms the flux of every face node (6 (N+1)^2
-// of them, strided over the lanes) into LDS, phase 2 gives each lane whole
-// nodes (strided): nine derivatives of E and of H along r, s, t, the two
-// curls, the lifted fluxes of the faces the node lies on, inverse mass and
-// the low-storage RK update.  Up to N = 11 (12^3 nodes: 125 KB of LDS, one
-// workgroup per CU).  Materials per node, flux coefficients per face node.
+// Mapping: a workgroup takes an element, or on meshes too small to fill the
+// chip a slab of its levels (GeoArgs::nslab slabs per element; every one
+// stages the whole element, the r, s, t lines of its nodes).  Half of the
+// waves update H, half E (nine derivative sums a lane instead of eighteen:
+// 254 -> under 128 VGPRs, twice the workgroups per CU), each lane one node
+// after another in the order of memory.
+//   0  every load of the element and of the slab's face nodes (geometry,
+//      partner traces) up front; the element into LDS;
+//   1  the flux of the slab's face nodes into LDS;
+//   2  per node: metrics, RK register and inverse material requested first,
+//      then the derivatives from LDS, the curl, the lifted fluxes of the
+//      faces the node lies on, inverse mass and the low-storage RK update.
+// Bound: on small meshes one workgroup's chain of phases (5 x 5 x 2 elements
+// at N = 11: 41 -> 13 us per stage), on large ones the bytes (10^3
+// elements at N = 7, in the Infinity Cache: 36 -> 32 us).
+// Up to N = 11 (12^3 nodes: 125 KB of LDS, one workgroup per CU).  Materials
+// per node, flux coefficients per face node.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -44,11 +54,14 @@ struct GeoArgs {
     int64_t npts;
     int32_t nelt;
     int32_t per_xcd;
+    int32_t nslab;                     // workgroups per element, each a run of levels
     double rka, rkb, dt;
     int32_t kflags;                    // bit 0 read k, bit 1 write k
 };
 
-constexpr int GEO_BS = 256;
+// Lanes of a workgroup: 16 waves per CU at one (N = 11), two (N = 8..10) or
+// three to four workgroups per CU, what their LDS allows.
+constexpr int geo_block(int n1) { return n1 >= 12 ? 1024 : n1 >= 9 ? 512 : 256; }
 
 // In-element volume index of in-face node q = a + n1 b on the reference's
 // face ef0 + 1 (0: y-, 1: x+, 2: y+, 3: x-, 4: z-, 5: z+), skpdat order
@@ -67,135 +80,181 @@ __device__ __forceinline__ int ed_face_node(int ef0, int q) {
     }
 }
 
-template <int N1, int MODE>
-__global__ void __launch_bounds__(GEO_BS) geo_stage_kernel(GeoArgs a) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1;
+template <int N1, int MODE, bool NT>
+__global__ void __launch_bounds__(geo_block(N1)) __attribute__((amdgpu_waves_per_eu(4)))
+geo_stage_kernel(GeoArgs a) {
+    constexpr int N2 = N1 * N1, N3 = N2 * N1, BS = geo_block(N1), W = BS / 64, GL = BS / 2, NFN = 6 * N2;
+    constexpr int CH = (N3 + 63) / 64, NLD = (6 * CH + W - 1) / W, NFL = (NFN + BS - 1) / BS;
     __shared__ double s_u[6 * N3];
-    __shared__ double s_f[6 * N2 * 6];   // [face node of the element][FH 0..2, FE 0..2]
+    __shared__ double s_f[6 * NFN];      // [FH 0..2, FE 0..2][face node of the slab]
     __shared__ double s_D[N2];
-    const int e = remap_element(blockIdx.x, a.nelt, a.per_xcd);
-    if (e >= a.nelt) return;
-    const int t = threadIdx.x;
+    // the slabs of an element follow each other on one XCD
+    const int slot = blockIdx.x >> 3;
+    const int e = (blockIdx.x & 7) * a.per_xcd + slot / a.nslab;
+    const int slab = slot % a.nslab;
+    if (e >= a.nelt || slot / a.nslab >= a.per_xcd) return;
+    const int kb = slab * N1 / a.nslab, ks = (slab + 1) * N1 / a.nslab - kb;   // levels kb .. kb + ks - 1
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int64_t eo = (int64_t)e * N3, fs = a.fs;
-    const int64_t so = (int64_t)e * 6 * N2;
 
-    for (int v = t; v < 6 * N3; v += GEO_BS) s_u[v] = a.uin[(v / N3) * fs + eo + v % N3];
-    for (int v = t; v < N2; v += GEO_BS) s_D[v] = a.D[v];
+    // ---- phase 0 ----
+    double ld[NLD];
+#pragma unroll
+    for (int n = 0; n < NLD; ++n) {
+        const int id = min(w + W * n, 6 * CH - 1), f = id / CH;
+        const int off = min((id - f * CH) * 64 + lane, N3 - 1);
+        ld[n] = (a.uin + f * fs + eo)[(unsigned)off];
+    }
+    // the slab's face nodes: its rows of the four side faces (reference
+    // order y-, x+, y+, x-), then z- and z+ where the slab touches them
+    const int side = 4 * N1 * ks, zlo = kb == 0 ? N2 : 0, zhi = kb + ks == N1 ? N2 : 0;
+    const int nf = MODE == GMODE_CURL ? 0 : side + zlo + zhi;
+    double up[NFL][6], fg[NFL][4], cf[NFL][4];
+    int32_t nb[NFL];
+    int own[NFL];
+    int64_t sl[NFL];
+#pragma unroll
+    for (int n = 0; n < NFL; ++n) {
+        const int x = t + BS * n;
+        int ef = 0, q = 0;
+        if (x < side) {
+            const int row = x / N1;
+            ef = (row >= ks) + (row >= 2 * ks) + (row >= 3 * ks);
+            q = x - row * N1 + N1 * (kb + row - ef * ks);
+        } else if (x < nf) {
+            const int z = x - side;
+            ef = z < zlo ? 4 : 5;
+            q = z < zlo ? z : z - zlo;
+        }
+        own[n] = ed_face_node<N1>(ef, q);
+        sl[n] = ((int64_t)e * 6 + ef) * N2 + q;
+        nb[n] = x < nf ? a.fnb[sl[n]] : FACE_NONE;
+    }
+#pragma unroll
+    for (int n = 0; n < NFL; ++n) {
+        const bool on = t + BS * n < nf;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) up[n][c] = nb[n] >= 0 ? a.uin[c * fs + nb[n]] : 0.0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            fg[n][c] = on ? a.fgeo[4 * sl[n] + c] : 0.0;
+            cf[n][c] = on ? a.fco[4 * sl[n] + c] : 0.0;
+        }
+    }
+    for (int v = t; v < N2; v += BS) s_D[v] = a.D[v];
+#pragma unroll
+    for (int n = 0; n < NLD; ++n) {
+        const int id = min(w + W * n, 6 * CH - 1), f = id / CH;
+        s_u[f * N3 + min((id - f * CH) * 64 + lane, N3 - 1)] = ld[n];
+    }
     __syncthreads();
 
-    // ---- phase 1: the flux at every face node of the element ----
-    if (MODE != GMODE_CURL) {
-        for (int fq = t; fq < 6 * N2; fq += GEO_BS) {
-            const int ef0 = fq / N2, q = fq % N2;
-            const int64_t s = so + fq;
-            const int own = ed_face_node<N1>(ef0, q);
-            const double n[3] = {a.fgeo[4 * s], a.fgeo[4 * s + 1], a.fgeo[4 * s + 2]};
-            const double L = a.fgeo[4 * s + 3];
-            const double cf[4] = {a.fco[4 * s], a.fco[4 * s + 1], a.fco[4 * s + 2], a.fco[4 * s + 3]};
-            const int32_t nb = a.fnb[s];
-            double um[6];
+    // ---- phase 1: the flux at the slab's face nodes ----
 #pragma unroll
-            for (int c = 0; c < 6; ++c) um[c] = s_u[c * N3 + own];
-            double sE[3], sH[3];
-            if (nb >= 0) {
-                // n x [E] = (-n x E-) + (-n' x E+), n' = -n
-                double dE[3], dH[3];
+    for (int n = 0; n < NFL; ++n) {
+        const int x = t + BS * n;
+        if (x >= nf) break;
+        const double nv[3] = {fg[n][0], fg[n][1], fg[n][2]};
+        const double L = fg[n][3];
+        double um[6];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    dH[c] = a.uin[c * fs + nb] - um[c];
-                    dE[c] = a.uin[(3 + c) * fs + nb] - um[3 + c];
-                }
-                gcross(n, dE, sE);
-                gcross(n, dH, sH);
+        for (int c = 0; c < 6; ++c) um[c] = s_u[c * N3 + own[n]];
+        double sE[3], sH[3];
+        if (nb[n] >= 0) {
+            // n x [E] = (-n x E-) + (-n' x E+), n' = -n
+            const double dH[3] = {up[n][0] - um[0], up[n][1] - um[1], up[n][2] - um[2]};
+            const double dE[3] = {up[n][3] - um[3], up[n][4] - um[4], up[n][5] - um[5]};
+            gcross(nv, dE, sE);
+            gcross(nv, dH, sH);
+        } else {
+            // no partner: gs leaves -n x E-, -n x H-; PEC doubles E, zeroes H
+            const double Em[3] = {-um[3], -um[4], -um[5]};
+            gcross(nv, Em, sE);
+            if (nb[n] == FACE_PEC) {
+                sE[0] *= 2.0; sE[1] *= 2.0; sE[2] *= 2.0;
+                sH[0] = sH[1] = sH[2] = 0.0;
             } else {
-                // no partner: gs leaves -n x E-, -n x H-; PEC doubles E, zeroes H
-                const double Em[3] = {-um[3], -um[4], -um[5]};
-                gcross(n, Em, sE);
-                if (nb == FACE_PEC) {
-                    sE[0] *= 2.0; sE[1] *= 2.0; sE[2] *= 2.0;
-                    sH[0] = sH[1] = sH[2] = 0.0;
-                } else {
-                    const double Hm[3] = {-um[0], -um[1], -um[2]};
-                    gcross(n, Hm, sH);
-                }
-            }
-            double fu[3], fw[3];
-            gcross(n, sH, fu);
-            gcross(n, sE, fw);
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                s_f[fq * 6 + c] = L * (cf[0] * sE[c] - cf[1] * fu[c]);
-                s_f[fq * 6 + 3 + c] = L * (cf[2] * sH[c] - cf[3] * fw[c]);
+                const double Hm[3] = {-um[0], -um[1], -um[2]};
+                gcross(nv, Hm, sH);
             }
         }
-        __syncthreads();
-    }
-
-    // ---- phase 2: whole nodes per lane ----
-    for (int v = t; v < N3; v += GEO_BS) {
-        const int i = v % N1, j = (v / N1) % N1, k = v / N2;
-        // d/dr, d/ds, d/dt of the six fields
-        double dr[6], ds[6], dt_[6];
+        double fu[3], fw[3];
+        gcross(nv, sH, fu);
+        gcross(nv, sE, fw);
 #pragma unroll
-        for (int c = 0; c < 6; ++c) { dr[c] = 0.0; ds[c] = 0.0; dt_[c] = 0.0; }
+        for (int c = 0; c < 3; ++c) {
+            s_f[c * NFN + x] = L * (cf[n][0] * sE[c] - cf[n][1] * fu[c]);
+            s_f[(3 + c) * NFN + x] = L * (cf[n][2] * sH[c] - cf[n][3] * fw[c]);
+        }
+    }
+    if (MODE != GMODE_CURL) __syncthreads();
+
+    // ---- phase 2: this half's fields at the slab's nodes, in the order of
+    // memory from the 128-byte line the slab starts in ----
+    const int grp = w >= W / 2 ? 1 : 0;
+    const int64_t so = eo + kb * N2;                       // the slab's first node
+    const int m = (int)(so & 15), nn = ks * N2;
+    const double *S0 = s_u + (grp ? 0 : 3) * N3, *S1 = S0 + N3, *S2 = S1 + N3;
+    const double sgn = grp ? 1.0 : -1.0;
+    const double *mp = (grp ? a.ieps : a.imu) + so;
+    for (int v = t - grp * GL - m; v < nn; v += GL) {
+        if (v < 0) continue;
+        const unsigned uv = (unsigned)v;
+        double G[9], ko[3] = {0.0, 0.0, 0.0}, mi = 0.0;
+#pragma unroll
+        for (int c = 0; c < 9; ++c) G[c] = (a.gmet + c * a.npts + so)[uv];
+        if (MODE == GMODE_RK && (a.kflags & 1)) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) ko[c] = ld_stream<NT>(a.kbuf + (3 * grp + c) * fs + so + uv);
+        }
+        if (MODE != GMODE_CURL) mi = mp[uv];
+        const int k = kb + v / N2, q = v % N2, j = q / N1, i = q % N1;
+        // d/dr, d/ds, d/dt of the other group's three fields
+        double dr[3] = {0.0, 0.0, 0.0}, ds[3] = {0.0, 0.0, 0.0}, dt_[3] = {0.0, 0.0, 0.0};
+#pragma unroll
         for (int l = 0; l < N1; ++l) {
             const double di = s_D[i + N1 * l], dj = s_D[j + N1 * l], dk = s_D[k + N1 * l];
             const int pr = l + N1 * j + N2 * k, ps = i + N1 * l + N2 * k, pt = i + N1 * j + N2 * l;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                dr[c] += di * s_u[c * N3 + pr];
-                ds[c] += dj * s_u[c * N3 + ps];
-                dt_[c] += dk * s_u[c * N3 + pt];
-            }
+            dr[0] += di * S0[pr]; dr[1] += di * S1[pr]; dr[2] += di * S2[pr];
+            ds[0] += dj * S0[ps]; ds[1] += dj * S1[ps]; ds[2] += dj * S2[ps];
+            dt_[0] += dk * S0[pt]; dt_[1] += dk * S1[pt]; dt_[2] += dk * S2[pt];
         }
-        const int64_t p = eo + v;
-        double G[9];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) G[c] = a.gmet[(int64_t)c * a.npts + p];
         // gradient component b of field c: dr G[0 + b] + ds G[3 + b] + dt G[6 + b]
         auto dx = [&](int c, int b) { return dr[c] * G[b] + ds[c] * G[3 + b] + dt_[c] * G[6 + b]; };
-        // rH = -curl E, rE = curl H
-        double r[6];
-        r[0] = -(dx(5, 1) - dx(4, 2));
-        r[1] = -(dx(3, 2) - dx(5, 0));
-        r[2] = -(dx(4, 0) - dx(3, 1));
-        r[3] = dx(2, 1) - dx(1, 2);
-        r[4] = dx(0, 2) - dx(2, 0);
-        r[5] = dx(1, 0) - dx(0, 1);
+        double r[3];
+        r[0] = sgn * (dx(2, 1) - dx(1, 2));
+        r[1] = sgn * (dx(0, 2) - dx(2, 0));
+        r[2] = sgn * (dx(1, 0) - dx(0, 1));
         if (MODE == GMODE_CURL) {
-            const double w = a.bmw[p];
+            const double wt = a.bmw[so + v];
 #pragma unroll
-            for (int c = 0; c < 6; ++c) a.res[c * fs + p] = w * r[c];
+            for (int c = 0; c < 3; ++c) a.res[(3 * grp + c) * fs + so + v] = wt * r[c];
             continue;
         }
         // lifted fluxes of the faces through this node (reference face order)
-        auto lift = [&](int ef0, int q) {
+        const double *fl = s_f + 3 * grp * NFN;
+        auto lift = [&](int x) {
 #pragma unroll
-            for (int c = 0; c < 6; ++c) r[c] += s_f[(ef0 * N2 + q) * 6 + c];
+            for (int c = 0; c < 3; ++c) r[c] += fl[c * NFN + x];
         };
-        if (j == 0) lift(0, i + N1 * k);
-        if (i == N1 - 1) lift(1, j + N1 * k);
-        if (j == N1 - 1) lift(2, i + N1 * k);
-        if (i == 0) lift(3, j + N1 * k);
-        if (k == 0) lift(4, i + N1 * j);
-        if (k == N1 - 1) lift(5, i + N1 * j);
-        const double im = a.imu[p], ie = a.ieps[p];
+        const int kr = (k - kb) * N1, fr = N1 * ks;
+        if (j == 0) lift(kr + i);
+        if (i == N1 - 1) lift(fr + kr + j);
+        if (j == N1 - 1) lift(2 * fr + kr + i);
+        if (i == 0) lift(3 * fr + kr + j);
+        if (k == 0) lift(side + q);
+        if (k == N1 - 1) lift(side + zlo + q);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            r[c] *= im;
-            r[3 + c] *= ie;
-        }
-        if (MODE == GMODE_RESIDUAL) {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) a.res[c * fs + p] = r[c];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const int64_t x = c * fs + p;
-                const double kold = (a.kflags & 1) ? a.kbuf[x] : 0.0;
-                const double kn = a.rka * kold + a.dt * r[c];
-                if (a.kflags & 2) a.kbuf[x] = kn;
-                a.uout[x] = s_u[c * N3 + v] + a.rkb * kn;
+            const int64_t x = (3 * grp + c) * fs + so;
+            r[c] *= mi;
+            if (MODE == GMODE_RESIDUAL) {
+                (a.res + x)[uv] = r[c];
+            } else {
+                const double kn = a.rka * ko[c] + a.dt * r[c];
+                if (a.kflags & 2) st_stream<NT>(a.kbuf + x + uv, kn);
+                st_stream<NT>(a.uout + x + uv, s_u[(3 * grp + c) * N3 + kb * N2 + v] + a.rkb * kn);
             }
         }
     }

@@ -208,6 +208,24 @@ int32_t general_refuses(const nkc_handle *, const char *what) {
     return fail(NKC_ERR_UNSUPPORTED, "%s is not built for general (non-box) hexahedra", what);
 }
 
+// What nkc_info reports as a general handle's threads per workgroup: the
+// number it has always given (the kernel takes 256 to 1024 with the order).
+constexpr int GEO_INFO_LANES = 256;
+
+// Workgroups per element of the general kernel: as many slabs of levels as
+// keep one workgroup on every CU of the XCD its elements are dealt to (32
+// CUs; us per stage at 1 / this many / twice as many slabs: 50 elements at N
+// = 11, 4 slabs: 24.1 / 13.1 / 18.9; 64 at N = 7, 4: 11.2 / 6.5 / 7.0; 27 at
+// N = 10, 8: 21.4 / 10.5 / 10.5), two where the LDS holds two workgroups and
+// they still start at once (216 at N = 9: 18.9 / 17.2 / 22.6), else whole
+// elements (1000 at N = 9: 59.0, 2 slabs 59.9).
+int geo_slabs(int n1, int64_t nelt) {
+    const int64_t per_xcd = (nelt + 7) / 8, lds = 8 * (int64_t)(6 * n1 * n1 * n1 + 37 * n1 * n1);
+    const int64_t ns = std::min<int64_t>(32 / per_xcd, n1);
+    if (ns >= 2) return (int)ns;
+    return 2 * per_xcd <= 32 * std::min<int64_t>(160 * 1024 / lds, 2) ? 2 : 1;
+}
+
 // One stage on a general mesh: the per-node-geometry kernel.
 int32_t launch_geo_stage(const DevMesh &dm, const StageArgs &a, int gmode, hipStream_t s) {
     GeoArgs g{};
@@ -231,7 +249,8 @@ int32_t launch_geo_stage(const DevMesh &dm, const StageArgs &a, int gmode, hipSt
     g.rkb = a.rkb;
     g.dt = a.dt;
     g.kflags = a.kflags;
-    if (!launch_geo(g, dm.n1, gmode, 8 * g.per_xcd, s))
+    g.nslab = geo_slabs(dm.n1, dm.nelt);
+    if (!launch_geo(g, dm.n1, gmode, dm.nt, 8 * g.per_xcd * g.nslab, s))
         return fail(NKC_ERR_UNSUPPORTED, "polynomial order N=%d not built for general hexahedra", dm.n1 - 1);
     HIPCHK(hipGetLastError());
     return NKC_OK;
@@ -2006,7 +2025,7 @@ int32_t nkc_info(nkc_handle *h, int64_t out[8]) {
     out[0] = h->m.npts;
     out[1] = h->m.mat;
     out[2] = 1;
-    out[3] = h->m.general ? GEO_BS : stage_block(n1);
+    out[3] = h->m.general ? GEO_INFO_LANES : stage_block(n1);
     out[4] = h->m.general ? (int64_t)sizeof(double) * (6 * n1 * n1 * n1 + 37 * n1 * n1)
                           : (int64_t)sizeof(double) * (6 * n1 * n1 * n1 + 25 * n1 * n1);
     out[5] = h->use_graph ? 1 : 0;
