@@ -296,6 +296,11 @@ int32_t nkc_adjoint_get_drude(nkc_handle *h, double *ga, double *gb);
  * nkc_adjoint_forward until nkc_adjoint_release, the next forward, a
  * set_* call or nkc_destroy; a cap (max_steps > 0) holds it to the
  * checkpoints plus one window of 5 max_steps stages.
+ * Between a set_* call (materials, source, Drude region) or the next forward
+ * and that handle's next nkc_adjoint_forward, at most a quarter of the
+ * device's memory may wait allocated for reuse; nkc_adjoint_release and
+ * nkc_destroy free it, and so does any allocation of this library that
+ * would otherwise fail.
  * nkc_adjoint_info: out[5] = {every, segments, S, K, device bytes held}. */
 int32_t nkc_adjoint_set_store(nkc_handle *h, int64_t max_steps);
 /* Free everything the adjoint holds (checkpoints, stage store, adjoint

@@ -75,14 +75,79 @@ bool supported_n1(int n1) { return n1 >= 4 && n1 <= 10; }
 // Orders the general-hexahedra kernel takes (nkc_create only).
 bool supported_n1_general(int n1) { return n1 >= GEO_MIN_N1 && n1 <= GEO_MAX_N1; }
 
+// Adjoint buffers between two passes.  An adjoint pass holds tens of GB and
+// every pass frees and allocates the same sizes: mapping 40 GB took 50 to
+// 400 ms, as much as the pass itself (16^3, N = 7, 40 steps).  When a set_*
+// call or the next forward drops a handle's adjoint, its buffers wait here
+// for that handle's next nkc_adjoint_forward, which takes those whose size
+// it needs and frees the rest.  At most a quarter of a device's memory
+// waits; nkc_adjoint_release and nkc_destroy give a handle's buffers back,
+// and an allocation that finds the device full takes back all of them.
+struct IdleBlock {
+    const void *owner;
+    int device;
+    double *p;
+    size_t bytes;
+};
+std::mutex idle_mu;
+std::vector<IdleBlock> idle_blocks;
+
+template <class F>
+size_t idle_drop(F which) {
+    std::lock_guard<std::mutex> lock(idle_mu);
+    size_t n = 0;
+    for (size_t b = idle_blocks.size(); b-- > 0;)
+        if (which(idle_blocks[b])) {
+            (void)hipFree(idle_blocks[b].p);
+            idle_blocks.erase(idle_blocks.begin() + b);
+            ++n;
+        }
+    return n;
+}
+
+double *idle_take(const void *owner, size_t bytes) {
+    std::lock_guard<std::mutex> lock(idle_mu);
+    for (size_t b = 0; b < idle_blocks.size(); ++b)
+        if (idle_blocks[b].owner == owner && idle_blocks[b].bytes == bytes) {
+            double *p = idle_blocks[b].p;
+            idle_blocks.erase(idle_blocks.begin() + b);
+            return p;
+        }
+    return nullptr;
+}
+
+// Bytes waiting for `owner` (any handle's on the device when null).
+size_t idle_bytes(const void *owner, int device) {
+    std::lock_guard<std::mutex> lock(idle_mu);
+    size_t n = 0;
+    for (const IdleBlock &b : idle_blocks)
+        if (owner ? b.owner == owner : b.device == device) n += b.bytes;
+    return n;
+}
+
+// hipMalloc that takes back the idle adjoint buffers when the device is full.
+template <class T>
+hipError_t dev_malloc(T **p, size_t bytes) {
+    hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        int dev = 0;
+        (void)hipGetDevice(&dev);
+        if (idle_drop([&](const IdleBlock &b) { return b.device == dev; })) {
+            (void)hipGetLastError();
+            e = hipMalloc((void **)p, bytes);
+        }
+    }
+    return e;
+}
+
 int32_t dev_alloc(double **p, size_t n) {
-    HIPCHK(hipMalloc((void **)p, sizeof(double) * n));
+    HIPCHK(dev_malloc(p, sizeof(double) * n));
     return NKC_OK;
 }
 
 template <class T>
 int32_t upload(T **dst, const std::vector<T> &src) {
-    HIPCHK(hipMalloc((void **)dst, sizeof(T) * (src.empty() ? 1 : src.size())));
+    HIPCHK(dev_malloc(dst, sizeof(T) * (src.empty() ? 1 : src.size())));
     if (!src.empty()) {
         const hipError_t e = hipMemcpy(*dst, src.data(), sizeof(T) * src.size(), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
@@ -133,9 +198,9 @@ int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     dm.jac = m.jac;
     dm.w = m.w;
     const size_t ub = sizeof(double) * 6 * (size_t)dm.fs;
-    HIPCHK(hipMalloc((void **)&dm.u[0], ub));
-    HIPCHK(hipMalloc((void **)&dm.u[1], ub));
-    HIPCHK(hipMalloc((void **)&dm.k, ub));
+    HIPCHK(dev_malloc(&dm.u[0], ub));
+    HIPCHK(dev_malloc(&dm.u[1], ub));
+    HIPCHK(dev_malloc(&dm.k, ub));
     HIPCHK(hipMemset(dm.u[0], 0, ub));
     HIPCHK(hipMemset(dm.u[1], 0, ub));
     HIPCHK(hipMemset(dm.k, 0, ub));
@@ -582,6 +647,7 @@ struct nkc_handle {
         std::vector<int64_t> slot_id;
         int cur_slot = 0;                 // slot queue_step_store writes
         size_t bytes = 0;                 // device bytes held by the adjoint
+        std::vector<std::pair<double *, size_t>> blocks;   // every buffer below, with its bytes
         bool have_grad = false;           // a backward sweep has filled the gradients
         double dt = 0.0, t0 = 0.0;
         double *ckpt = nullptr;           // nseg x 6 fs: the state at the start of each segment
@@ -757,11 +823,20 @@ int32_t capture(nkc_handle *h, double dt) {
     return NKC_OK;
 }
 
-void free_adjoint(nkc_handle *h) {
+// keep: leave the buffers to this handle's next nkc_adjoint_forward (see
+// IdleBlock); a caller that keeps them has waited for the handle's stream or
+// queues its own work on it.
+void free_adjoint(nkc_handle *h, bool keep = false) {
     auto &A = h->adj;
-    double *p[] = {A.ckpt, A.st_u, A.st_r, A.lam[0], A.lam[1], A.kap[0], A.kap[1], A.geps, A.gmu, A.ufin,
-                   A.kfin, A.ckJ, A.stJ, A.lamJ, A.kapJ, A.gA, A.gB, A.Jfin, A.kJfin, A.sub, A.subJ};
-    for (double *q : p) (void)hipFree(q);
+    size_t fr = 0, tot = 0;
+    if (keep && !A.blocks.empty() && hipMemGetInfo(&fr, &tot) == hipSuccess &&
+        A.bytes + idle_bytes(nullptr, h->device) <= tot / 4) {
+        std::lock_guard<std::mutex> lock(idle_mu);
+        for (const auto &b : A.blocks) idle_blocks.push_back({h, h->device, b.first, b.second});
+    } else {
+        for (const auto &b : A.blocks) (void)hipFree(b.first);
+    }
+    if (!keep) idle_drop([&](const IdleBlock &b) { return b.owner == h; });
     A = nkc_handle::Adj();
 }
 
@@ -858,7 +933,7 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
         if ((rc = dev_mesh_upload(hm, h->m))) break;
         // element Jacobians and GLL weights of bm1 for the diagnostics
         if ((rc = upload(&h->djac, hm.jac)) || (rc = upload(&h->dw, hm.w))) break;
-        if (hipMalloc((void **)&h->tdev, 14 * sizeof(double)) != hipSuccess ||
+        if (dev_malloc(&h->tdev, 14 * sizeof(double)) != hipSuccess ||
             hipMemset(h->tdev, 0, 14 * sizeof(double)) != hipSuccess ||
             hipStreamSynchronize(nullptr) != hipSuccess) { rc = fail(NKC_ERR_HIP, "hipMalloc time"); break; }
     } while (0);
@@ -1222,7 +1297,7 @@ int32_t nkc_residual(nkc_handle *h, double rktime, double *reshn, double *resen,
     if (!h || !reshn || !resen) return fail(NKC_ERR_ARG, "null handle or output");
     const DevMesh &m = h->m;
     if (ld < m.npts) return fail(NKC_ERR_ARG, "ld < npts");
-    if (!h->res) HIPCHK(hipMalloc((void **)&h->res, sizeof(double) * 6 * m.fs));
+    if (!h->res) HIPCHK(dev_malloc(&h->res, sizeof(double) * 6 * m.fs));
     HIPCHK(hipStreamSynchronize(h->stream));
     if (uses_time(h)) {
         hipLaunchKernelGGL(stage_time, dim3(1), dim3(1), 0, h->stream, h->tdev, rktime, src_time(h));
@@ -1244,7 +1319,7 @@ int32_t nkc_curl(nkc_handle *h, double *reshn, double *resen, int64_t ld) {
     if (ld < m.npts) return fail(NKC_ERR_ARG, "ld < npts");
     int32_t rc;
     if ((rc = ensure_diag(h))) return rc;
-    if (!h->res) HIPCHK(hipMalloc((void **)&h->res, sizeof(double) * 6 * m.fs));
+    if (!h->res) HIPCHK(dev_malloc(&h->res, sizeof(double) * 6 * m.fs));
     HIPCHK(hipStreamSynchronize(h->stream));
     if (m.general) {
         StageArgs a = mesh_args(m);
@@ -1276,7 +1351,7 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     if (!h) return fail(NKC_ERR_ARG, "null handle");
     if (h->m.general && (amp != nullptr)) return general_refuses(h, "a source");
     HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h);                      // the stored trajectory has the old source
+    free_adjoint(h, true);                 // the stored trajectory has the old source
     h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->src_off); h->src_off = nullptr;
     (void)hipFree(h->src_amp); h->src_amp = nullptr;
@@ -1318,7 +1393,7 @@ int32_t nkc_set_source_time(nkc_handle *h, int32_t kind, double omega, double ph
     if (kind != 0 && kind != 1) return fail(NKC_ERR_ARG, "source time kind %d not 0 or 1", kind);
     if (!std::isfinite(omega) || !std::isfinite(phase)) return fail(NKC_ERR_ARG, "source omega/phase not finite");
     HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h);                      // the stored trajectory has the old source
+    free_adjoint(h, true);                 // the stored trajectory has the old source
     h->src_kind = kind;
     h->src_om = omega;
     h->src_ph = phase;
@@ -1367,7 +1442,7 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     (void)hipFree(h->dkJ); h->dkJ = nullptr;
     (void)hipFree(h->dpar); h->dpar = nullptr;
     (void)hipFree(h->dresJ); h->dresJ = nullptr;
-    free_adjoint(h);                      // the stored trajectory has the old region
+    free_adjoint(h, true);                 // the stored trajectory has the old region
     h->m.layout = -1;                     // the step's kernel instance may change
     h->ndrude = 0;
     h->ndelem = 0;
@@ -2097,7 +2172,7 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps_in, const double *mu_
     for (int64_t p = 0; p < npts; ++p)
         if (!(eps[p] > 0.0) || !(mu[p] > 0.0)) return fail(NKC_ERR_ARG, "material not positive at node %lld", (long long)p);
     HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h);                      // the stored trajectory has the old materials
+    free_adjoint(h, true);                 // the stored trajectory has the old materials
     // the new tables replace the old ones (host and device) only once all
     // three are on the device, so a failed upload leaves the handle as it was
     HostMesh hm = h->hm;
@@ -2129,8 +2204,22 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps_in, const double *mu_
 namespace {
 
 int32_t dev_alloc_counted(nkc_handle *h, double **p, size_t n) {
-    h->adj.bytes += sizeof(double) * n;
-    return dev_alloc(p, n);
+    const size_t bytes = sizeof(double) * n;
+    *p = idle_take(h, bytes);
+    int32_t rc;
+    if (!*p && (rc = dev_alloc(p, n))) return rc;
+    h->adj.bytes += bytes;
+    h->adj.blocks.push_back({*p, bytes});
+    return NKC_OK;
+}
+
+// Free device memory as the adjoint's layout counts it: what is free and
+// what waits for this handle.
+int32_t adjoint_room(const nkc_handle *h, size_t *fr) {
+    size_t tot = 0;
+    HIPCHK(hipMemGetInfo(fr, &tot));
+    *fr += idle_bytes(h, h->device);
+    return NKC_OK;
 }
 
 // Every buffer of the adjoint for the layout fixed by nkc_adjoint_forward:
@@ -2167,8 +2256,8 @@ int32_t alloc_adjoint(nkc_handle *h) {
     if (h->adj_store_cap > 0) {
         S = std::min(S, h->adj_store_cap);
     } else {
-        size_t fr = 0, tot = 0;
-        HIPCHK(hipMemGetInfo(&fr, &tot));
+        size_t fr = 0;
+        if ((rc = adjoint_room(h, &fr))) return rc;
         const size_t state = sizeof(double) * (blk + jsz);
         const size_t room = (size_t)(0.7 * (double)fr);
         // S steps of store plus ceil(every / S) window starts
@@ -2181,8 +2270,8 @@ int32_t alloc_adjoint(nkc_handle *h) {
     // other half stays free for co-resident allocations)
     int64_t K = 1;
     if (S == A.every && h->adj_store_cap == 0) {
-        size_t fr = 0, tot = 0;
-        HIPCHK(hipMemGetInfo(&fr, &tot));
+        size_t fr = 0;
+        if ((rc = adjoint_room(h, &fr))) return rc;
         const size_t win = per_step * S + sizeof(double) * blk;
         K = std::max<int64_t>(1, std::min<int64_t>(A.nseg, (int64_t)((0.5 * (double)fr) / (double)win)));
     }
@@ -2196,8 +2285,8 @@ int32_t alloc_adjoint(nkc_handle *h) {
     // each window once, with no pass to rebuild its segment's window starts
     A.sub_all = false;
     if (A.nsub_max > 1) {
-        size_t fr = 0, tot = 0;
-        HIPCHK(hipMemGetInfo(&fr, &tot));
+        size_t fr = 0;
+        if ((rc = adjoint_room(h, &fr))) return rc;
         const size_t need = sizeof(double) * (blk + jsz) * (size_t)(A.nseg * A.nsub_max);
         A.sub_all = need <= fr / 4;
     }
@@ -2207,6 +2296,7 @@ int32_t alloc_adjoint(nkc_handle *h) {
         if ((rc = dev_alloc_counted(h, &A.stJ, jsz * 5 * S * K))) return rc;
         if ((rc = dev_alloc_counted(h, &A.subJ, jsz * nsub))) return rc;
     }
+    idle_drop([&](const IdleBlock &b) { return b.owner == h; });   // sizes this layout has no use for
     return NKC_OK;
 }
 
@@ -2370,7 +2460,7 @@ int32_t nkc_adjoint_forward(nkc_handle *h, double *time, double dt, int64_t nste
     if (h->npml) return fail(NKC_ERR_UNSUPPORTED, "the adjoint of a PML is not built");
     if (h->ninc) return fail(NKC_ERR_UNSUPPORTED, "the adjoint with an incident field is not built");
     if (h->ngraph) return fail(NKC_ERR_UNSUPPORTED, "the adjoint with a graphene sheet is not built");
-    free_adjoint(h);
+    free_adjoint(h, true);
     auto &A = h->adj;
     A.nsteps = nsteps;
     A.every = every < nsteps ? every : nsteps;
@@ -2610,7 +2700,7 @@ int32_t nkc_batch_create(int32_t ncav, const nkc_box_desc *d, nkc_batch **out) {
         cat.nelt = off;
         b->bins.emplace_back();
         if ((rc = dev_mesh_upload(cat, b->bins.back()))) break;
-        if (hipMalloc((void **)&b->bins.back().dt_e, sizeof(double) * cat.nelt) != hipSuccess) {
+        if (dev_malloc(&b->bins.back().dt_e, sizeof(double) * cat.nelt) != hipSuccess) {
             rc = fail(NKC_ERR_HIP, "hipMalloc dt table");
             break;
         }
