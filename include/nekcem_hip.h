@@ -125,6 +125,10 @@ int32_t nkc_set_state(nkc_handle *h, const double *hn, const double *en,
 int32_t nkc_get_state(nkc_handle *h, double *hn, double *en, double *khn,
                       double *ken, int64_t ld);
 
+/* The six fields at n nodes (0-based), out[6][n] = (Hx, Hy, Hz, Ex, Ey, Ez);
+ * both arrays in host or device memory. */
+int32_t nkc_get_state_at(nkc_handle *h, int64_t n, const int64_t *nodes, double *out);
+
 /* nsteps calls of cem_maxwell_op_rk (src/cem_maxwell.F:327-345): 5-stage
  * low-storage RK per step, each stage one fused kernel, the step replayed
  * from a captured hipGraph.  *time += nsteps*dt (time_advancing_pde,
@@ -283,6 +287,11 @@ int32_t nkc_adjoint_forward(nkc_handle *h, double *time, double dt, int64_t nste
                             int64_t every);
 int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *lamE,
                              int64_t ld, double *geps, double *gmu);
+/* nkc_adjoint_backward for a loss of the fields at n nodes (0-based, host or
+ * device memory, like seeds[6][n] = dL/d(Hx, Hy, Hz, Ex, Ey, Ez) there):
+ * the other seeds are zero; a node listed twice gets both of its seeds. */
+int32_t nkc_adjoint_backward_at(nkc_handle *h, int64_t n, const int64_t *nodes,
+                                const double *seeds, double *geps, double *gmu);
 int32_t nkc_adjoint_get_drude(nkc_handle *h, double *ga, double *gb);
 /* A segment is reversed in windows of S <= every steps whose 5 S stages (state
  * and residual, plus the Drude current) are kept at once; window starts are

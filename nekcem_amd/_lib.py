@@ -68,6 +68,7 @@ SIGNATURES = [
     ("nkc_destroy", C.c_int32, [C.c_void_p]),
     ("nkc_set_state", C.c_int32, [C.c_void_p, _dp, _dp, _dp, _dp, C.c_int64]),
     ("nkc_get_state", C.c_int32, [C.c_void_p, _dp, _dp, _dp, _dp, C.c_int64]),
+    ("nkc_get_state_at", C.c_int32, [C.c_void_p, C.c_int64, C.POINTER(C.c_int64), _dp]),
     ("nkc_step", C.c_int32, [C.c_void_p, _dp, C.c_double, C.c_int64]),
     ("nkc_residual", C.c_int32, [C.c_void_p, C.c_double, _dp, _dp, C.c_int64]),
     ("nkc_curl", C.c_int32, [C.c_void_p, _dp, _dp, C.c_int64]),
@@ -77,6 +78,7 @@ SIGNATURES = [
     ("nkc_set_materials", C.c_int32, [C.c_void_p, _dp, _dp]),
     ("nkc_adjoint_forward", C.c_int32, [C.c_void_p, _dp, C.c_double, C.c_int64, C.c_int64]),
     ("nkc_adjoint_backward", C.c_int32, [C.c_void_p, _dp, _dp, C.c_int64, _dp, _dp]),
+    ("nkc_adjoint_backward_at", C.c_int32, [C.c_void_p, C.c_int64, C.POINTER(C.c_int64), _dp, _dp, _dp]),
     ("nkc_adjoint_get_drude", C.c_int32, [C.c_void_p, _dp, _dp]),
     ("nkc_set_lorentz", C.c_int32, [C.c_void_p, C.c_int64, _ip, _dp, _dp, _dp]),
     ("nkc_get_lorentz", C.c_int32, [C.c_void_p, _dp, _dp, _dp]),

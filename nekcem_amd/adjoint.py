@@ -20,9 +20,10 @@ cem_maxwell_op_rk (src/cem_maxwell.F:327-345) with a usersrc-style source.
 PyTorch is only the autograd plumbing.  The tensors stay where they are:
 with GPU tensors the parameters, the initial state, the probe fields, the
 adjoint seeds and the gradients go between torch and the library as device
-pointers (device-to-device copies); only the material and Drude tables,
-which the library builds on the host, stage their per-node inputs through
-host memory.  CPU tensors go through the same calls as host pointers.
+pointers (device-to-device copies); only the Drude tables, which the library
+builds on the host, stage their per-node inputs through host memory.  Of the
+final state only the probes' values leave the library, and of the adjoint's
+seeds only theirs enter it.  CPU tensors go through the same calls as host pointers.
 torch ships its own HIP runtime; the two share one HSA runtime, and torch
 sees the GPU, only if torch's is loaded first: import torch (and call
 torch.cuda.init()) before the first MaxwellSolver of the process.
@@ -107,6 +108,10 @@ if torch is not None:
         """double* of a contiguous float64 tensor (host or device memory)."""
         return None if t is None else C.cast(C.c_void_p(t.data_ptr()), _dp)
 
+    def _iptr(t):
+        """int64_t* of a contiguous int64 tensor."""
+        return C.cast(C.c_void_p(t.data_ptr()), C.POINTER(C.c_int64))
+
     def _ready(*ts):
         """The library copies synchronously, outside torch's streams: let
         torch's pending work on these tensors finish first."""
@@ -125,6 +130,9 @@ if torch is not None:
             E0 = torch.as_tensor(np.asarray(problem.E0), dtype=torch.float64, device=dev).reshape(3, n).contiguous()
             pr = torch.as_tensor(np.asarray(problem.probes), dtype=torch.long, device=dev)
             extra = {}
+            if pr.dim() == 1 and len(pr) and 0 <= int(pr.min()) and int(pr.max()) < n:
+                # each probe node once, and where it stands in that list
+                extra["nodes"], extra["which"] = torch.unique(pr, return_inverse=True)
             if isinstance(problem, DrudeProbeProblem):
                 extra["owner"] = torch.as_tensor(np.asarray(problem.owner), dtype=torch.long, device=dev)
                 extra["dindex"] = np.ascontiguousarray(np.asarray(problem.dindex) + 1, dtype=np.int32)
@@ -141,10 +149,16 @@ if torch is not None:
 
     def _probe_fields(problem, dev):
         """The six fields at the probes after the forward, a (6, nprobes)
-        tensor on dev: the state copied device to device, then gathered."""
+        tensor on dev, gathered on the device."""
         s = problem.solver
         n = s.npts
-        _, _, pr, _ = _problem_tensors(problem, dev)
+        _, _, pr, extra = _problem_tensors(problem, dev)
+        if "nodes" in extra:
+            out = torch.empty((6, len(pr)), dtype=torch.float64, device=dev)
+            _ready(out)
+            _lib.check(s._L.nkc_get_state_at(s._h, len(pr), _iptr(pr.contiguous()), _ptr(out)))
+            return out
+        # torch's own indexing rules for every other list of probes
         H = torch.empty((3, n), dtype=torch.float64, device=dev)
         E = torch.empty((3, n), dtype=torch.float64, device=dev)
         _ready(H)
@@ -157,12 +171,18 @@ if torch is not None:
         s = problem.solver
         n = s.npts
         dev = grad_out.device
-        _, _, pr, _ = _problem_tensors(problem, dev)
+        _, _, pr, extra = _problem_tensors(problem, dev)
         g = grad_out.detach().to(torch.float64)
-        lamH = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[:3])
-        lamE = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[3:])
         ge = torch.empty(n, dtype=torch.float64, device=dev) if want_material else None
         gm = torch.empty(n, dtype=torch.float64, device=dev) if want_material else None
+        if "nodes" in extra:
+            nodes = extra["nodes"]
+            seeds = torch.zeros((6, len(nodes)), dtype=torch.float64, device=dev).index_add_(1, extra["which"], g)
+            _ready(seeds)
+            _lib.check(s._L.nkc_adjoint_backward_at(s._h, len(nodes), _iptr(nodes), _ptr(seeds), _ptr(ge), _ptr(gm)))
+            return ge, gm
+        lamH = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[:3])
+        lamE = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[3:])
         _ready(lamH)
         _lib.check(s._L.nkc_adjoint_backward(s._h, _ptr(lamH), _ptr(lamE), n, _ptr(ge), _ptr(gm)))
         return ge, gm

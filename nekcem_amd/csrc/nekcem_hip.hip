@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 #include <array>
+#include <functional>
 #include <mutex>
 
 #include "../../include/nekcem_hip.h"
@@ -25,6 +26,7 @@
 #include "diag_kernels.hpp"
 #include "geo_kernel.hpp"
 #include "geo_launch.hpp"
+#include "material_kernels.hpp"
 #include "mesh_tables.hpp"
 #include "order_launch.hpp"
 #include "restart_io.hpp"
@@ -615,6 +617,10 @@ struct nkc_handle {
     HostMesh hm;
     double C0 = 1.0;
     double *yz = nullptr;                 // (sqrt(eps/mu), sqrt(mu/eps)) per ieps entry, adjoint only
+    bool yz_ok = false;                   // formed from the present materials
+    bool hm_stale = false;                // hm.ieps/imu are older than the device's tables
+    double *list = nullptr;               // node_list: room for `listed` nodes and their values
+    int64_t listed = 0;
     int64_t adj_store_cap = 0;            // cap on the adjoint's stage-store window (0: from free memory)
     int32_t adj_grads = 3;                // bit 0: eps/mu gradients, bit 1: Drude gradients
     double tune_us[NLAYOUT] = {NAN, NAN, NAN, NAN, NAN, NAN, NAN, NAN};   // tuner's stage times per layout
@@ -840,17 +846,70 @@ void free_adjoint(nkc_handle *h, bool keep = false) {
     A = nkc_handle::Adj();
 }
 
-// Admittance/impedance pairs for the adjoint's material gradient, built
-// from the same inverse-material tables the stage kernel reads.
+// Pinned per-workgroup results of a check over the nodes.
+int32_t check_buffer(nkc_handle *h) {
+    if (!h->red) HIPCHK(hipHostMalloc((void **)&h->red, sizeof(unsigned long long) * CHECK_BLOCKS, hipHostMallocDefault));
+    return NKC_OK;
+}
+
+// One lane per item, at most 8 workgroups of 256 per CU.
+dim3 item_grid(int64_t n, int rows = 1) {
+    return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(2048, (n + 255) / 256)), rows);
+}
+
+// Entries of the handle's material tables: per node or per element.
+int64_t material_entries(const nkc_handle *h) { return h->m.mat == MAT_NODE ? h->m.npts : h->m.nelt; }
+
 int32_t ensure_yz(nkc_handle *h) {
-    if (h->yz) return NKC_OK;
-    const size_t n = h->hm.ieps.size();
-    std::vector<double> yz(2 * n);
-    for (size_t x = 0; x < n; ++x) {
-        yz[2 * x] = std::sqrt(h->hm.imu[x] / h->hm.ieps[x]);
-        yz[2 * x + 1] = std::sqrt(h->hm.ieps[x] / h->hm.imu[x]);
+    if (h->yz_ok) return NKC_OK;
+    const int64_t n = material_entries(h);
+    int32_t rc;
+    if (!h->yz && (rc = dev_alloc(&h->yz, 2 * n))) return rc;
+    hipLaunchKernelGGL(admittance_pairs, item_grid(n), dim3(256), 0, h->stream, (const double *)h->m.ieps,
+                       (const double *)h->m.imu, n, h->yz);
+    HIPCHK(hipGetLastError());
+    h->yz_ok = true;
+    return NKC_OK;
+}
+
+// The inverse materials on the host, for the set-up of a PML or a sheet;
+// nkc_set_materials leaves them on the device.
+int32_t host_materials(nkc_handle *h) {
+    if (!h->hm_stale) return NKC_OK;
+    const int64_t n = h->m.npts;
+    std::vector<double> ie(n), im(n);
+    HIPCHK(hipStreamSynchronize(h->stream));
+    HIPCHK(hipMemcpy(ie.data(), h->m.ieps, sizeof(double) * n, hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(im.data(), h->m.imu, sizeof(double) * n, hipMemcpyDeviceToHost));
+    h->hm.ieps = std::move(ie);
+    h->hm.imu = std::move(im);
+    h->hm_stale = false;
+    return NKC_OK;
+}
+
+// Node lists and their values on the device, 7 n doubles' worth, kept and
+// grown as lists need (nkc_get_state_at, nkc_adjoint_backward_at).
+int32_t node_list(nkc_handle *h, int64_t n, const int64_t *nodes, int64_t **dn, double **dv) {
+    std::vector<int64_t> hn;
+    hn.resize(n);
+    HIPCHK(hipMemcpy(hn.data(), nodes, sizeof(int64_t) * n, hipMemcpyDefault));
+    for (int64_t i = 0; i < n; ++i)
+        if (hn[i] < 0 || hn[i] >= h->m.npts)
+            return fail(NKC_ERR_ARG, "listed node %lld is not a node (%lld of them)", (long long)hn[i],
+                        (long long)h->m.npts);
+    HIPCHK(hipStreamSynchronize(h->stream));
+    if (h->listed < n) {
+        (void)hipFree(h->list);
+        h->list = nullptr;
+        h->listed = 0;
+        const int32_t rc = dev_alloc(&h->list, 7 * (size_t)n);
+        if (rc) return rc;
+        h->listed = n;
     }
-    return upload(&h->yz, yz);
+    *dn = reinterpret_cast<int64_t *>(h->list);
+    *dv = h->list + n;
+    HIPCHK(hipMemcpy(*dn, hn.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice));
+    return NKC_OK;
 }
 
 void free_handle(nkc_handle *h) {
@@ -858,6 +917,8 @@ void free_handle(nkc_handle *h) {
     free_adjoint(h);
     (void)hipFree(h->yz);
     h->yz = nullptr;
+    (void)hipFree(h->list);
+    h->list = nullptr;
     dev_mesh_free(h->m);
     (void)hipFree(h->res); (void)hipFree(h->tdev);
     if (h->red) (void)hipHostFree(h->red);
@@ -1256,6 +1317,23 @@ int32_t nkc_get_state(nkc_handle *h, double *hn, double *en, double *khn, double
         rc = copy_fields_d2h(m.k, m.fs, 0, khn ? khn : tmp.data(), ken ? ken : tmp.data(), m.npts, ld);
         if (rc) return rc;
     }
+    return NKC_OK;
+}
+
+int32_t nkc_get_state_at(nkc_handle *h, int64_t n, const int64_t *nodes, double *out) {
+    if (!h || n < 0 || (n && (!nodes || !out))) return fail(NKC_ERR_ARG, "null handle or array");
+    if (n == 0) return NKC_OK;
+    int64_t *dn = nullptr;
+    double *dv = nullptr;
+    const int32_t rc = node_list(h, n, nodes, &dn, &dv);
+    if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(nullptr));
+    hipLaunchKernelGGL(gather_nodes, item_grid(n, 6), dim3(256), 0, h->stream, (const double *)h->m.u[h->cur], h->m.fs,
+                       (const int64_t *)dn, n, dv);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(h->stream));
+    HIPCHK(hipMemcpy(out, dv, sizeof(double) * 6 * n, hipMemcpyDefault));
+    HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
 }
 
@@ -1801,6 +1879,7 @@ int32_t nkc_setup_pml(nkc_handle *h, const int8_t *pml_face, int32_t thick, doub
     std::vector<double> sig;
     double ext[12];
     std::string err;
+    if ((rc = host_materials(h))) return rc;
     if ((rc = pml_tables(h->hm, h->hxyz.data(), h->m.fs, pml_face, thick, order, referr, elems, sig, ext, err)))
         return fail(rc, "%s", err.c_str());
     if (extents)
@@ -1950,6 +2029,7 @@ int32_t nkc_set_graphene(nkc_handle *h, int64_t ngraph, const int32_t *graphinde
             for (int c = 0; c < 3; ++c) st[(b * 15 + 3 * sl + c) * n2 + q] = fjn[j + ld * (c + 3 * (sl + 1))];
     }
     h->gr_face = face;
+    if ((rc = host_materials(h))) return rc;
     sheet_coefs(h, par);
     const std::vector<double> zero(st.size(), 0.0);
     if ((rc = upload(&h->gpar, par)) || (rc = upload(&h->gA[h->cur], st)) || (rc = upload(&h->gA[h->cur ^ 1], st)) ||
@@ -2068,7 +2148,8 @@ int32_t nkc_restart_read(nkc_handle *h, const char *path, int32_t *istep, int32_
 
 int32_t nkc_check_finite(nkc_handle *h, double *maxabs) {
     if (!h) return fail(NKC_ERR_ARG, "null handle");
-    if (!h->red) HIPCHK(hipHostMalloc((void **)&h->red, sizeof(unsigned long long) * CHECK_BLOCKS, hipHostMallocDefault));
+    int32_t rc = check_buffer(h);
+    if (rc) return rc;
     const int nb = (int)std::min<int64_t>(CHECK_BLOCKS, (h->m.npts + 255) / 256);
     hipLaunchKernelGGL(maxabs_kernel, dim3(nb), dim3(256), 0, h->stream, h->m.u[h->cur], h->m.fs, h->m.npts, h->red);
     HIPCHK(hipGetLastError());
@@ -2160,40 +2241,81 @@ int32_t nkc_tune(nkc_handle *h, double *out) {
     return NKC_OK;
 }
 
-int32_t nkc_set_materials(nkc_handle *h, const double *eps_in, const double *mu_in) {
-    if (!h || !eps_in || !mu_in) return fail(NKC_ERR_ARG, "null handle or material array");
+namespace {
+
+int32_t bad_node(int64_t p) { return fail(NKC_ERR_ARG, "material not positive at node %lld", (long long)p); }
+
+}  // namespace
+
+int32_t nkc_set_materials(nkc_handle *h, const double *eps, const double *mu) {
+    if (!h || !eps || !mu) return fail(NKC_ERR_ARG, "null handle or material array");
     if (h->m.general && (true)) return general_refuses(h, "replacing the materials");
-    const int64_t npts = h->m.npts;
-    // the tables are built on the host from the caller's arrays (host or device memory)
-    std::vector<double> eps_h, mu_h;
-    int32_t rc0;
-    if ((rc0 = stage_host(eps_h, eps_in, npts)) || (rc0 = stage_host(mu_h, mu_in, npts))) return rc0;
-    const double *eps = eps_h.data(), *mu = mu_h.data();
-    for (int64_t p = 0; p < npts; ++p)
-        if (!(eps[p] > 0.0) || !(mu[p] > 0.0)) return fail(NKC_ERR_ARG, "material not positive at node %lld", (long long)p);
-    HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h, true);                 // the stored trajectory has the old materials
-    // the new tables replace the old ones (host and device) only once all
-    // three are on the device, so a failed upload leaves the handle as it was
-    HostMesh hm = h->hm;
-    set_node_materials(hm, eps, mu, h->C0);
-    double *fco = nullptr, *ieps = nullptr, *imu = nullptr;
+    DevMesh &m = h->m;
+    const int64_t npts = m.npts;
     int32_t rc;
-    if ((rc = upload(&fco, hm.fco)) || (rc = upload(&ieps, hm.ieps)) || (rc = upload(&imu, hm.imu))) {
-        (void)hipFree(fco); (void)hipFree(ieps); (void)hipFree(imu);
-        return rc;
+    if ((rc = check_buffer(h))) return rc;
+    HIPCHK(hipStreamSynchronize(h->stream));
+    // eps and mu go to the device, where they are checked before anything of
+    // the handle changes, and become the tables in place
+    double *ieps = nullptr, *imu = nullptr, *fco = m.mat == MAT_NODE ? m.fco : nullptr;
+    auto give_back = [&](int32_t code) {
+        (void)hipFree(ieps);
+        (void)hipFree(imu);
+        return code;
+    };
+    if ((rc = dev_alloc(&ieps, npts)) || (rc = dev_alloc(&imu, npts)) ||
+        (!fco && (rc = dev_alloc(&fco, m.nelt * 24 * (size_t)m.n1 * m.n1)))) {
+        if (h->adj.blocks.empty()) return give_back(rc);
+        // the stored trajectory, which this call drops, holds the memory: check on the host, then drop it
+        (void)give_back(rc);
+        (void)hipGetLastError();
+        ieps = imu = nullptr;
+        std::vector<double> he, hmu;
+        if ((rc = stage_host(he, eps, npts)) || (rc = stage_host(hmu, mu, npts))) return rc;
+        for (int64_t p = 0; p < npts; ++p)
+            if (!(he[p] > 0.0) || !(hmu[p] > 0.0)) return bad_node(p);
+        free_adjoint(h);
+        return nkc_set_materials(h, eps, mu);
     }
-    h->hm = std::move(hm);
-    (void)hipFree(h->yz); h->yz = nullptr;
-    (void)hipFree(h->m.fco); (void)hipFree(h->m.ieps); (void)hipFree(h->m.imu);
-    h->m.fco = fco;
-    h->m.ieps = ieps;
-    h->m.imu = imu;
-    h->m.mat = MAT_NODE;
+    auto give_all_back = [&](int32_t code) {
+        if (fco != m.fco) (void)hipFree(fco);
+        return give_back(code);
+    };
+    const size_t bytes = sizeof(double) * npts;
+    if (hipMemcpy(ieps, eps, bytes, hipMemcpyDefault) != hipSuccess ||
+        hipMemcpy(imu, mu, bytes, hipMemcpyDefault) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+        return give_all_back(fail(NKC_ERR_HIP, "copy of the materials: %s", hipGetErrorString(hipGetLastError())));
+    const int nb = (int)std::min<int64_t>(CHECK_BLOCKS, (npts + 255) / 256);
+    hipLaunchKernelGGL(bad_material, dim3(nb), dim3(256), 0, h->stream, (const double *)ieps, (const double *)imu,
+                       npts, h->red);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(h->stream) != hipSuccess)
+        return give_all_back(fail(NKC_ERR_HIP, "material check"));
+    const unsigned long long bad = *std::min_element(h->red, h->red + nb);
+    if (bad != ~0ull) return give_all_back(bad_node((int64_t)bad));
+    free_adjoint(h, true);                 // the stored trajectory has the old materials
+    const int64_t nface = m.nelt * 6 * m.n1 * m.n1;
+    hipLaunchKernelGGL(face_coefs, item_grid(nface), dim3(256), 0, h->stream, (const double *)ieps,
+                       (const double *)imu, (const int32_t *)m.nbr, m.n1, m.nelt, (int)HOST_FACE_PEC, h->C0, fco);
+    hipLaunchKernelGGL(invert_pair, item_grid(npts), dim3(256), 0, h->stream, ieps, imu, npts);
+    HIPCHK(hipGetLastError());
+    if (m.mat != MAT_NODE) {
+        (void)hipFree(h->yz);              // one pair per element
+        h->yz = nullptr;
+        (void)hipFree(m.fco);
+        m.fco = fco;
+    }
+    h->yz_ok = false;
+    (void)hipFree(m.ieps); (void)hipFree(m.imu);
+    m.ieps = ieps;
+    m.imu = imu;
+    m.mat = MAT_NODE;
+    h->hm.mat = 1;
+    h->hm_stale = true;
     if (h->ngraph) {
         // the sheet's Yfac and yconduc follow the materials
-        const size_t n2 = (size_t)h->m.n1 * h->m.n1;
+        const size_t n2 = (size_t)m.n1 * m.n1;
         std::vector<double> par(h->gr_face.size() * 14 * n2);
+        if ((rc = host_materials(h))) return rc;
         HIPCHK(hipMemcpy(par.data(), h->gpar, sizeof(double) * par.size(), hipMemcpyDeviceToHost));
         sheet_coefs(h, par);
         HIPCHK(hipMemcpy(h->gpar, par.data(), sizeof(double) * par.size(), hipMemcpyHostToDevice));
@@ -2513,13 +2635,13 @@ int32_t nkc_adjoint_forward(nkc_handle *h, double *time, double dt, int64_t nste
     return NKC_OK;
 }
 
-int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *lamE, int64_t ld,
-                             double *geps, double *gmu) {
-    if (!h || !lamH || !lamE) return fail(NKC_ERR_ARG, "null handle or adjoint seed");
+namespace {
+
+// The backward sweep; seed() adds the adjoint of the final state to the
+// zeroed A.lam[0], complete when it returns or queued on the handle's stream.
+int32_t backward_sweep(nkc_handle *h, const std::function<int32_t()> &seed, double *geps, double *gmu) {
     auto &A = h->adj;
-    if (A.nseg == 0) return fail(NKC_ERR_ARG, "no nkc_adjoint_forward run to differentiate");
     DevMesh &m = h->m;
-    if (ld < m.npts) return fail(NKC_ERR_ARG, "ld < npts");
     const size_t blk = 6 * (size_t)m.fs, jsz = drude_size(h);
     const double t_end = h->t_host;
     int32_t rc;
@@ -2535,7 +2657,8 @@ int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *la
         HIPCHK(hipMemset(A.gA, 0, sizeof(double) * jsz / 3));
         HIPCHK(hipMemset(A.gB, 0, sizeof(double) * jsz / 3));
     }
-    if ((rc = copy_fields_h2d(A.lam[0], m.fs, 0, lamH, lamE, m.npts, ld))) return rc;
+    HIPCHK(hipStreamSynchronize(nullptr));   // the fills, which the handle's stream does not wait for
+    if ((rc = seed())) return rc;
     // the RK registers restart from zero at a segment or window start (the
     // first stage multiplies them by a_1 = 0)
     auto start_from = [&](const double *J, int64_t step) -> int32_t {
@@ -2585,6 +2708,38 @@ int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *la
     if (gmu) HIPCHK(hipMemcpy(gmu, A.gmu, sizeof(double) * m.npts, hipMemcpyDefault));
     HIPCHK(hipStreamSynchronize(nullptr));
     return NKC_OK;
+}
+
+}  // namespace
+
+int32_t nkc_adjoint_backward(nkc_handle *h, const double *lamH, const double *lamE, int64_t ld,
+                             double *geps, double *gmu) {
+    if (!h || !lamH || !lamE) return fail(NKC_ERR_ARG, "null handle or adjoint seed");
+    if (h->adj.nseg == 0) return fail(NKC_ERR_ARG, "no nkc_adjoint_forward run to differentiate");
+    if (ld < h->m.npts) return fail(NKC_ERR_ARG, "ld < npts");
+    return backward_sweep(
+        h, [&] { return copy_fields_h2d(h->adj.lam[0], h->m.fs, 0, lamH, lamE, h->m.npts, ld); }, geps, gmu);
+}
+
+int32_t nkc_adjoint_backward_at(nkc_handle *h, int64_t n, const int64_t *nodes, const double *seeds,
+                                double *geps, double *gmu) {
+    if (!h || n < 0 || (n && (!nodes || !seeds))) return fail(NKC_ERR_ARG, "null handle or adjoint seed");
+    if (h->adj.nseg == 0) return fail(NKC_ERR_ARG, "no nkc_adjoint_forward run to differentiate");
+    int64_t *dn = nullptr;
+    double *dv = nullptr;
+    int32_t rc;
+    if (n && (rc = node_list(h, n, nodes, &dn, &dv))) return rc;
+    if (n) HIPCHK(hipMemcpy(dv, seeds, sizeof(double) * 6 * n, hipMemcpyDefault));
+    return backward_sweep(
+        h,
+        [&]() -> int32_t {
+            if (n)
+                hipLaunchKernelGGL(scatter_nodes, item_grid(n, 6), dim3(256), 0, h->stream, h->adj.lam[0], h->m.fs,
+                                   (const int64_t *)dn, n, (const double *)dv);
+            HIPCHK(hipGetLastError());
+            return NKC_OK;
+        },
+        geps, gmu);
 }
 
 int32_t nkc_adjoint_get_drude(nkc_handle *h, double *ga, double *gb) {
