@@ -15,32 +15,31 @@
 // forward recompute.  Each face node gathers both halves of the transposed
 // flux of its face: its own flux and the neighbour's flux on the shared face,
 // so every output has a single owner (no atomics).
+//
+// The workgroup's shape and phases are the forward stage's (BoxShape):
+//   0  lambda, kappa, the stage residual, the gradient and the inverse
+//      material in the order of memory, 64-node chunks that start on
+//      128-byte lines; v = P kt into LDS, kappa out at once from the same
+//      lanes, lambda kept in registers;
+//   1  each wave takes whole faces: the transposed flux (four tangential
+//      components) and the face's part of the material gradient into LDS;
+//   2  per lane a column's run of levels: the transposed curl and the faces;
+//   3  the sums through the element's place in LDS back to the lanes that
+//      hold lambda and the gradient, and out in whole lines.
+//
+// What bounds it: with the gradients, at N = 7, 600 MB of HBM traffic per
+// stage at 16^3 (101 us at the card's four-stream rate) and the latency of
+// three dependent rounds of loads with three workgroups on a CU; without
+// them, the bytes.  Whole-line stores from the lanes that loaded, tangential
+// traces, a split of the levels as the stage's and equal-work ranges under a
+// Drude region took, per stage with the gradients, N = 4 (28^3) 469 -> 350
+// us, N = 5 (24^3) 364 -> 285, N = 6 (20^3) 304 -> 260, N = 7 (16^3) 190 ->
+// 165, N = 8 (16^3) 380 -> 280, N = 9 (12^3) 213 -> 155; without them, with a
+// Drude region, N = 7 (16^3) 173 -> 118, N = 9 (12^3) 216 -> 110.
 #pragma once
-#include "stage_args.hpp"
+#include "box_kernel.hpp"
 
 namespace nkc {
-
-// Whether the reversed stage's outputs and residual stream past L2: at N = 7 a
-// role's level is 64 doubles, whole cache lines from one wave; at the other
-// orders a level straddles lines and the plain forms are faster.
-template <int N1>
-constexpr bool nt_streams() { return N1 == 8; }
-
-// Four roles of (N+1)^2 lanes padded to whole waves: role & 1 selects the
-// update group (0: H, 1: E), role >> 1 the half of the levels; LDS as
-// u(i,j,k) of field f at f*N3 + idx, XOR-swizzled for power-of-two N1.
-template <int N1>
-struct Shape {
-    static constexpr int N2 = N1 * N1, N3 = N2 * N1;
-    static constexpr int ROLES = 4;
-    static constexpr int LANES = ((N2 + 63) / 64) * 64;
-    static constexpr int BS = LANES * ROLES;
-    static constexpr int KH = (N1 + 1) / 2;           // levels in the lower half
-    static constexpr bool SWZ = (N1 & (N1 - 1)) == 0;
-    __device__ static __forceinline__ int idx(int i, int j, int k) {
-        return (SWZ ? (i ^ j) : i) + N1 * j + N2 * k;
-    }
-};
 
 struct AdjArgs {
     const double *__restrict__ lam_in;  // 6 fields, stride fs
@@ -72,20 +71,9 @@ struct AdjArgs {
     const double *__restrict__ stJ;
     double *__restrict__ gA;
     double *__restrict__ gB;
+    int32_t xcd_bal;                    // equal-work element ranges, as in StageArgs
+    int32_t xcd_lo[9];
 };
-
-// Material data at one node: inverse permittivity and permeability and the
-// admittance/impedance pair, from the per-element or per-node tables.
-struct NodeMat {
-    double ie, im, Y, Z;
-};
-
-template <int N1, int MAT>
-__device__ __forceinline__ NodeMat node_mat(const AdjArgs &a, int e, int64_t node) {
-    const int64_t x = (MAT == MAT_ELEM) ? (int64_t)e : node;
-    const double2 yz = *reinterpret_cast<const double2 *>(a.yz + 2 * x);
-    return NodeMat{a.ieps[x], a.imu[x], yz.x, yz.y};
-}
 
 // Flux coefficients of one side of a face, (Y02, C02Y, Z02, C02Z) =
 // (-Y1/(2Y0), C0/(2Y0), Z1/(2Z0), C0/(2Z0)), from hy = 1/(2Y0) and
@@ -108,388 +96,476 @@ __device__ __forceinline__ void coef_bar(double gY02, double gC02Y, double gZ02,
     Zb1 = gZ02 * hz;
 }
 
-// Transposed flux at one face node of this element (normal sg e_AX), both
-// halves of the shared face, plus the eps/mu gradient at the own node.
-//   vo, uo: own v = P kt and own stage state (H then E)
-//   vn, un: the neighbour's at the paired node (interior faces)
+// Transposed flux at one face node of this element (normal sg along the
+// face's axis), both halves of the shared face, plus the material gradient's
+// factor at the own node.  Every vector is (H t1, H t2, E t1, E t2): a face's
+// flux and its transpose have no component along the normal, and n x (v1, v2)
+// = sg (-v2, v1).
+//   vo: own v = P kt; vn: the neighbour's at the paired node (interior faces)
+//   d: the jumps the stage's flux saw (PEC: E doubled, H zero; no partner:
+//      minus the own traces)
 //   L, Ln: own / neighbour lift factors
-//   mo: own material; Yn, Zn: the neighbour's admittance and impedance
+//   Yo, Zo, Yn, Zn: own and neighbour admittance and impedance
 // The flux coefficients are formed here from the admittances/impedances as
 // cem_maxwell_materials averages them (src/cem_maxwell.F:262-325): interior
 // Y0 = (Y- + Y+)/2, Y1 = Y+; PEC Y0 = Y1 = Y-; no partner Y0 = Y-/2, Y1 = 0.
-// Out: adj (H then E) added to B^T v at the own node; ge, gm gradients.
-template <int AX>
-__device__ __forceinline__ void adj_face(double sg, int type, const double vo[6], const double uo[6],
-                                         const double vn[6], const double un[6],
-                                         double L, double Ln, double C0,
-                                         const NodeMat &mo, double Yn, double Zn,
-                                         double adj[6], double &ge, double &gm) {
-    const double Yo = mo.Y, Zo = mo.Z;
+// Out: adj added to B^T v at the own node; dq with g_eps = dq/eps, g_mu =
+// -dq/mu (Y = sqrt(eps/mu), Z = sqrt(mu/eps): dY/deps = Y/(2 eps), dZ/deps =
+// -Z/(2 eps)).
+template <bool GM>
+__device__ __forceinline__ void adj_face(double sg, int type, const double vo[4], const double vn[4],
+                                         const double d[4], double L, double Ln, double C0,
+                                         double Yo, double Zo, double Yn, double Zn, double adj[4], double &dq) {
     double Ys, Zs;                       // twice the averages
     if (type >= 0) { Ys = Yo + Yn; Zs = Zo + Zn; }
     else if (type == FACE_PEC) { Ys = 2.0 * Yo; Zs = 2.0 * Zo; }
     else { Ys = Yo; Zs = Zo; }
     const double hy = 0.5 / (0.5 * Ys), hz = 0.5 / (0.5 * Zs);
-    double cf[4];
+    double cf[4], cfn[4];
     side_coef(hy, hz, Ys - Yo, Zs - Zo, C0, cf);
-    double aH[3], aE[3];
+    double av[4], bv[4];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) { aH[c] = L * vo[c]; aE[c] = L * vo[3 + c]; }
-    double sE[3], sH[3];
-    if (type >= 0) {
-        double dE[3] = {un[3] - uo[3], un[4] - uo[4], un[5] - uo[5]};
-        double dH[3] = {un[0] - uo[0], un[1] - uo[1], un[2] - uo[2]};
-        ncross<AX>(sg, dE, sE);
-        ncross<AX>(sg, dH, sH);
-    } else {
-        double Em[3] = {-uo[3], -uo[4], -uo[5]};
-        double Hm[3] = {-uo[0], -uo[1], -uo[2]};
-        ncross<AX>(sg, Em, sE);
-        if (type == FACE_PEC) {
-            sE[0] *= 2.0; sE[1] *= 2.0; sE[2] *= 2.0;
-            sH[0] = sH[1] = sH[2] = 0.0;
-        } else {
-            ncross<AX>(sg, Hm, sH);
-        }
-    }
-    // own half: F_H = Y02 sE - C02Y n x sH, F_E = Z02 sH - C02Z n x sE
-    double NaH[3], NaE[3], NNaH[3], NNaE[3];
-    ncross<AX>(sg, aH, NaH);
-    ncross<AX>(sg, aE, NaE);
-    ncross<AX>(sg, NaH, NNaH);
-    ncross<AX>(sg, NaE, NNaE);
+    for (int c = 0; c < 4; ++c) { av[c] = L * vo[c]; bv[c] = Ln * vn[c]; }
+    // own half: F_H = Y02 sE - C02Y n x sH, F_E = Z02 sH - C02Z n x sE, sE = n x d_E, sH = n x d_H
     if (type == FACE_PEC) {
-        // sE = -2 n x E-, sH = 0
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            adj[c] = 0.0;
-            adj[3 + c] = 2.0 * cf[0] * NaH[c] + 2.0 * cf[3] * NNaE[c];
-        }
+        adj[0] = 0.0;
+        adj[1] = 0.0;
+        adj[2] = -2.0 * cf[0] * (sg * av[1]) - 2.0 * cf[3] * av[2];
+        adj[3] = 2.0 * cf[0] * (sg * av[0]) - 2.0 * cf[3] * av[3];
     } else {
-        // d/d(jump): gE = -Y02 N aH - C02Z N^2 aE ; gH = -C02Y N^2 aH - Z02 N aE;
         // the own traces enter the jumps with a minus sign
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            adj[3 + c] = cf[0] * NaH[c] + cf[3] * NNaE[c];
-            adj[c] = cf[1] * NNaH[c] + cf[2] * NaE[c];
-        }
+        adj[0] = -cf[1] * av[0] - cf[2] * (sg * av[3]);
+        adj[1] = -cf[1] * av[1] + cf[2] * (sg * av[2]);
+        adj[2] = -cf[0] * (sg * av[1]) - cf[3] * av[2];
+        adj[3] = cf[0] * (sg * av[0]) - cf[3] * av[3];
     }
-    double NsH[3], NsE[3];
-    ncross<AX>(sg, sH, NsH);
-    ncross<AX>(sg, sE, NsE);
-    double gY02 = 0, gC02Y = 0, gZ02 = 0, gC02Z = 0;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        gY02 += aH[c] * sE[c];
-        gC02Y -= aH[c] * NsH[c];
-        gZ02 += aE[c] * sH[c];
-        gC02Z -= aE[c] * NsE[c];
-    }
-    double dY, dZ;
     if (type >= 0) {
-        double Yb0, Yb1, Zb0, Zb1;
-        coef_bar(gY02, gC02Y, gZ02, gC02Z, hy, hz, Ys - Yo, Zs - Zo, C0, Yb0, Yb1, Zb0, Zb1);
-        dY = 0.5 * Yb0;
-        dZ = 0.5 * Zb0;
         // neighbour half: its normal is -n, its jump vectors equal ours
-        double cfn[4];
         side_coef(hy, hz, Ys - Yn, Zs - Zn, C0, cfn);
-        double bH[3], bE[3], NbH[3], NbE[3], NNbH[3], NNbE[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) { bH[c] = Ln * vn[c]; bE[c] = Ln * vn[3 + c]; }
-        ncross<AX>(sg, bH, NbH);
-        ncross<AX>(sg, bE, NbE);
-        ncross<AX>(sg, NbH, NNbH);
-        ncross<AX>(sg, NbE, NNbE);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            adj[3 + c] += cfn[0] * NbH[c] - cfn[3] * NNbE[c];
-            adj[c] += -cfn[1] * NNbH[c] + cfn[2] * NbE[c];
-        }
-        double hY02 = 0, hC02Y = 0, hZ02 = 0, hC02Z = 0;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            hY02 += bH[c] * sE[c];
-            hC02Y += bH[c] * NsH[c];
-            hZ02 += bE[c] * sH[c];
-            hC02Z += bE[c] * NsE[c];
-        }
-        coef_bar(hY02, hC02Y, hZ02, hC02Z, hy, hz, Ys - Yn, Zs - Zn, C0, Yb0, Yb1, Zb0, Zb1);
-        dY += 0.5 * Yb0 + Yb1;
-        dZ += 0.5 * Zb0 + Zb1;
-    } else if (type == FACE_PEC) {
-        double Yb0, Yb1, Zb0, Zb1;
-        coef_bar(gY02, gC02Y, gZ02, gC02Z, hy, hz, Yo, Zo, C0, Yb0, Yb1, Zb0, Zb1);
-        dY = Yb0 + Yb1;
-        dZ = Zb0 + Zb1;
-    } else {
-        double Yb0, Yb1, Zb0, Zb1;
-        coef_bar(gY02, gC02Y, gZ02, gC02Z, hy, hz, 0.0, 0.0, C0, Yb0, Yb1, Zb0, Zb1);
-        dY = 0.5 * Yb0;
-        dZ = 0.5 * Zb0;
+        adj[0] += cfn[1] * bv[0] - cfn[2] * (sg * bv[3]);
+        adj[1] += cfn[1] * bv[1] + cfn[2] * (sg * bv[2]);
+        adj[2] += cfn[3] * bv[2] - cfn[0] * (sg * bv[1]);
+        adj[3] += cfn[3] * bv[3] + cfn[0] * (sg * bv[0]);
     }
-    // Y = sqrt(eps/mu), Z = sqrt(mu/eps): dY/deps = Y/(2 eps), dZ/deps = -Z/(2 eps)
-    const double dq = 0.5 * (dY * Yo - dZ * Zo);
-    ge = dq * mo.ie;
-    gm = -dq * mo.im;
+    if constexpr (GM) {
+        const double sE[2] = {-sg * d[3], sg * d[2]}, sH[2] = {-sg * d[1], sg * d[0]};
+        double Yb0, Yb1, Zb0, Zb1, dY, dZ;
+        const double Y1 = type >= 0 ? Ys - Yo : type == FACE_PEC ? Yo : 0.0;
+        const double Z1 = type >= 0 ? Zs - Zo : type == FACE_PEC ? Zo : 0.0;
+        coef_bar(av[0] * sE[0] + av[1] * sE[1], av[0] * d[0] + av[1] * d[1], av[2] * sH[0] + av[3] * sH[1],
+                 av[2] * d[2] + av[3] * d[3], hy, hz, Y1, Z1, C0, Yb0, Yb1, Zb0, Zb1);
+        if (type == FACE_PEC) {
+            dY = Yb0 + Yb1;
+            dZ = Zb0 + Zb1;
+        } else {
+            dY = 0.5 * Yb0;
+            dZ = 0.5 * Zb0;
+        }
+        if (type >= 0) {
+            coef_bar(bv[0] * sE[0] + bv[1] * sE[1], -(bv[0] * d[0] + bv[1] * d[1]), bv[2] * sH[0] + bv[3] * sH[1],
+                     -(bv[2] * d[2] + bv[3] * d[3]), hy, hz, Ys - Yn, Zs - Zn, C0, Yb0, Yb1, Zb0, Zb1);
+            dY += 0.5 * Yb0 + Yb1;
+            dZ += 0.5 * Zb0 + Zb1;
+        }
+        dq = 0.5 * (dY * Yo - dZ * Zo);
+    }
 }
 
-// GM = 1: also the eps/mu gradients (needs the stage residual); GM = 0: the
+// Waves per SIMD the register allocator keeps to (0: free), as box_waves.
+// At N = 7 with the gradients 128 VGPRs would spill 50 bytes a lane, which
+// costs more than the fourth workgroup on a CU gives (16^3: 180 us a stage
+// against 162); at N = 8 and 9 168 VGPRs would leave one 8-wave workgroup.
+constexpr int adjoint_waves(int n1, bool gm) { return n1 < 7 ? 0 : (n1 == 8 && gm) ? 3 : 4; }
+
+// GM: also the eps/mu gradients (needs the stage residual); otherwise the
 // adjoint state and the Drude gradients only (no residual store is read).
-// A 4-wave workgroup is held to 3 waves per SIMD (168 VGPRs, a few spills:
-// three elements per CU, as its LDS allows), so that lambda can stay in
-// registers from its load to the update instead of being read twice.
-template <int N1, int MAT, int GM>
-__global__ void __launch_bounds__(Shape<N1>::BS) __attribute__((amdgpu_waves_per_eu(Shape<N1>::BS <= 256 ? 3 : 1)))
+// NT: non-temporal residual loads and output stores.
+template <int N1, int MAT, bool GM, bool NT>
+__global__ void __launch_bounds__(BoxShape<N1>::BS)
+    __attribute__((amdgpu_waves_per_eu(adjoint_waves(N1, GM) ? adjoint_waves(N1, GM) : 1)))
 adjoint_kernel(AdjArgs a) {
-    using S = Shape<N1>;
-    constexpr int N2 = S::N2, N3 = S::N3, KH = S::KH, LANES = S::LANES;
-    // level loop unrolled except at N1 = 10, where unrolling costs
-    // a wave per SIMD (240 VGPRs against 179)
-    constexpr int LVL_UNROLL = (N1 >= 10) ? 1 : KH;
-    __shared__ double s_v[6 * N3];      // v = P kt, swizzled like s_u
-    __shared__ double s_f[32 * N2];     // [face 0..3][adjH 3, adjE 3, geps, gmu][q]
-    __shared__ double s_D[N2];
-    __shared__ double s_g[GM ? 2 * N3 : 1];   // [grp][k N2 + q]: gradient without the face terms
+    using S = BoxShape<N1>;
+    constexpr int N2 = S::N2, N3 = S::N3, KL = S::KL, WG = S::WG;
+    constexpr int FS = GM ? 5 : 4;          // per face: H t1, H t2, E t1, E t2 (, dq)
+    __shared__ double s_v[6 * N3];          // v = P kt, then the sums of phase 2
+    __shared__ double s_f[6 * FS * N2];     // [face][component][a + n1 b]
+    __shared__ double s_D[N2];              // D(l,i) at [i + n1 l]
 
-    const int e = remap_element(blockIdx.x, a.nelt, a.per_xcd);
+    const int e = stage_element<true>(a, blockIdx.x, a.nelt);
     if (e >= a.nelt) return;
-    const int t = threadIdx.x;
-    const int role = t / LANES, q = t % LANES;
-    const bool act = q < N2;
-    const int i = q % N1, j = q / N1;
-    const int grp = role & 1;            // 0: H fields, 1: E fields
-    const int half = role >> 1;
-    const int k0 = half ? KH : 0;
-    const int64_t eo = (int64_t)e * N3;
-    const int64_t fs = a.fs;
-    const int fo = 3 * grp;              // this role's field offset
-
-    // ---- phase 0: this role's fields and levels.  v = P kt goes to LDS;
-    // the kappa output and the inverse-mass part of the material gradient
-    // (d r/d m = -r/m, so -kt.r/m) need no other lane and are finished
-    // here, so that the role's lambda, kappa, r and g streams are all
-    // loaded up front ----
-    if (t < N2) s_D[t] = a.D[t];
-    double lm[3][KH];                    // lambda of the role's levels, kept for the update
-    if (act) {
-        double kp[3][KH], rr[3][KH], gg[KH], pm[KH];
-        double *g = grp ? a.geps : a.gmu;
-#pragma unroll
-        for (int kk = 0; kk < KH; ++kk) {
-            const int k = k0 + kk;
-            const bool ok = k < N1;
-            const int64_t node = eo + k * N2 + q;
-            if (MAT == MAT_ELEM) pm[kk] = grp ? a.ieps[e] : a.imu[e];
-            else pm[kk] = ok ? (grp ? a.ieps[node] : a.imu[node]) : 0.0;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const int64_t p = (fo + c) * fs + node;
-                lm[c][kk] = ok ? a.lam_in[p] : 0.0;
-                kp[c][kk] = ok ? a.kap_in[p] : 0.0;
-                rr[c][kk] = (GM && ok) ? ld_stream<nt_streams<N1>()>(a.rs + p) : 0.0;
-            }
-            gg[kk] = (GM && ok) ? g[node] : 0.0;
-        }
-#pragma unroll
-        for (int kk = 0; kk < KH; ++kk) {
-            const int k = k0 + kk;
-            if (k >= N1) break;
-            const int64_t node = eo + k * N2 + q;
-            double kr = 0.0;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const double kt = kp[c][kk] + a.rkb * lm[c][kk];
-                s_v[(fo + c) * N3 + S::idx(i, j, k)] = pm[kk] * kt;
-                kr += kt * rr[c][kk];
-                st_stream<nt_streams<N1>()>(a.kap_out + (fo + c) * fs + node, a.rka * kt);
-            }
-            if (GM) s_g[grp * N3 + k * N2 + q] = gg[kk] - a.dt * kr * pm[kk];
-        }
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int grp = w >= WG ? 1 : 0;        // 0: H fields, 1: E fields
+    const int wg = w - grp * WG;
+    const int rl = t - grp * S::GL;
+    // lanes past the last node repeat it, in the same wave (see box_kernel)
+    int part, q;
+    if (S::PAD) {
+        part = __builtin_amdgcn_readfirstlane(rl / S::PL);
+        q = min(rl - part * S::PL, N2 - 1);
+    } else {
+        const int r2 = min(rl, S::KS * N2 - 1);
+        part = r2 / N2;
+        q = r2 - part * N2;
     }
-    const double *geo = a.geo + (int64_t)e * 9;
-    __syncthreads();
+    const int j = q / N1, i = q - j * N1;
+    constexpr int BASE = N1 / S::KS, REM = N1 % S::KS;
+    const int k0 = part * BASE + (part < REM ? part : REM);
+    const int kn = BASE + (part < REM ? 1 : 0);
+    auto run_has = [&](int kk) { return REM == 0 || kk < kn; };
+    const int64_t eo = (int64_t)e * N3, fs = a.fs;
+    if (t < N2) s_D[t % N1 * N1 + t / N1] = a.D[t];
 
-    // ---- phase 1: role r takes x/y face r at face node (i,j) ----
-    if (act) {
-        const int r = role;
-        const int nb = a.nbr[e * 6 + r];
-        int vi, vj, vk;
-        int64_t nbn;
-        if (r == 0) { vi = 0;      vj = i;      vk = j; nbn = (N1 - 1) + N1 * i + N2 * j; }
-        if (r == 1) { vi = N1 - 1; vj = i;      vk = j; nbn = 0 + N1 * i + N2 * j; }
-        if (r == 2) { vi = i;      vj = 0;      vk = j; nbn = i + N1 * (N1 - 1) + N2 * j; }
-        if (r == 3) { vi = i;      vj = N1 - 1; vk = j; nbn = i + N2 * j; }
-        const int64_t own = eo + vi + N1 * vj + N2 * vk;
-        double vo[6], uo[6], vn[6], un[6];
+    // ---- phase 0: this wave's chunks of its group's fields ----
+    const int m = S::G == 16 ? 0 : (int)(eo & 15);
+    unsigned sto[S::NST];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            vo[c] = s_v[c * N3 + S::idx(vi, vj, vk)];
-            uo[c] = GM ? a.us[c * fs + own] : 0.0;    // the jumps feed the eps/mu gradient only
-        }
-        double Yn = 1.0, Zn = 1.0, Ln = 0.0;
-        const NodeMat mo = node_mat<N1, MAT>(a, e, own);
-        if (nb >= 0) {
-            const int64_t pn = (int64_t)nb * N3 + nbn;
-            const NodeMat mn = node_mat<N1, MAT>(a, nb, pn);
-            Yn = mn.Y;
-            Zn = mn.Z;
+    for (int n = 0; n < S::NST; ++n) {
+        int x = (wg + WG * n) * 64 + lane - m;
+        if (S::G != 16 && n == 0) x = max(x, 0);
+        if ((n + 1) * WG * 64 > N3) x = min(x, N3 - 1);
+        sto[n] = 8u * (unsigned)x;
+    }
+    // offsets zero-extended where they are used, so that the addresses stay
+    // a scalar base and 32 bits
+    auto here = [&] {
 #pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const double pm = (c < 3) ? mn.im : mn.ie;
-                vn[c] = pm * (a.kap_in[c * fs + pn] + a.rkb * a.lam_in[c * fs + pn]);
-                un[c] = GM ? a.us[c * fs + pn] : 0.0;
+        for (int n = 0; n < S::NST; ++n) asm volatile("" : "+v"(sto[n]));
+    };
+    here();
+    // a chunk past the element's end (N = 4 only)
+    auto past = [&](int n) { return S::WG * S::NST * 64 - N3 >= 64 && (wg + WG * n) * 64 - m >= N3; };
+    // chunk n's place in an LDS field
+    auto place = [&](double *f, int n) -> double * {
+        return S::SWZ ? f + (wg + WG * n) * 64 + S::idx(lane % N1, (lane / N1) % N1, lane / N2) : at(f, sto[n]);
+    };
+    double *const own = s_v + 3 * grp * N3;
+    const int64_t go = 3 * grp * fs + eo;
+    // neighbour traces of this wave's faces (a wall reads the element
+    // itself, unused): v = P kt, the stage's jumps, the materials
+    double vn[S::NF][4], fd[S::NF][4], fy[S::NF][4], fL[S::NF][2], fk[S::NF][4], fl[S::NF][4], fi[S::NF][2];
+    [[maybe_unused]] double fo[S::NF][4], fn[S::NF][4];
+    int fown[S::NF], ftype[S::NF];
+    auto load_face = [&](int n) {
+        const int id = min(w + 2 * WG * n, 6 * S::FC - 1), f = id / S::FC;
+        const int ax = f >> 1, side = f & 1;
+        int fq = (id - f * S::FC) * 64 + lane;
+        if (N2 % 64 != 0) fq = min(fq, N2 - 1);
+        const int fb = fq / N1, fa = fq - fb * N1;
+        ftype[n] = a.nbr[e * 6 + f];
+        const int M = side ? N1 - 1 : 0;
+        const int on = pick3(ax, N1 * fa + N2 * fb, fa + N2 * fb, fa + N1 * fb);
+        const int st = pick3(ax, 1, N1, N2);
+        const unsigned opp = 8u * (unsigned)(on + (N1 - 1 - M) * st), mine = 8u * (unsigned)(on + M * st);
+        if (S::SWZ) fown[n] = ax == 0 ? S::idx(M, fa, fb) : ax == 1 ? S::idx(fa, M, fb) : S::idx(fa, fb, M);
+        else fown[n] = on + M * st;
+        const int ne = ftype[n] >= 0 ? ftype[n] : e;
+        const int64_t po = (int64_t)ne * N3;
+        const int64_t c1 = pick3(ax, fs, 2 * fs, (int64_t)0), c2 = pick3(ax, 2 * fs, (int64_t)0, fs);
+        const int64_t off[4] = {c1, c2, c1 + 3 * fs, c2 + 3 * fs};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            fk[n][c] = *at(a.kap_in + po + off[c], opp);
+            fl[n][c] = *at(a.lam_in + po + off[c], opp);
+            if constexpr (GM) {
+                fo[n][c] = *at(a.us + eo + off[c], mine);
+                fn[n][c] = *at(a.us + po + off[c], opp);
             }
-            Ln = a.geo[(int64_t)nb * 9 + 3 + (r ^ 1)];
+        }
+        if (MAT == MAT_ELEM) {
+            fi[n][0] = a.imu[ne];
+            fi[n][1] = a.ieps[ne];
+            fy[n][0] = a.yz[2 * e];
+            fy[n][1] = a.yz[2 * e + 1];
+            fy[n][2] = a.yz[2 * ne];
+            fy[n][3] = a.yz[2 * ne + 1];
         } else {
-#pragma unroll
-            for (int c = 0; c < 6; ++c) { vn[c] = 0.0; un[c] = 0.0; }
+            fi[n][0] = *at(a.imu + po, opp);
+            fi[n][1] = *at(a.ieps + po, opp);
+            const double2 yo = *reinterpret_cast<const double2 *>(at(a.yz + 2 * eo, 2 * mine));
+            const double2 yn = *reinterpret_cast<const double2 *>(at(a.yz + 2 * po, 2 * opp));
+            fy[n][0] = yo.x;
+            fy[n][1] = yo.y;
+            fy[n][2] = yn.x;
+            fy[n][3] = yn.y;
         }
-        double adj[6], ge, gm;
-        const double sg = (r & 1) ? 1.0 : -1.0;
-        if (r < 2) adj_face<0>(sg, nb, vo, uo, vn, un, geo[3 + r], Ln, a.C0, mo, Yn, Zn, adj, ge, gm);
-        else       adj_face<1>(sg, nb, vo, uo, vn, un, geo[3 + r], Ln, a.C0, mo, Yn, Zn, adj, ge, gm);
+        fL[n][0] = a.geo[(int64_t)e * 9 + 3 + f];
+        fL[n][1] = a.geo[(int64_t)ne * 9 + 3 + (f ^ 1)];
+    };
+    // a face's loads reduced to what its flux needs
+    auto settle = [&](int n) {
 #pragma unroll
-        for (int c = 0; c < 6; ++c) s_f[(r * 8 + c) * N2 + q] = adj[c];
-        if (GM) {
-            s_f[(r * 8 + 6) * N2 + q] = ge;
-            s_f[(r * 8 + 7) * N2 + q] = gm;
+        for (int c = 0; c < 4; ++c) {
+            vn[n][c] = fi[n][c < 2 ? 0 : 1] * (fk[n][c] + a.rkb * fl[n][c]);
+            fd[n][c] = 0.0;
+            if constexpr (GM) {
+                const double wall = ftype[n] == FACE_PEC ? (c < 2 ? 0.0 : -2.0) : -1.0;
+                fd[n][c] = ftype[n] >= 0 ? fn[n][c] - fo[n][c] : wall * fo[n][c];
+                asm volatile("" : "+v"(vn[n][c]), "+v"(fd[n][c]));
+            }
         }
-    }
-    __syncthreads();
-    if (!act) return;
+    };
+    // what the registers hold: the first face's loads in flight with the
+    // chunks' (N = 7 with the gradients: 180 -> 162 us), one face's loads at a
+    // time, lambda from its load to the update (read again at N = 9 with the
+    // gradients, 12^3: 165 -> 150 us)
+    constexpr bool EARLY = GM == (N1 == 8), ONE = GM && N1 != 8, HOLD = !(GM && N1 == 10);
 
-    // ---- phase 2: this role's levels ----
-    const double gx = geo[0], gy = geo[1], gz = geo[2];
-    const int src = grp ? 0 : 3;          // v of the other group
-    const double sgn = grp ? 1.0 : -1.0;
-    const double *S0 = s_v + (src + 0) * N3;
-    const double *S1 = s_v + (src + 1) * N3;
-    const double *S2 = s_v + (src + 2) * N3;
-    const int zface = half ? 5 : 4;
-    const int nbz = a.nbr[e * 6 + zface];
-    // z face of this half (level kz), for this role's fields, ahead of the
-    // level loop so that its temporaries are dead before the curl sums
-    const int kz = half ? N1 - 1 : 0;
-    double zadj[3], zg;
+    // kept to the end: lambda and, with GM, kt.r
+    double lm[3][S::NST];
+    [[maybe_unused]] double kr[GM ? S::NST : 1];
+    const double *const mp = (grp ? a.ieps : a.imu);
+    double *const g = (grp ? a.geps : a.gmu) + eo;
     {
-        const int k = kz;
-        const int64_t node = eo + k * N2 + q;
-        const int64_t nbn = half ? (int64_t)q : (int64_t)(N1 - 1) * N2 + q;
-        double vo[6], uo[6], vn[6], un[6];
+        double kt[3][S::NST], pm[S::NST];
+        [[maybe_unused]] double rr[3][GM ? S::NST : 1];
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            vo[c] = s_v[c * N3 + S::idx(i, j, k)];
-            uo[c] = GM ? a.us[c * fs + node] : 0.0;
-        }
-        double Yn = 1.0, Zn = 1.0, Ln = 0.0;
-        const NodeMat mo = node_mat<N1, MAT>(a, e, node);
-        if (nbz >= 0) {
-            const int64_t pn = (int64_t)nbz * N3 + nbn;
-            const NodeMat mn = node_mat<N1, MAT>(a, nbz, pn);
-            Yn = mn.Y;
-            Zn = mn.Z;
+        for (int n = 0; n < S::NST; ++n) pm[n] = MAT == MAT_ELEM ? mp[e] : *at(mp + eo, sto[n]);
 #pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const double pm = (c < 3) ? mn.im : mn.ie;
-                vn[c] = pm * (a.kap_in[c * fs + pn] + a.rkb * a.lam_in[c * fs + pn]);
-                un[c] = GM ? a.us[c * fs + pn] : 0.0;
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int n = 0; n < S::NST; ++n) {
+                lm[c][n] = *at(a.lam_in + go + c * fs, sto[n]);
+                kt[c][n] = *at(a.kap_in + go + c * fs, sto[n]);
+                if constexpr (GM) rr[c][n] = ld_stream<NT>(at(a.rs + go + c * fs, sto[n]));
             }
-            Ln = a.geo[(int64_t)nbz * 9 + 3 + (zface ^ 1)];
-        } else {
+        if (EARLY) load_face(0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < 6; ++c) { vn[c] = 0.0; un[c] = 0.0; }
+        for (int n = 0; n < S::NST; ++n) {
+            if constexpr (GM) kr[n] = 0.0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                kt[c][n] = kt[c][n] + a.rkb * lm[c][n];
+                if constexpr (GM) kr[n] += kt[c][n] * rr[c][n];
+                *place(own + c * N3, n) = pm[n] * kt[c][n];
+            }
+            // summed here, not where it is used with every value it reads held until then
+            if constexpr (GM) asm volatile("" : "+v"(kr[n]));
         }
-        double adj[6], ge, gm;
-        adj_face<2>(half ? 1.0 : -1.0, nbz, vo, uo, vn, un, geo[3 + zface], Ln, a.C0,
-                    mo, Yn, Zn, adj, ge, gm);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) zadj[c] = adj[fo + c];
-        zg = grp ? ge : gm;
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int n = 0; n < S::NST; ++n)
+                if (!past(n)) st_stream<NT>(at(a.kap_out + go + c * fs, sto[n]), a.rka * kt[c][n]);
     }
-    double Dr[N1], Ds[N1];
+    // the other faces behind the chunks'
+    if (!EARLY) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_face(0);
+    }
+    if (ONE) settle(0);
 #pragma unroll
-    for (int l = 0; l < N1; ++l) { Dr[l] = s_D[l + N1 * i]; Ds[l] = s_D[l + N1 * j]; }
-#pragma unroll LVL_UNROLL
-    for (int kk = 0; kk < KH; ++kk) {
-        const int k = k0 + kk;
-        if (k >= N1) break;
-        // transposed volume curl: sums over l with D(l, .)
-        double S1_r = 0, S2_r = 0, S0_s = 0, S2_s = 0, S0_t = 0, S1_t = 0;
+    for (int n = 1; n < S::NF; ++n) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_face(n);
+        if (ONE) settle(n);
+    }
+    if constexpr (!ONE) {
+#pragma unroll
+        for (int n = 0; n < S::NF; ++n) settle(n);
+    }
+    __syncthreads();
+
+    // ---- phase 1: each wave takes whole faces (or halves of one) ----
+#pragma unroll
+    for (int n = 0; n < S::NF; ++n) {
+        const int id = w + 2 * WG * n, f = id / S::FC;
+        if (6 * S::FC % (2 * WG) != 0 && id >= 6 * S::FC) break;
+        const int ax = f >> 1;
+        int fq = (id - f * S::FC) * 64 + lane;
+        if (N2 % 64 != 0) fq = min(fq, N2 - 1);
+        const double *s1 = s_v + pick3(ax, 1, 2, 0) * N3 + fown[n], *s2 = s_v + pick3(ax, 2, 0, 1) * N3 + fown[n];
+        const double vo[4] = {s1[0], s2[0], s1[3 * N3], s2[3 * N3]};
+        double adj[4], dq = 0.0;
+        adj_face<GM>(f & 1 ? 1.0 : -1.0, ftype[n], vo, vn[n], fd[n], fL[n][0], fL[n][1], a.C0, fy[n][0], fy[n][1],
+                     fy[n][2], fy[n][3], adj, dq);
+        double *o = s_f + f * FS * N2 + fq;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c * N2] = adj[c];
+        if constexpr (GM) o[4 * N2] = dq;
+    }
+    __syncthreads();
+
+    // ---- phase 2: this lane's levels, the transposed curl: sums over l
+    // with D(l, .) of the other group's v ----
+    const double *geo = a.geo + (int64_t)e * 9;
+    const double sgn = grp ? 1.0 : -1.0;
+    const double gx = sgn * geo[0], gy = sgn * geo[1], gz = sgn * geo[2];
+    const double *S0 = s_v + (grp ? 0 : 3) * N3, *S1 = S0 + N3, *S2 = S1 + N3;
+    double R0[KL], R1[KL], R2[KL];
+#pragma unroll
+    for (int kk = 0; kk < KL; ++kk) R0[kk] = R1[kk] = R2[kk] = 0.0;
+    {
+        double dk[S::PAD ? KL : 1];
+        if constexpr (S::PAD) {
+            const int wl = lane < N1 ? lane : 0;
+#pragma unroll
+            for (int kk = 0; kk < KL; ++kk) dk[kk] = s_D[(run_has(kk) ? k0 + kk : N1 - 1) + N1 * wl];
+        }
 #pragma unroll
         for (int l = 0; l < N1; ++l) {
-            const int pr = S::idx(l, j, k), ps = S::idx(i, l, k), pt = S::idx(i, j, l);
-            const double dlk = s_D[l + N1 * k];
-            S1_r += Dr[l] * S1[pr];
-            S2_r += Dr[l] * S2[pr];
-            S0_s += Ds[l] * S0[ps];
-            S2_s += Ds[l] * S2[ps];
-            S0_t += dlk * S0[pt];
-            S1_t += dlk * S1[pt];
-        }
-        double w[3];
-        w[0] = sgn * (gy * S2_s - gz * S1_t);
-        w[1] = sgn * (gz * S0_t - gx * S2_r);
-        w[2] = sgn * (gx * S1_r - gy * S0_s);
-        double gface = 0.0;
-        const int vloc = k * N2 + q;
-        const int64_t node = eo + vloc;
-        if (k == kz) {
+            const double v0 = S0[S::idx(i, j, l)], v1 = S1[S::idx(i, j, l)];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += zadj[c];
-            gface += zg;
-        }
-        if (i == 0) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += s_f[(0 * 8 + fo + c) * N2 + j + N1 * k];
-            gface += s_f[(0 * 8 + 6 + (1 - grp)) * N2 + j + N1 * k];
-        }
-        if (i == N1 - 1) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += s_f[(1 * 8 + fo + c) * N2 + j + N1 * k];
-            gface += s_f[(1 * 8 + 6 + (1 - grp)) * N2 + j + N1 * k];
-        }
-        if (j == 0) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += s_f[(2 * 8 + fo + c) * N2 + i + N1 * k];
-            gface += s_f[(2 * 8 + 6 + (1 - grp)) * N2 + i + N1 * k];
-        }
-        if (j == N1 - 1) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += s_f[(3 * 8 + fo + c) * N2 + i + N1 * k];
-            gface += s_f[(3 * 8 + 6 + (1 - grp)) * N2 + i + N1 * k];
-        }
-        if (grp == 1 && a.drude_off) {
-            // r_J = -a J + b E, r_E -= J/eps: lambda_E += dt b ktJ,
-            // lambda_J += dt (-v_E - a ktJ), kappa_J = a_i ktJ;
-            // d/da = -ktJ.J, d/db = ktJ.E at the stage input
-            const int dd = a.drude_off[e];
-            if (dd >= 0) {
-                const int64_t jb = (int64_t)dd * 3 * N3 + vloc;
-                const int64_t pp = (int64_t)dd * N3 + vloc;
-                const double pa = a.dpar[pp * 2 + 0], pb = a.dpar[pp * 2 + 1];
-                double sJ = 0.0, sE = 0.0;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const double lj = a.lamJ[jb + c * N3];
-                    const double kt = a.kapJ[jb + c * N3] + a.rkb * lj;
-                    const double vE = s_v[(3 + c) * N3 + S::idx(i, j, k)];
-                    w[c] += pb * kt;
-                    a.lamJ[jb + c * N3] = lj + a.dt * (-vE - pa * kt);
-                    a.kapJ[jb + c * N3] = a.rka * kt;
-                    sJ += kt * a.stJ[jb + c * N3];
-                    sE += kt * a.us[(3 + c) * fs + node];
-                }
-                a.gA[pp] -= a.dt * sJ;
-                a.gB[pp] += a.dt * sE;
+            for (int kk = 0; kk < KL; ++kk) {
+                const double d = S::PAD ? bcast_lane(dk[S::PAD ? kk : 0], l) : s_D[k0 + kk + N1 * l];
+                R0[kk] += d * v1;
+                R1[kk] += d * v0;
             }
         }
-        double *g = grp ? a.geps : a.gmu;
-        if (GM) g[node] = s_g[grp * N3 + vloc] + a.dt * gface;
+    }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const int64_t p = (fo + c) * fs + node;
-            st_stream<nt_streams<N1>()>(a.lam_out + p, lm[c][kk] + a.dt * w[c]);
+    for (int kk = 0; kk < KL; ++kk) {
+        R0[kk] *= -gz;
+        R1[kk] *= gz;
+    }
+    // the faces: along x and y every level, along z the first and last
+    if (i == 0 || i == N1 - 1) {
+        const double *fx = s_f + (i == 0 ? 0 : FS) * N2 + j + N1 * k0;
+#pragma unroll
+        for (int kk = 0; kk < KL; ++kk)
+            if (run_has(kk)) {
+                R1[kk] += fx[2 * grp * N2 + N1 * kk];
+                R2[kk] += fx[(2 * grp + 1) * N2 + N1 * kk];
+            }
+    }
+    if (j == 0 || j == N1 - 1) {
+        const double *fy2 = s_f + (j == 0 ? 2 * FS : 3 * FS) * N2 + i + N1 * k0;
+#pragma unroll
+        for (int kk = 0; kk < KL; ++kk)
+            if (run_has(kk)) {
+                R2[kk] += fy2[2 * grp * N2 + N1 * kk];
+                R0[kk] += fy2[(2 * grp + 1) * N2 + N1 * kk];
+            }
+    }
+    if (k0 == 0) {
+        const double *fz = s_f + 4 * FS * N2 + q;
+        R0[0] += fz[2 * grp * N2];
+        R1[0] += fz[(2 * grp + 1) * N2];
+    }
+    if (k0 + kn == N1) {
+        const double *fz = s_f + 5 * FS * N2 + q;
+        constexpr int KE = BASE - 1;     // the last run is a short one
+        R0[KE] += fz[2 * grp * N2];
+        R1[KE] += fz[(2 * grp + 1) * N2];
+    }
+    // keep the sums here (see box_kernel)
+#pragma unroll
+    for (int kk = 0; kk < KL; ++kk) {
+        asm volatile("" : "+v"(R0[kk]), "+v"(R1[kk]), "+v"(R2[kk]));
+    }
+    constexpr bool DSREG = N1 < 10;
+    double Dr[N1], Ds[DSREG ? N1 : 1];
+#pragma unroll
+    for (int l = 0; l < N1; ++l) Dr[l] = s_D[i + N1 * l];
+    if constexpr (DSREG) {
+#pragma unroll
+        for (int l = 0; l < N1; ++l) Ds[l] = s_D[j + N1 * l];
+    }
+#pragma unroll
+    for (int kk = 0; kk < KL; ++kk) {
+        if (!run_has(kk)) break;
+        const int k = k0 + kk;
+        double S1_r = 0, S2_r = 0, S0_s = 0, S2_s = 0;
+#pragma unroll
+        for (int l = 0; l < N1; ++l) {
+            const int pr = S::idx(l, j, k), ps = S::idx(i, l, k);
+            const double dsl = DSREG ? Ds[DSREG ? l : 0] : s_D[j + N1 * l];
+            S1_r += Dr[l] * S1[pr];
+            S2_r += Dr[l] * S2[pr];
+            S0_s += dsl * S0[ps];
+            S2_s += dsl * S2[ps];
+        }
+        R0[kk] += gy * S2_s;
+        R1[kk] -= gx * S2_r;
+        R2[kk] += gx * S1_r - gy * S0_s;
+        asm volatile("" : "+v"(R0[kk]), "+v"(R1[kk]), "+v"(R2[kk]));
+    }
+    if constexpr (!HOLD) {
+        here();
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int n = 0; n < S::NST; ++n) lm[c][n] = *at(a.lam_in + go + c * fs, sto[n]);
+    }
+    if (grp == 1 && a.drude_off) {
+        // r_J = -a J + b E, r_E -= J/eps: lambda_E += dt b ktJ,
+        // lambda_J += dt (-v_E - a ktJ), kappa_J = a_i ktJ;
+        // d/da = -ktJ.J, d/db = ktJ.E at the stage input.  In place: the
+        // lanes that repeat a node read it in the same instruction as its own
+        // lane, which alone writes
+        const int dd = a.drude_off[e];
+        if (dd >= 0) {
+            here();
+            double *const lJ = a.lamJ + (int64_t)dd * 3 * N3, *const kJ = a.kapJ + (int64_t)dd * 3 * N3;
+            const double *const sJ = a.stJ + (int64_t)dd * 3 * N3, *const uE = a.us + 3 * fs + eo;
+            double *const gA = a.gA + (int64_t)dd * N3, *const gB = a.gB + (int64_t)dd * N3;
+#pragma unroll
+            for (int n = 0; n < S::NST; ++n) {
+                if (past(n)) break;
+                const bool mine = (wg + WG * n) * 64 + lane - m == (int)(sto[n] / 8);
+                const double2 ab = *reinterpret_cast<const double2 *>(at(a.dpar + (int64_t)dd * 2 * N3, 2 * sto[n]));
+                double lj[3], kt[3], tA = 0.0, tB = 0.0;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    lj[c] = *at(lJ, sto[n], 8 * c * N3);
+                    kt[c] = *at(kJ, sto[n], 8 * c * N3) + a.rkb * lj[c];
+                    tA += kt[c] * *at(sJ, sto[n], 8 * c * N3);
+                    tB += kt[c] * *at(uE + c * fs, sto[n]);
+                }
+                const double ga = *at(gA, sto[n]) - a.dt * tA, gbn = *at(gB, sto[n]) + a.dt * tB;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    lm[c][n] += a.dt * (ab.y * kt[c]);
+                    lj[c] += a.dt * (-*place(own + c * N3, n) - ab.x * kt[c]);
+                }
+                if (mine) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        *at(lJ, sto[n], 8 * c * N3) = lj[c];
+                        *at(kJ, sto[n], 8 * c * N3) = a.rka * kt[c];
+                    }
+                    *at(gA, sto[n]) = ga;
+                    *at(gB, sto[n]) = gbn;
+                }
+            }
+        }
+    }
+
+    // ---- phase 3 ----
+    __syncthreads();   // every read of v is done
+#pragma unroll
+    for (int kk = 0; kk < KL; ++kk) {
+        if (!run_has(kk)) break;
+        const int x = S::idx(i, j, k0 + kk);
+        own[x] = R0[kk];
+        own[N3 + x] = R1[kk];
+        own[2 * N3 + x] = R2[kk];
+    }
+    __syncthreads();
+    here();
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int n = 0; n < S::NST; ++n)
+            if (!past(n)) st_stream<NT>(at(a.lam_out + go + c * fs, sto[n]), lm[c][n] + a.dt * *place(own + c * N3, n));
+    if constexpr (GM) {
+        // g_m = dt/m (+- dq of the node's faces - kt.r), dq from LDS
+        double gv[S::NST], pm[S::NST];
+#pragma unroll
+        for (int n = 0; n < S::NST; ++n) {
+            gv[n] = *at(g, sto[n]);
+            pm[n] = MAT == MAT_ELEM ? mp[e] : *at(mp + eo, sto[n]);
+        }
+#pragma unroll
+        for (int n = 0; n < S::NST; ++n) {
+            const int v = (int)(sto[n] / 8), vk = v / N2, vj = v / N1 - N1 * vk, vi = v - N1 * (v / N1);
+            const double *f = s_f + 4 * N2;
+            double dq = 0.0;
+            if (vi == 0 || vi == N1 - 1) dq += f[(vi ? FS : 0) * N2 + vj + N1 * vk];
+            if (vj == 0 || vj == N1 - 1) dq += f[(vj ? 3 * FS : 2 * FS) * N2 + vi + N1 * vk];
+            if (vk == 0 || vk == N1 - 1) dq += f[(vk ? 5 * FS : 4 * FS) * N2 + vi + N1 * vj];
+            if (!past(n)) *at(g, sto[n]) = gv[n] + a.dt * pm[n] * ((grp ? dq : -dq) - kr[n]);
         }
     }
 }

@@ -158,8 +158,8 @@ __device__ __forceinline__ void sheet_current(const StageArgs &a, int b, int q, 
 // instance reads the equal-work ranges (those with in-stage physics, whose
 // elements differ in cost; the plain instances keep the registers the table
 // would take).
-template <bool BAL>
-__device__ __forceinline__ int stage_element(const StageArgs &a, int b, int nelt) {
+template <bool BAL, class Args>
+__device__ __forceinline__ int stage_element(const Args &a, int b, int nelt) {
     if (BAL && a.xcd_bal) {
         const int x = b & 7, e = a.xcd_lo[x] + (b >> 3);
         return e < a.xcd_lo[x + 1] ? e : nelt;

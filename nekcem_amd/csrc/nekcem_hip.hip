@@ -1065,11 +1065,26 @@ int32_t stage_host(std::vector<T> &out, const T *src, int64_t n) {
     return NKC_OK;
 }
 
+// Whether a reversed stage streams its outputs and the residual past the
+// caches: once lambda and kappa, in and out, and the stage's state (30 doubles
+// a node) no longer fit the Infinity Cache.  Per stage, plain / non-temporal:
+// N = 7 at 10^3 (123 MB) 24 / 28 us, at 13^3 with the gradients (270 MB) 94 /
+// 87; N = 9 with a Drude region at 8^3 (123 MB) 39 / 43, at 12^3 (415 MB) 119
+// / 112; N = 5 with the gradients at 18^3 (302 MB) 127 / 112.
+bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
+
 int32_t launch_adjoint(const DevMesh &dm, const AdjArgs &a0, hipStream_t s) {
-    const int per_xcd = (int)((dm.nelt + 7) / 8);
-    const int grid = 8 * per_xcd;
     AdjArgs a = a0;
-    a.per_xcd = per_xcd;
+    a.per_xcd = (int)((dm.nelt + 7) / 8);
+    int len = a.per_xcd;
+    if (a.drude_off && dm.xcd_lo.size() == 9) {
+        len = 0;
+        for (int x = 0; x < 8; ++x) len = std::max(len, dm.xcd_lo[x + 1] - dm.xcd_lo[x]);
+        std::copy(dm.xcd_lo.begin(), dm.xcd_lo.end(), a.xcd_lo);
+        a.xcd_bal = 1;
+    }
+    const int grid = 8 * len;
+    const bool nt = adjoint_nt(dm.npts);
     a.D = dm.D;
     a.geo = dm.geo;
     a.nbr = dm.nbr;
@@ -1078,13 +1093,13 @@ int32_t launch_adjoint(const DevMesh &dm, const AdjArgs &a0, hipStream_t s) {
     a.fs = dm.fs;
     a.nelt = (int32_t)dm.nelt;
     switch (dm.n1) {
-    case 4: launch_adjoint_n4(a, dm.mat, grid, s); break;
-    case 5: launch_adjoint_n5(a, dm.mat, grid, s); break;
-    case 6: launch_adjoint_n6(a, dm.mat, grid, s); break;
-    case 7: launch_adjoint_n7(a, dm.mat, grid, s); break;
-    case 8: launch_adjoint_n8(a, dm.mat, grid, s); break;
-    case 9: launch_adjoint_n9(a, dm.mat, grid, s); break;
-    case 10: launch_adjoint_n10(a, dm.mat, grid, s); break;
+    case 4: launch_adjoint_n4(a, dm.mat, nt, grid, s); break;
+    case 5: launch_adjoint_n5(a, dm.mat, nt, grid, s); break;
+    case 6: launch_adjoint_n6(a, dm.mat, nt, grid, s); break;
+    case 7: launch_adjoint_n7(a, dm.mat, nt, grid, s); break;
+    case 8: launch_adjoint_n8(a, dm.mat, nt, grid, s); break;
+    case 9: launch_adjoint_n9(a, dm.mat, nt, grid, s); break;
+    case 10: launch_adjoint_n10(a, dm.mat, nt, grid, s); break;
     default: return fail(NKC_ERR_UNSUPPORTED, "polynomial order N=%d not built", dm.n1 - 1);
     }
     HIPCHK(hipGetLastError());

@@ -43,12 +43,17 @@ void launch_m(const StageArgs &a, int mode, bool nt, int grid, hipStream_t s) {
     }
 }
 
+template <int N1, int MAT, bool GM>
+void launch_adj_g(const AdjArgs &a, bool nt, int grid, hipStream_t s) {
+    const dim3 bs(BoxShape<N1>::BS);
+    if (nt) hipLaunchKernelGGL((adjoint_kernel<N1, MAT, GM, true>), dim3(grid), bs, 0, s, a);
+    else hipLaunchKernelGGL((adjoint_kernel<N1, MAT, GM, false>), dim3(grid), bs, 0, s, a);
+}
+
 template <int N1, int MAT>
-void launch_adj_t(const AdjArgs &a, int grid, hipStream_t s) {
-    if (a.rs)
-        hipLaunchKernelGGL((adjoint_kernel<N1, MAT, 1>), dim3(grid), dim3(Shape<N1>::BS), 0, s, a);
-    else
-        hipLaunchKernelGGL((adjoint_kernel<N1, MAT, 0>), dim3(grid), dim3(Shape<N1>::BS), 0, s, a);
+void launch_adj_t(const AdjArgs &a, bool nt, int grid, hipStream_t s) {
+    if (a.rs) launch_adj_g<N1, MAT, true>(a, nt, grid, s);
+    else launch_adj_g<N1, MAT, false>(a, nt, grid, s);
 }
 
 }  // namespace
@@ -61,9 +66,9 @@ void NKC_CAT(launch_stage_n, NKC_N1)(const StageArgs &a, int mat, int mode, bool
     else launch_m<NKC_N1, MAT_NODE>(a, mode, nt, grid, s);
 }
 
-void NKC_CAT(launch_adjoint_n, NKC_N1)(const AdjArgs &a, int mat, int grid, hipStream_t s) {
-    if (mat == MAT_ELEM) launch_adj_t<NKC_N1, MAT_ELEM>(a, grid, s);
-    else launch_adj_t<NKC_N1, MAT_NODE>(a, grid, s);
+void NKC_CAT(launch_adjoint_n, NKC_N1)(const AdjArgs &a, int mat, bool nt, int grid, hipStream_t s) {
+    if (mat == MAT_ELEM) launch_adj_t<NKC_N1, MAT_ELEM>(a, nt, grid, s);
+    else launch_adj_t<NKC_N1, MAT_NODE>(a, nt, grid, s);
 }
 
 #undef NKC_CAT

@@ -22,7 +22,7 @@ constexpr int box_waves(int n1, int feat) { return n1 < 7 ? 0 : (n1 == 8 && feat
 // nt: k and the outputs past the caches (see stage_nt)
 #define NKC_DECL_ORDER(n)                                                                          \
     void launch_stage_n##n(const StageArgs &a, int mat, int mode, bool nt, int grid, hipStream_t s); \
-    void launch_adjoint_n##n(const AdjArgs &a, int mat, int grid, hipStream_t s);
+    void launch_adjoint_n##n(const AdjArgs &a, int mat, bool nt, int grid, hipStream_t s);
 NKC_DECL_ORDER(4)
 NKC_DECL_ORDER(5)
 NKC_DECL_ORDER(6)
