@@ -190,6 +190,17 @@ struct DevMesh {
 // MB) 116.9 / 110.0.
 bool stage_nt(int64_t npts) { return 18.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
 
+// Whether a reversed stage streams its outputs and the residual past the
+// caches: once lambda and kappa, in and out, and the stage's state (30 doubles
+// a node) no longer fit the Infinity Cache.  Per stage, plain / non-temporal:
+// N = 7 at 10^3 (123 MB) 24 / 28 us, at 13^3 with the gradients (270 MB) 94 /
+// 87; N = 9 with a Drude region at 8^3 (123 MB) 39 / 43, at 12^3 (415 MB) 119
+// / 112; N = 5 with the gradients at 18^3 (302 MB) 127 / 112.  The forward's
+// kept stages, whose outputs no later stage of the step finds in the caches
+// again, change sides there too: N = 9 with a Drude region at 10^3 (240 MB) 60
+// / 66 us, at 12^3 115 / 98; N = 5 at 13^3 (114 MB) 25 / 30, at 18^3 80 / 70.
+bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
+
 int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     dm.n1 = m.n1;
     dm.mat = m.mat ? MAT_NODE : MAT_ELEM;
@@ -341,14 +352,15 @@ int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_
         b.xcd_bal = 1;
         grid = 8 * std::max(len, 1);
     }
+    const bool nt = a.st_r || a.st_J ? adjoint_nt(dm.npts) : dm.nt;
     switch (dm.n1) {
-    case 4: launch_stage_n4(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 5: launch_stage_n5(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 6: launch_stage_n6(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 7: launch_stage_n7(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 8: launch_stage_n8(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 9: launch_stage_n9(b, dm.mat, mode, dm.nt, grid, s); break;
-    case 10: launch_stage_n10(b, dm.mat, mode, dm.nt, grid, s); break;
+    case 4: launch_stage_n4(b, dm.mat, mode, nt, grid, s); break;
+    case 5: launch_stage_n5(b, dm.mat, mode, nt, grid, s); break;
+    case 6: launch_stage_n6(b, dm.mat, mode, nt, grid, s); break;
+    case 7: launch_stage_n7(b, dm.mat, mode, nt, grid, s); break;
+    case 8: launch_stage_n8(b, dm.mat, mode, nt, grid, s); break;
+    case 9: launch_stage_n9(b, dm.mat, mode, nt, grid, s); break;
+    case 10: launch_stage_n10(b, dm.mat, mode, nt, grid, s); break;
     default: return fail(NKC_ERR_UNSUPPORTED, "polynomial order N=%d not built", dm.n1 - 1);
     }
     HIPCHK(hipGetLastError());
@@ -1064,14 +1076,6 @@ int32_t stage_host(std::vector<T> &out, const T *src, int64_t n) {
     if (n > 0) HIPCHK(hipMemcpy(out.data(), src, sizeof(T) * (size_t)n, hipMemcpyDefault));
     return NKC_OK;
 }
-
-// Whether a reversed stage streams its outputs and the residual past the
-// caches: once lambda and kappa, in and out, and the stage's state (30 doubles
-// a node) no longer fit the Infinity Cache.  Per stage, plain / non-temporal:
-// N = 7 at 10^3 (123 MB) 24 / 28 us, at 13^3 with the gradients (270 MB) 94 /
-// 87; N = 9 with a Drude region at 8^3 (123 MB) 39 / 43, at 12^3 (415 MB) 119
-// / 112; N = 5 with the gradients at 18^3 (302 MB) 127 / 112.
-bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
 
 int32_t launch_adjoint(const DevMesh &dm, const AdjArgs &a0, hipStream_t s) {
     AdjArgs a = a0;
