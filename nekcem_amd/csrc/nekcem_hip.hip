@@ -251,6 +251,10 @@ constexpr int NLAYOUT = NKC_NLAYOUT;
 // (E lanes of a Drude element spent 33 against 18 us in the level phase at
 // N = 9, 24^3, a workgroup's life ~1.6 times the others').
 constexpr double DRUDE_WORK = 1.6;
+// The same of a PML element: 27 more doubles a node beside 24.  N = 8, 20^3,
+// per stage: 358 us with equal counts, 339 at 1.4, 330 at 1.7, 324 at 2, 328
+// at 2.4; N = 7, 16^3: 118, 111, 114, 116, 118.
+constexpr double PML_WORK = 1.7;
 
 // Whether a layout number names a kernel at this order.
 bool layout_built(int n1, int layout) {
@@ -625,6 +629,7 @@ struct nkc_handle {
     double *lL = nullptr, *lkL = nullptr, *lpar = nullptr, *lresL = nullptr;
     std::vector<int64_t> lor_slot;        // listed node -> lelem 6 n3 + vloc
     std::vector<int64_t> drude_slot;      // listed node -> compact (elem*3*n3 + vloc)
+    std::vector<int64_t> drude_elems;     // mesh elements of the region
     // host copy of the element tables (material updates, adjoint)
     HostMesh hm;
     double C0 = 1.0;
@@ -839,6 +844,36 @@ int32_t capture(nkc_handle *h, double dt) {
     }
     h->graph_dt = dt;
     return NKC_OK;
+}
+
+// Element bounds of 8 contiguous ranges of equal work, one per XCD, when
+// Drude and PML elements cost more than the others (elements in order, so
+// each XCD still takes a compact run of the mesh).  A PML fills the first and
+// the last layers of the element order: with equal counts two of the XCDs
+// would work on PML elements alone (equal counts / equal work, PML: N = 8 at
+// 12^3 76.5 / 70 us, N = 5 at 20^3 115 / 108, N = 9 at 9^3 63.0 / 61.4; Drude:
+// N = 9 at 12^3 87.6 / 84.1).  Only when the chip's resident workgroups (16
+// waves a CU) do not hold the mesh at once: there a longer range is a second
+// round on its XCD (PML, N = 9 at 8^3, one round: 40 / 51; N = 7 at 8^3 20.6 /
+// 22.5; Drude, N = 9 at 8^3 30.9 / 31.8).
+void balance_xcds(nkc_handle *h) {
+    h->m.xcd_lo.clear();
+    const int64_t n = h->m.nelt;
+    if (h->drude_elems.empty() && h->pml_elems.empty()) return;
+    if (n * stage_block(h->m.n1) <= (int64_t)256 * 16 * 64) return;
+    std::vector<double> work(n, 1.0);
+    double total = (double)n;
+    for (int64_t e : h->drude_elems) { work[e] += DRUDE_WORK - 1.0; total += DRUDE_WORK - 1.0; }
+    for (int64_t e : h->pml_elems) { work[e] += PML_WORK - 1.0; total += PML_WORK - 1.0; }
+    std::vector<int32_t> lo(9, (int32_t)n);
+    lo[0] = 0;
+    double acc = 0.0;
+    int x = 1;
+    for (int64_t e = 0; e < n && x < 8; ++e) {
+        acc += work[e];
+        while (x < 8 && acc >= total * x / 8.0) lo[x++] = (int32_t)(e + 1);
+    }
+    h->m.xcd_lo = lo;
 }
 
 // keep: leave the buffers to this handle's next nkc_adjoint_forward (see
@@ -1497,24 +1532,6 @@ int32_t nkc_set_source_time(nkc_handle *h, int32_t kind, double omega, double ph
     return drop_graphs(h);                // the captured stages carry the old factor
 }
 
-// Element bounds of 8 contiguous ranges of equal work, one per XCD, when the
-// elements with off[e] >= 0 cost w times the others (elements in order,
-// so each XCD still takes a compact run of the mesh).
-std::vector<int32_t> xcd_ranges(const std::vector<int32_t> &off, double w) {
-    const int64_t n = (int64_t)off.size();
-    double total = 0.0;
-    for (int64_t e = 0; e < n; ++e) total += off[e] >= 0 ? w : 1.0;
-    std::vector<int32_t> lo(9, (int32_t)n);
-    lo[0] = 0;
-    double acc = 0.0;
-    int x = 1;
-    for (int64_t e = 0; e < n && x < 8; ++e) {
-        acc += off[e] >= 0 ? w : 1.0;
-        while (x < 8 && acc >= total * x / 8.0) lo[x++] = (int32_t)(e + 1);
-    }
-    return lo;
-}
-
 int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, const double *params_in,
                       const double *J_in, const double *kJ_in) {
     if (!h) return fail(NKC_ERR_ARG, "null handle");
@@ -1544,7 +1561,8 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     h->ndrude = 0;
     h->ndelem = 0;
     h->drude_slot.clear();
-    h->m.xcd_lo.clear();
+    h->drude_elems.clear();
+    balance_xcds(h);
     int32_t rc = drop_graphs(h);
     if (rc || ndrude == 0) return rc;
     if (ndrude < 0 || !dindex || !params) return fail(NKC_ERR_ARG, "bad Drude node list");
@@ -1578,7 +1596,9 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     if ((rc = upload(&h->drude_off, off))) return rc;   // last: switches the term on
     h->ndrude = ndrude;
     h->ndelem = nde;
-    h->m.xcd_lo = xcd_ranges(off, DRUDE_WORK);
+    for (int64_t e = 0; e < m.nelt; ++e)
+        if (off[e] >= 0) h->drude_elems.push_back(e);
+    balance_xcds(h);
     return NKC_OK;
 }
 
@@ -1826,6 +1846,7 @@ void free_pml(nkc_handle *h) {
     (void)hipFree(h->presP); h->presP = nullptr;
     h->npml = 0;
     h->pml_elems.clear();
+    balance_xcds(h);
 }
 
 // Install a PML on the mesh elements `elems` (0-based, ascending): sig and
@@ -1843,6 +1864,7 @@ int32_t install_pml(nkc_handle *h, const std::vector<int64_t> &elems, const std:
     if ((rc = upload(&h->pml_off, off))) return rc;     // last: switches the term on
     h->npml = (int64_t)elems.size();
     h->pml_elems = elems;
+    balance_xcds(h);
     return NKC_OK;
 }
 
