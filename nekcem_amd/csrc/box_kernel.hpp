@@ -47,6 +47,9 @@
 
 namespace nkc {
 
+// Runs a workgroup splits a group's levels into.
+constexpr int level_runs(int n1) { return n1 <= 5 ? n1 : (n1 % 3 == 0 ? 3 : 2); }
+
 // Launch shape and LDS layout for polynomial order N1 - 1.
 //   A group's levels are split into KS runs of (N+1)^2 lanes: padded to
 //   whole waves (PAD) when two runs fill them well (N = 7: 64 of 64 lanes,
@@ -59,7 +62,7 @@ namespace nkc {
 template <int N1>
 struct BoxShape {
     static constexpr int N2 = N1 * N1, N3 = N2 * N1;
-    static constexpr int KS = N1 <= 5 ? N1 : (N1 % 3 == 0 ? 3 : 2);
+    static constexpr int KS = level_runs(N1);
     static constexpr bool PAD = KS == 2;
     static constexpr int PL = PAD ? (N2 + 63) / 64 * 64 : N2;        // lanes per run of levels
     static constexpr int GL = (KS * PL + 63) / 64 * 64;              // lanes per group
@@ -184,12 +187,17 @@ __device__ __forceinline__ void load_coef(const StageArgs &a, int e, int f, int 
 // NT: non-temporal k loads and output stores (chosen by the launcher from
 // the mesh's size).
 // OCC > 0: waves per SIMD the register allocator keeps to.
-template <int N1, int MAT, int MODE, int FEAT, bool NT, int OCC>
+// SL > 1: an element in SL workgroups, each with a slab of its levels (small
+// meshes without a sheet, whose state a face's one workgroup updates; see
+// stage_slabs).
+template <int N1, int MAT, int MODE, int FEAT, bool NT, int OCC, int SL = 1>
 __global__ void __launch_bounds__(BoxShape<N1>::BS) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1)))
 box_kernel(StageArgs a) {
     using S = BoxShape<N1>;
-    constexpr int N2 = S::N2, N3 = S::N3, KL = S::KL, WG = S::WG;
+    constexpr int RUNS = S::KS * SL;         // runs of levels of an element
+    constexpr int N2 = S::N2, N3 = S::N3, KL = (N1 + RUNS - 1) / RUNS, WG = S::WG;
     constexpr bool RK = MODE != MODE_RESIDUAL;
+    static_assert(SL == 1 || (FEAT <= 2 && RUNS <= N1), "slabs");
     // N = 9: the misaligned level loads of k measured 507 us plain, 518
     // non-temporal (24^3); every other order 3-4 % faster non-temporal
     constexpr bool NTK = NT && N1 != 10;
@@ -198,7 +206,10 @@ box_kernel(StageArgs a) {
     __shared__ double s_f[6 * FS * N2];     // [face][FH t1, FH t2, FE t1, FE t2 (, FE n)][a + n1 b]
     __shared__ double s_D[N2];              // D(i,l) at [i + n1 l]
 
-    const int e = stage_element<(FEAT >= 1)>(a, blockIdx.x, a.nelt);
+    // an element's slabs follow each other on its XCD
+    const int slab = SL > 1 ? (blockIdx.x >> 3) % SL : 0;
+    const int e = stage_element<(FEAT >= 1)>(a, SL > 1 ? (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / SL) : blockIdx.x,
+                                             a.nelt);
     if (e >= a.nelt) return;
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -218,10 +229,15 @@ box_kernel(StageArgs a) {
         q = r2 - part * N2;
     }
     const int j = q / N1, i = q - j * N1;
-    constexpr int BASE = N1 / S::KS, REM = N1 % S::KS;
-    const int k0 = part * BASE + (part < REM ? part : REM);
-    const int kn = BASE + (part < REM ? 1 : 0);
+    constexpr int BASE = N1 / RUNS, REM = N1 % RUNS;
+    const int run = slab * S::KS + part;
+    const int k0 = run * BASE + (run < REM ? run : REM);
+    const int kn = BASE + (run < REM ? 1 : 0);
     const int64_t eo = (int64_t)e * N3, fs = a.fs;
+    // the slab's nodes, x0 to x1
+    const int ra = slab * S::KS, rb = ra + S::KS;
+    const int x0 = SL > 1 ? N2 * (ra * BASE + min(ra, REM)) : 0, x1 = SL > 1 ? N2 * (rb * BASE + min(rb, REM)) : N3;
+    constexpr int NX = SL > 1 ? N2 * S::KS * KL : N3;    // at most
 
     // ---- phase 0: every global load of the element, issued up front ----
     const double *ug = a.uin + 3 * grp * fs + eo;
@@ -612,13 +628,18 @@ box_kernel(StageArgs a) {
         // -a J - b P + c E, resP = J; the RK update from the stage-start E
         // (still in LDS), in the order of memory: every load of an element
         // at once instead of a round trip per level.  Each node by one lane.
+        constexpr int NLX = SL > 1 ? ((NX + 63) / 64 + WG - 1) / WG : S::NLD;
+        auto place = [&](int v) {
+            if (SL > 1) return S::idx(v % N1, v / N1 % N1, v / N2);
+            return S::SWZ ? (v - lane) + S::idx(lane % N1, (lane / N1) % N1, lane / N2) : v;
+        };
         if (dd >= 0) {
             const int64_t jb = (int64_t)dd * 3 * N3;
 #pragma unroll
-            for (int n = 0; n < S::NLD; ++n) {
-                const int v = (wg + WG * n) * 64 + lane;
-                if (v >= N3) continue;
-                const double *uo = own + (S::SWZ ? (v - lane) + S::idx(lane % N1, (lane / N1) % N1, lane / N2) : v);
+            for (int n = 0; n < NLX; ++n) {
+                const int v = x0 + (wg + WG * n) * 64 + lane;
+                if (v >= x1) continue;
+                const double *uo = own + place(v);
                 const double pa = a.dpar[((int64_t)dd * N3 + v) * 2], pb = a.dpar[((int64_t)dd * N3 + v) * 2 + 1];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
@@ -639,10 +660,10 @@ box_kernel(StageArgs a) {
         if (lo >= 0) {
             const int64_t lb = (int64_t)lo * 6 * N3;
 #pragma unroll
-            for (int n = 0; n < S::NLD; ++n) {
-                const int v = (wg + WG * n) * 64 + lane;
-                if (v >= N3) continue;
-                const double *uo = own + (S::SWZ ? (v - lane) + S::idx(lane % N1, (lane / N1) % N1, lane / N2) : v);
+            for (int n = 0; n < NLX; ++n) {
+                const int v = x0 + (wg + WG * n) * 64 + lane;
+                if (v >= x1) continue;
+                const double *uo = own + place(v);
                 const double *lp = a.lpar + ((int64_t)lo * N3 + v) * 3;
                 const double la = lp[0], lbp = lp[1], lc = lp[2];
 #pragma unroll
@@ -668,13 +689,15 @@ box_kernel(StageArgs a) {
     if constexpr (RK) {
         // ---- phase 3: the outputs leave in the order of memory, 64-node
         // chunks that start on 128-byte lines, first k, then u ----
-        const int m = S::G == 16 ? 0 : (int)(eo & 15);
-        unsigned sto[S::NST];
+        constexpr bool LINE = S::G == 16 && (SL == 1 || (N2 * S::KS * BASE % 16 == 0 && REM == 0));
+        constexpr int NST = SL > 1 ? ((NX + (LINE ? 0 : 15) + 63) / 64 + WG - 1) / WG : S::NST;
+        const int m = LINE ? 0 : (int)((eo + x0) & 15);
+        unsigned sto[NST];
 #pragma unroll
-        for (int n = 0; n < S::NST; ++n) {
-            int x = (wg + WG * n) * 64 + lane - m;
-            if (S::G != 16 && n == 0) x = max(x, 0);
-            if ((n + 1) * WG * 64 > N3) x = min(x, N3 - 1);
+        for (int n = 0; n < NST; ++n) {
+            int x = x0 + (wg + WG * n) * 64 + lane - m;
+            if (!LINE && n == 0) x = max(x, x0);
+            if (SL > 1 || (n + 1) * WG * 64 > N3) x = min(x, x1 - 1);
             sto[n] = 8u * (unsigned)x;
         }
         auto flush = [&](double *dst) {
@@ -682,10 +705,17 @@ box_kernel(StageArgs a) {
 #pragma unroll
             for (int c = 0; c < 3; ++c)
 #pragma unroll
-                for (int n = 0; n < S::NST; ++n) {
-                    // a chunk past the element's end (N = 4 only)
-                    if (S::WG * S::NST * 64 - N3 >= 64 && (wg + WG * n) * 64 - m >= N3) break;
+                for (int n = 0; n < NST; ++n) {
+                    // a chunk past the end (N = 4, and slabs)
+                    if (SL > 1 ? x0 + (wg + WG * n) * 64 - m >= x1
+                               : S::WG * NST * 64 - N3 >= 64 && (wg + WG * n) * 64 - m >= N3)
+                        break;
                     const double *x = own + c * N3;
+                    if (SL > 1 && S::SWZ) {
+                        const int v = (int)(sto[n] / 8);
+                        st_stream<NT>(at(p + c * fs, sto[n]), x[S::idx(v % N1, v / N1 % N1, v / N2)]);
+                        continue;
+                    }
                     const double v = S::SWZ ? x[(wg + WG * n) * 64 + S::idx(lane % N1, (lane / N1) % N1, lane / N2)] : *at(x, sto[n]);
                     st_stream<NT>(at(p + c * fs, sto[n]), v);
                 }

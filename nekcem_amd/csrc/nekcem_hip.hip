@@ -201,6 +201,22 @@ bool stage_nt(int64_t npts) { return 18.0 * sizeof(double) * (double)npts > 256.
 // / 66 us, at 12^3 115 / 98; N = 5 at 13^3 (114 MB) 25 / 30, at 18^3 80 / 70.
 bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
 
+// Workgroups an element is split over: the most whose slabs fit the 256 CUs
+// side by side, so that a small mesh does not leave CUs idle while a few work
+// through whole elements; each loads the whole element and takes its own levels.
+// Per stage, one workgroup / slabs: N = 7 at 4^3 7.7 / 5.0 us (4), at 5^3 8.2
+// / 6.1 (2; 6.6 at 4), N = 5 at 4^3 5.0 / 4.3 (2), N = 6 at 4^3 6.5 / 5.3 (2),
+// N = 8 at 4^3 8.7 / 6.3 (3), at 6^3 10.1 / 11.6 (2), N = 9 at 3^3 11.5 / 6.3
+// (5), at 5^3 12.7 / 10.1 (2), at 6^3 13.6 / 14.5 (2); with a Drude region N =
+// 7 at 4^3 10.8 / 7.3, N = 9 at 4^3 17.3 / 11.1; with a PML N = 9 at 5^3 27.4 /
+// 16.9.  N = 7's 4-wave workgroups gain from two slabs up to two per CU: 6^3
+// 8.6 / 7.9, 8^3 12.5 / 12.1.
+int stage_slabs(int n1, int64_t nelt) {
+    for (int sl = 5; sl > 1; --sl)
+        if (slabs_built(n1, sl) && nelt * sl <= 256) return sl;
+    return n1 == 8 && nelt <= 512 ? 2 : 1;
+}
+
 int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     dm.n1 = m.n1;
     dm.mat = m.mat ? MAT_NODE : MAT_ELEM;
@@ -357,14 +373,16 @@ int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_
         grid = 8 * std::max(len, 1);
     }
     const bool nt = a.st_r || a.st_J ? adjoint_nt(dm.npts) : dm.nt;
+    const bool whole = mode != MODE_RK || nt || a.gr_off || a.st_r || a.st_J || b.xcd_bal;
+    const int sl = whole ? 1 : stage_slabs(dm.n1, dm.nelt);
     switch (dm.n1) {
-    case 4: launch_stage_n4(b, dm.mat, mode, nt, grid, s); break;
-    case 5: launch_stage_n5(b, dm.mat, mode, nt, grid, s); break;
-    case 6: launch_stage_n6(b, dm.mat, mode, nt, grid, s); break;
-    case 7: launch_stage_n7(b, dm.mat, mode, nt, grid, s); break;
-    case 8: launch_stage_n8(b, dm.mat, mode, nt, grid, s); break;
-    case 9: launch_stage_n9(b, dm.mat, mode, nt, grid, s); break;
-    case 10: launch_stage_n10(b, dm.mat, mode, nt, grid, s); break;
+    case 4: launch_stage_n4(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 5: launch_stage_n5(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 6: launch_stage_n6(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 7: launch_stage_n7(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 8: launch_stage_n8(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 9: launch_stage_n9(b, dm.mat, mode, nt, sl, grid, s); break;
+    case 10: launch_stage_n10(b, dm.mat, mode, nt, sl, grid, s); break;
     default: return fail(NKC_ERR_UNSUPPORTED, "polynomial order N=%d not built", dm.n1 - 1);
     }
     HIPCHK(hipGetLastError());
