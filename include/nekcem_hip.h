@@ -130,8 +130,7 @@ int32_t nkc_get_state(nkc_handle *h, double *hn, double *en, double *khn,
 int32_t nkc_get_state_at(nkc_handle *h, int64_t n, const int64_t *nodes, double *out);
 
 /* nsteps calls of cem_maxwell_op_rk (src/cem_maxwell.F:327-345): 5-stage
- * low-storage RK per step, each stage one fused kernel, the step replayed
- * from a captured hipGraph.  *time += nsteps*dt (time_advancing_pde,
+ * low-storage RK per step, each stage one fused kernel.  *time += nsteps*dt (time_advancing_pde,
  * src/cem_drive.F:639).  Asynchronous on the handle's stream; the next
  * get_state or nkc_sync waits for it. */
 int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps);
@@ -395,10 +394,11 @@ int32_t nkc_stream(nkc_handle *h, void **stream);
  * (0 per element, 1 per node), out[2] = elements per workgroup,
  * out[3] = threads per workgroup (general handles: 256, whatever their kernel
  * takes), out[4] = LDS bytes per workgroup,
- * out[5] = graph capture enabled (1/0). */
+ * out[5] = the setting of nkc_set_graph. */
 int32_t nkc_info(nkc_handle *h, int64_t out[8]);
 
-/* Enable (1, default) or disable (0) hipGraph replay in nkc_step. */
+/* 1 (default) or 0, reported by nkc_info.  nkc_step launches its kernels
+ * directly with either: replaying a captured step took 3 us longer. */
 int32_t nkc_set_graph(nkc_handle *h, int32_t enable);
 
 /* Stage-kernel layouts (no counterpart in the reference): numbers a caller

@@ -3,10 +3,10 @@
 // Host side of the MI355X Maxwell step.  A mesh of one polynomial order is a
 // DevMesh: the compact per-element tables of mesh_tables.hpp on the device
 // plus the ping-pong state buffers and the RK register.  A handle
-// (nkc_create / nkc_create_box) owns one DevMesh, a stream and the captured
-// step graphs; a batch (nkc_batch_create) owns one DevMesh per polynomial
-// order holding all its cavities back to back, one stream per order, and a
-// graph whose per-order branches run side by side.
+// (nkc_create / nkc_create_box) owns one DevMesh and a stream; a batch
+// (nkc_batch_create) owns one DevMesh per polynomial order holding all its
+// cavities back to back, one stream per order, and a graph whose per-order
+// branches run side by side.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -522,7 +522,7 @@ __device__ double src_factor(const SrcTime &s, double t) {
 
 // Start of a step whose stages need the time: t[2 + 2 s], t[3 + 2 s] = time
 // and source factor of stage s, then time = time + dt (src/cem_drive.F:639)
-// on the device, so a replayed graph sees the right stage times.  One small
+// on the device, so a step needs no value from the host.  One small
 // launch a step instead of an exp or sin in every lane of every stage (N =
 // 8, 22^3, source: 308 -> 290 us per stage).
 struct StageC {
@@ -605,8 +605,6 @@ struct nkc_handle {
     int cur = 0;                          // which u buffer holds the state
     bool use_graph = true;
     bool keep_k = false;                  // last stage writes the RK register (nkc_set_keep_k)
-    double graph_dt = NAN;
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
     // t_host: time at the start of the next step.  tdev (14 doubles): [0] the
     // same on the device, kept when a source or an incident field needs it
     // (tdev_ok: it is current); [2 + 2 s], [3 + 2 s] the time and source
@@ -831,39 +829,6 @@ int32_t queue_step(nkc_handle *h, int from, double dt) {
     return NKC_OK;
 }
 
-int32_t drop_graphs(nkc_handle *h) {
-    for (int i = 0; i < 2; ++i)
-        if (h->gexec[i]) {
-            HIPCHK(hipGraphExecDestroy(h->gexec[i]));
-            h->gexec[i] = nullptr;
-        }
-    h->graph_dt = NAN;
-    return NKC_OK;
-}
-
-int32_t capture(nkc_handle *h, double dt) {
-    int32_t rc = drop_graphs(h);
-    if (rc) return rc;
-    for (int from = 0; from < 2; ++from) {
-        HIPCHK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-        rc = queue_step(h, from, dt);
-        hipGraph_t g = nullptr;
-        const hipError_t ee = hipStreamEndCapture(h->stream, &g);
-        if (rc || ee != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
-            return rc ? rc : fail(NKC_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(ee));
-        }
-        const hipError_t ei = hipGraphInstantiate(&h->gexec[from], g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (ei != hipSuccess) {
-            h->gexec[from] = nullptr;
-            return fail(NKC_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(ei));
-        }
-    }
-    h->graph_dt = dt;
-    return NKC_OK;
-}
-
 // Element bounds of 8 contiguous ranges of equal work, one per XCD, when
 // Drude and PML elements cost more than the others (elements in order, so
 // each XCD still takes a compact run of the mesh).  A PML fills the first and
@@ -978,7 +943,6 @@ int32_t node_list(nkc_handle *h, int64_t n, const int64_t *nodes, int64_t **dn, 
 }
 
 void free_handle(nkc_handle *h) {
-    drop_graphs(h);
     free_adjoint(h);
     (void)hipFree(h->yz);
     h->yz = nullptr;
@@ -1166,8 +1130,7 @@ int32_t launch_adjoint(const DevMesh &dm, const AdjArgs &a0, hipStream_t s) {
 // One forward step of the segment recompute: stage s of step `slot` reads
 // its input from stage store slot 5 slot + s and writes the next stage's
 // input to the following slot, so every stage input is kept at no extra
-// traffic; the stage residual goes to the matching st_r slot (not captured:
-// the store offsets change with the slot).
+// traffic; the stage residual goes to the matching st_r slot.
 int32_t queue_step_store(nkc_handle *h, double dt, int64_t slot) {
     const int64_t blk = 6 * h->m.fs;
     auto &A = h->adj;
@@ -1422,21 +1385,12 @@ int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps) {
     if (h->m.layout < 0) h->m.layout = 0;
     const int32_t rt = current_time(h);
     if (rt) return rt;
-    if (h->use_graph) {
-        if (!(h->graph_dt == dt)) {
-            const int32_t rc = capture(h, dt);
-            if (rc) return rc;
-        }
-        for (int64_t s = 0; s < nsteps; ++s) {
-            HIPCHK(hipGraphLaunch(h->gexec[h->cur], h->stream));
-            h->cur ^= 1;
-        }
-    } else {
-        for (int64_t s = 0; s < nsteps; ++s) {
-            const int32_t rc = queue_step(h, h->cur, dt);
-            if (rc) return rc;
-            h->cur ^= 1;
-        }
+    // direct launches: a captured step replayed took 3 us longer at every size
+    // (4^3: N = 5 28.0 / 24.5 us, N = 7 41.4 / 38.3; 3^3, N = 9 60.8 / 57.5)
+    for (int64_t s = 0; s < nsteps; ++s) {
+        const int32_t rc = queue_step(h, h->cur, dt);
+        if (rc) return rc;
+        h->cur ^= 1;
     }
     for (int64_t s = 0; s < nsteps; ++s) time_passed(h, dt);   // same sums as the device
     if (time) *time = h->t_host;
@@ -1505,8 +1459,8 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->src_off); h->src_off = nullptr;
     (void)hipFree(h->src_amp); h->src_amp = nullptr;
-    int32_t rc = drop_graphs(h);
-    if (rc || !amp) return rc;
+    int32_t rc = NKC_OK;
+    if (!amp) return rc;
     if (!dir || !(tw != 0.0) || !std::isfinite(t0) || !std::isfinite(tw)) return fail(NKC_ERR_ARG, "bad source direction/time");
     const DevMesh &m = h->m;
     const int n1 = m.n1, n2 = n1 * n1, n3 = n2 * n1;
@@ -1547,7 +1501,7 @@ int32_t nkc_set_source_time(nkc_handle *h, int32_t kind, double omega, double ph
     h->src_kind = kind;
     h->src_om = omega;
     h->src_ph = phase;
-    return drop_graphs(h);                // the captured stages carry the old factor
+    return NKC_OK;
 }
 
 int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, const double *params_in,
@@ -1581,8 +1535,8 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     h->drude_slot.clear();
     h->drude_elems.clear();
     balance_xcds(h);
-    int32_t rc = drop_graphs(h);
-    if (rc || ndrude == 0) return rc;
+    int32_t rc = NKC_OK;
+    if (ndrude == 0) return rc;
     if (ndrude < 0 || !dindex || !params) return fail(NKC_ERR_ARG, "bad Drude node list");
     const DevMesh &m = h->m;
     const int n3 = m.n1 * m.n1 * m.n1;
@@ -1648,7 +1602,6 @@ int32_t nkc_set_coords(nkc_handle *h, const double *xm1, const double *ym1, cons
     HIPCHK(hipStreamSynchronize(h->stream));
     h->hxyz = xyz;
     if (h->xyz) {
-        // in place: captured steps that read the coordinates stay valid
         HIPCHK(hipMemcpy(h->xyz, xyz.data(), sizeof(double) * xyz.size(), hipMemcpyHostToDevice));
         return NKC_OK;
     }
@@ -1802,8 +1755,8 @@ int32_t nkc_set_lorentz(nkc_handle *h, int64_t nlor, const int32_t *lindex, cons
     h->nlor = 0;
     h->nlelem = 0;
     h->lor_slot.clear();
-    int32_t rc = drop_graphs(h);
-    if (rc || nlor == 0) return rc;
+    int32_t rc = NKC_OK;
+    if (nlor == 0) return rc;
     if (nlor < 0 || !lindex || !params) return fail(NKC_ERR_ARG, "bad Lorentz node list");
     const DevMesh &m = h->m;
     const int n3 = m.n1 * m.n1 * m.n1;
@@ -1892,7 +1845,7 @@ int32_t reset_pml(nkc_handle *h) {
     free_adjoint(h);
     h->m.layout = -1;                     // the step's kernel instance may change
     free_pml(h);
-    return drop_graphs(h);
+    return NKC_OK;
 }
 
 }  // namespace
@@ -2040,8 +1993,8 @@ int32_t nkc_set_graphene(nkc_handle *h, int64_t ngraph, const int32_t *graphinde
     free_adjoint(h);
     h->m.layout = -1;                     // the step's kernel instance may change
     free_sheet(h);
-    int32_t rc = drop_graphs(h);
-    if (rc || ngraph == 0) return rc;
+    int32_t rc = NKC_OK;
+    if (ngraph == 0) return rc;
     const int64_t nelt = h->m.nelt;
     const int n1 = h->m.n1, n2 = n1 * n1;
     const int64_t nxzfl = nelt * 6 * n2;
@@ -2132,8 +2085,8 @@ int32_t nkc_set_incident(nkc_handle *h, int64_t nface, const int32_t *faces, con
     h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->inc_mask); h->inc_mask = nullptr;
     h->ninc = 0;
-    int32_t rc = drop_graphs(h);
-    if (rc || nface == 0) return rc;
+    int32_t rc = NKC_OK;
+    if (nface == 0) return rc;
     if (nface < 0 || !faces || !k || !hamp || !eamp) return fail(NKC_ERR_ARG, "bad incident-field face list");
     for (int c = 0; c < 3; ++c)
         if (!std::isfinite(k[c]) || !std::isfinite(hamp[c]) || !std::isfinite(eamp[c]))
@@ -2253,7 +2206,6 @@ int32_t nkc_set_graph(nkc_handle *h, int32_t enable) {
     if (!h) return fail(NKC_ERR_ARG, "null handle");
     HIPCHK(hipStreamSynchronize(h->stream));
     h->use_graph = enable != 0;
-    if (!h->use_graph) return drop_graphs(h);
     return NKC_OK;
 }
 
@@ -2262,7 +2214,7 @@ int32_t nkc_set_keep_k(nkc_handle *h, int32_t keep) {
     HIPCHK(hipStreamSynchronize(h->stream));
     if (h->keep_k == (keep != 0)) return NKC_OK;
     h->keep_k = keep != 0;
-    return drop_graphs(h);   // the captured step carries the stage flags
+    return NKC_OK;
 }
 
 int32_t nkc_set_layout(nkc_handle *h, int32_t layout) {
@@ -2275,7 +2227,7 @@ int32_t nkc_set_layout(nkc_handle *h, int32_t layout) {
         return fail(NKC_ERR_UNSUPPORTED, "layout %d carries no PML, incident field or graphene sheet", layout);
     HIPCHK(hipStreamSynchronize(h->stream));
     h->m.layout = layout;
-    return drop_graphs(h);
+    return NKC_OK;
 }
 
 int32_t nkc_get_layout(nkc_handle *h, double *out) {
@@ -2292,7 +2244,6 @@ int32_t nkc_tune(nkc_handle *h, double *out) {
     int32_t rc = tune_stage(h->m, &f, drude_size(h), lorentz_size(h), pml_size(h), sheet_size(h), h->m.u[h->cur], h->stream,
                        h->tune_us);
     if (rc) return rc;
-    if ((rc = drop_graphs(h))) return rc;
     if (out) {
         for (int l = 0; l < NLAYOUT; ++l) out[l] = h->tune_us[l];
         out[NLAYOUT] = h->m.layout;
@@ -2379,7 +2330,7 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps, const double *mu) {
         sheet_coefs(h, par);
         HIPCHK(hipMemcpy(h->gpar, par.data(), sizeof(double) * par.size(), hipMemcpyHostToDevice));
     }
-    return drop_graphs(h);
+    return NKC_OK;
 }
 
 namespace {
