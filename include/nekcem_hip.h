@@ -421,8 +421,7 @@ int32_t nkc_get_layout(nkc_handle *h, double *out);
 /* ---- batches of independent cavities --------------------------------
  * Many independent box cavities of different sizes and polynomial orders
  * advance together: cavities of one order share one element table, each
- * order's RK stage is one launch, the orders run side by side, and a whole
- * step is one graph replay.  The reference's only way to run independent
+ * order's RK stage is one launch, and the orders run side by side.  The reference's only way to run independent
  * cases at once is one MPI session per case (neknek, src/nek5_comm_mpi.F:
  * 45-119); no entry point there corresponds to these. */
 typedef struct nkc_batch nkc_batch;
