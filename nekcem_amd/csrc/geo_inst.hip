@@ -8,7 +8,7 @@ namespace nkc {
 namespace {
 template <int N1>
 void launch_geo_n(const GeoArgs &a, int mode, bool nt, int grid, hipStream_t s) {
-    const dim3 g(grid), bs(geo_block(N1));
+    const dim3 g(grid), bs(geo_block(N1, mode == GMODE_RK && nt));
     if (mode == GMODE_RK && nt) hipLaunchKernelGGL((geo_stage_kernel<N1, GMODE_RK, true>), g, bs, 0, s, a);
     else if (mode == GMODE_RK) hipLaunchKernelGGL((geo_stage_kernel<N1, GMODE_RK, false>), g, bs, 0, s, a);
     else if (mode == GMODE_RESIDUAL) hipLaunchKernelGGL((geo_stage_kernel<N1, GMODE_RESIDUAL, false>), g, bs, 0, s, a);

@@ -60,8 +60,12 @@ struct GeoArgs {
 };
 
 // Lanes of a workgroup: 16 waves per CU at one (N = 11), two (N = 8..10) or
-// three to four workgroups per CU, what their LDS allows.
-constexpr int geo_block(int n1) { return n1 >= 12 ? 1024 : n1 >= 9 ? 512 : 256; }
+// three to four workgroups per CU, what their LDS allows.  At N = 7 the three
+// 4-wave workgroups its LDS allows on a CU serve meshes whose stages stream
+// (nt), two of 8 waves with one face node a lane those in the caches: 6^3
+// 10.1 / 9.5 us, 8^3 18.4 / 16.7, 10^3 31.2 / 29.6, 12^3 48.4 / 47.2, 16^3
+// 134.9 / 141.5.
+constexpr int geo_block(int n1, bool nt) { return n1 >= 12 ? 1024 : n1 >= 9 || (n1 == 8 && !nt) ? 512 : 256; }
 
 // In-element volume index of in-face node q = a + n1 b on the reference's
 // face ef0 + 1 (0: y-, 1: x+, 2: y+, 3: x-, 4: z-, 5: z+), skpdat order
@@ -81,9 +85,9 @@ __device__ __forceinline__ int ed_face_node(int ef0, int q) {
 }
 
 template <int N1, int MODE, bool NT>
-__global__ void __launch_bounds__(geo_block(N1)) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(geo_block(N1, NT)) __attribute__((amdgpu_waves_per_eu(4)))
 geo_stage_kernel(GeoArgs a) {
-    constexpr int N2 = N1 * N1, N3 = N2 * N1, BS = geo_block(N1), W = BS / 64, GL = BS / 2, NFN = 6 * N2;
+    constexpr int N2 = N1 * N1, N3 = N2 * N1, BS = geo_block(N1, NT), W = BS / 64, GL = BS / 2, NFN = 6 * N2;
     constexpr int CH = (N3 + 63) / 64, NLD = (6 * CH + W - 1) / W, NFL = (NFN + BS - 1) / BS;
     __shared__ double s_u[6 * N3];
     __shared__ double s_f[6 * NFN];      // [FH 0..2, FE 0..2][face node of the slab]

@@ -11,7 +11,7 @@ struct GeoArgs;
 constexpr int GEO_MIN_N1 = 4, GEO_MAX_N1 = 12;
 
 // Launch one stage (mode: GMODE_RK, GMODE_RESIDUAL, GMODE_CURL; nt: k and
-// the outputs past the caches) over grid workgroups of geo_block(n1) lanes;
+// the outputs past the caches) over grid workgroups of geo_block lanes;
 // false if the order is not built.
 bool launch_geo(const GeoArgs &a, int n1, int mode, bool nt, int grid, hipStream_t s);
 
