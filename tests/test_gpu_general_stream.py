@@ -1,10 +1,8 @@
 """The general kernel at N = 7 on a mesh whose stages stream past the caches
-(workgroups of four waves) against the same elements on a small mesh (eight
-waves): blocks of a curved mesh side by side, unconnected.
-
-Tolerance: coordinates shifted by up to 1400 round at 2e-13, which is 1e-11 of
-a metric at a node spacing of 0.03; a step changes the fields by dt times their
-derivative, about a hundredth, so two steps stay below 1e-12; 1e-11 is asked.
+(workgroups of four waves) against the first of its elements on a mesh that
+does not (eight waves): blocks of a curved mesh side by side, unconnected.
+The blocks both meshes have lie at the same coordinates and every node sums
+in the same order, so they are equal bit for bit.
 """
 import numpy as np
 import pytest
@@ -18,19 +16,18 @@ pytestmark = pytest.mark.gpu
 
 def test_streamed_mesh_equals_small_mesh():
     print("[case] general stream N=7", flush=True)
-    N, copies = 7, 912
+    N, few, many = 7, 70, 912
     rng = np.random.default_rng(1)
     n = 4 * (N + 1) ** 3
     F = rng.standard_normal((6, n))
     out = []
-    for c in (70, copies):
+    for c in (few, many):
         mesh = _mesh(N, c)
         s = MaxwellSolver(mesh)
-        assert (s.npts * 18 * 8 > 256 * 2 ** 20) == (c == copies)
+        assert (s.npts * 18 * 8 > 256 * 2 ** 20) == (c == many)
         V = np.tile(F, (1, c))
         s.set_state(V[:3], V[3:])
         s.step(1e-4, 2)
-        out.append(np.concatenate(s.get_state()).reshape(6, c, n))
+        out.append(np.concatenate(s.get_state()).reshape(6, c, n)[:, :few])
         s.close()
-    want = out[0][:, :1]
-    assert np.max(np.abs(out[1] - want)) <= 1e-11 * np.max(np.abs(want))
+    assert np.array_equal(out[0], out[1])
