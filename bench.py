@@ -354,7 +354,7 @@ def dispersive(nel=24, N=9, nsteps=2000, every=100, ndir=2, nprobe=64, seed=5, l
     t_adj = time.perf_counter() - t0
     g_gam = np.bincount(owner, weights=ga, minlength=ne)
     g_wp = 2.0 * wp * np.bincount(owner, weights=gb, minlength=ne)
-    lay = s.layout()
+    lay = s.layout()["layout"]
     print(f"[bench] dispersive: stage layout {lay}", file=log, flush=True)
     print(f"[bench] dispersive: forward {t_fwd:.3f} s ({nsteps} steps), forward+checkpoints "
           f"{t_fwd_ckpt:.3f} s, backward {t_adj:.3f} s, loss {loss:.4e}, adjoint {info}",
@@ -484,7 +484,7 @@ def main():
         solver.set_layout(args.layout)
     solver.step(dt, args.warmup)
     solver.sync()
-    layout = solver.layout()
+    layout = solver.layout()["layout"]
     print(f"[bench] stage layout {layout}", file=sys.stderr, flush=True)
     timer = StreamTimer(solver.stream())
     solver.sync()
@@ -570,7 +570,7 @@ def main():
                                f"{npts} GLL points x 6 fields, per-element eps U[1,4], "
                                f"8 plane waves, upwind, CFL 0.25, RK5 (5 stages/step)",
                    "nelt": mesh.nelt, "N": args.N, "npts": npts,
-                   "graph": not args.no_graph, "stage_layout": layout},
+                   "graph": False, "stage_layout": layout},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": traffic_src,

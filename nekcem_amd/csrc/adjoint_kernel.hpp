@@ -27,10 +27,10 @@
 //   3  the sums through the element's place in LDS back to the lanes that
 //      hold lambda and the gradient, and out in whole lines.
 //
-// What bounds it: with the gradients, at N = 7, 600 MB of HBM traffic per
-// stage at 16^3 (101 us at the card's four-stream rate) and the latency of
-// three dependent rounds of loads with three workgroups on a CU; without
-// them, the bytes.  Whole-line stores from the lanes that loaded, tangential
+// What bounds it: HBM.  With the gradients at N = 7, 16^3, a stage moves 0.90
+// GB (151 us at the card's four-stream rate) for 0.67 GB of algorithmic
+// bytes: the x-face reads of the stage state touch one node per 64-byte row
+// and so every line of the element and of its x-neighbours.  Whole-line stores from the lanes that loaded, tangential
 // traces, a split of the levels as the stage's and equal-work ranges under a
 // Drude region took, per stage with the gradients, N = 4 (28^3) 469 -> 350
 // us, N = 5 (24^3) 364 -> 285, N = 6 (20^3) 304 -> 260, N = 7 (16^3) 190 ->
