@@ -78,14 +78,6 @@ __global__ void invert_pair(double *__restrict__ a, double *__restrict__ b, int6
     }
 }
 
-// Admittance/impedance pairs for the adjoint's material gradient, from the
-// inverse-material tables the stage kernel reads.
-__global__ void admittance_pairs(const double *__restrict__ ieps, const double *__restrict__ imu, int64_t n,
-                                 double *__restrict__ yz) {
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x)
-        reinterpret_cast<double2 *>(yz)[p] = make_double2(sqrt(imu[p] / ieps[p]), sqrt(ieps[p] / imu[p]));
-}
-
 // The six fields at n listed nodes, out[6][n].
 __global__ void gather_nodes(const double *__restrict__ u, int64_t fs, const int64_t *__restrict__ node, int64_t n,
                              double *__restrict__ out) {

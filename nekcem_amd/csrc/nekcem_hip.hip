@@ -648,8 +648,6 @@ struct nkc_handle {
     // host copy of the element tables (material updates, adjoint)
     HostMesh hm;
     double C0 = 1.0;
-    double *yz = nullptr;                 // (sqrt(eps/mu), sqrt(mu/eps)) per ieps entry, adjoint only
-    bool yz_ok = false;                   // formed from the present materials
     bool hm_stale = false;                // hm.ieps/imu are older than the device's tables
     double *list = nullptr;               // node_list: room for `listed` nodes and their values
     int64_t listed = 0;
@@ -886,21 +884,6 @@ dim3 item_grid(int64_t n, int rows = 1) {
     return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(2048, (n + 255) / 256)), rows);
 }
 
-// Entries of the handle's material tables: per node or per element.
-int64_t material_entries(const nkc_handle *h) { return h->m.mat == MAT_NODE ? h->m.npts : h->m.nelt; }
-
-int32_t ensure_yz(nkc_handle *h) {
-    if (h->yz_ok) return NKC_OK;
-    const int64_t n = material_entries(h);
-    int32_t rc;
-    if (!h->yz && (rc = dev_alloc(&h->yz, 2 * n))) return rc;
-    hipLaunchKernelGGL(admittance_pairs, item_grid(n), dim3(256), 0, h->stream, (const double *)h->m.ieps,
-                       (const double *)h->m.imu, n, h->yz);
-    HIPCHK(hipGetLastError());
-    h->yz_ok = true;
-    return NKC_OK;
-}
-
 // The inverse materials on the host, for the set-up of a PML or a sheet;
 // nkc_set_materials leaves them on the device.
 int32_t host_materials(nkc_handle *h) {
@@ -943,8 +926,6 @@ int32_t node_list(nkc_handle *h, int64_t n, const int64_t *nodes, int64_t **dn, 
 
 void free_handle(nkc_handle *h) {
     free_adjoint(h);
-    (void)hipFree(h->yz);
-    h->yz = nullptr;
     (void)hipFree(h->list);
     h->list = nullptr;
     dev_mesh_free(h->m);
@@ -2298,12 +2279,9 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps, const double *mu) {
     hipLaunchKernelGGL(invert_pair, item_grid(npts), dim3(256), 0, h->stream, ieps, imu, npts);
     HIPCHK(hipGetLastError());
     if (m.mat != MAT_NODE) {
-        (void)hipFree(h->yz);              // one pair per element
-        h->yz = nullptr;
         (void)hipFree(m.fco);
         m.fco = fco;
     }
-    h->yz_ok = false;
     (void)hipFree(m.ieps); (void)hipFree(m.imu);
     m.ieps = ieps;
     m.imu = imu;
@@ -2524,7 +2502,6 @@ int32_t reverse_window(nkc_handle *h, int64_t seg, int64_t q, int &li) {
             a.rkb = RK4B[st];
             a.dt = A.dt;
             a.C0 = h->C0;
-            a.yz = h->yz;
             if (h->ndrude) {
                 a.drude_off = h->drude_off;
                 a.dpar = h->dpar;
@@ -2644,7 +2621,6 @@ int32_t backward_sweep(nkc_handle *h, const std::function<int32_t()> &seed, doub
     const size_t blk = 6 * (size_t)m.fs, jsz = drude_size(h);
     const double t_end = h->t_host;
     int32_t rc;
-    if ((rc = ensure_yz(h))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     HIPCHK(hipMemset(A.lam[0], 0, sizeof(double) * blk));
     HIPCHK(hipMemset(A.kap[0], 0, sizeof(double) * blk));
@@ -2771,7 +2747,6 @@ int32_t nkc_adjoint_apply(nkc_handle *h, const double *kH, const double *kE, dou
     double *zero = nullptr, *kap = nullptr, *out = nullptr, *kout = nullptr, *g = nullptr;
     int32_t rc = NKC_OK;
     do {
-        if ((rc = ensure_yz(h))) break;
         if ((rc = dev_alloc(&zero, blk)) || (rc = dev_alloc(&kap, blk)) || (rc = dev_alloc(&out, blk)) ||
             (rc = dev_alloc(&kout, blk)) || (rc = dev_alloc(&g, 2 * m.fs)))
             break;
@@ -2794,7 +2769,6 @@ int32_t nkc_adjoint_apply(nkc_handle *h, const double *kH, const double *kE, dou
         a.rkb = 0.0;
         a.dt = 1.0;
         a.C0 = h->C0;
-        a.yz = h->yz;
         if ((rc = launch_adjoint(m, a, h->stream))) break;
         if (hipStreamSynchronize(h->stream) != hipSuccess) { rc = fail(NKC_ERR_HIP, "sync"); break; }
         rc = copy_fields_d2h(out, m.fs, 0, aH, aE, m.npts, ld);
