@@ -627,7 +627,9 @@ box_kernel(StageArgs a) {
         // cem_maxwell_drude: resJ = -a J + b E; cem_maxwell_lorentz: resJ =
         // -a J - b P + c E, resP = J; the RK update from the stage-start E
         // (still in LDS), in the order of memory: every load of an element
-        // at once instead of a round trip per level.  Each node by one lane.
+        // at once instead of a round trip per level.  Each node by one lane,
+        // once every wave has read the currents its levels take
+        if ((a.drude_off && a.drude_off[e] >= 0) || (a.lor_off && a.lor_off[e] >= 0)) __syncthreads();
         constexpr int NLX = SL > 1 ? ((NX + 63) / 64 + WG - 1) / WG : S::NLD;
         auto place = [&](int v) {
             if (SL > 1) return S::idx(v % N1, v / N1 % N1, v / N2);
