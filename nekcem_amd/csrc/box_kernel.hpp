@@ -286,11 +286,15 @@ box_kernel(StageArgs a) {
     // this lane's nodes: RK register, inverse materials, source amplitude
     const unsigned node0 = 8u * (unsigned)(k0 * N2 + q);
     auto run_has = [&](int kk) { return REM == 0 || kk < kn; };   // a short run skips its last slot
-    // KLATE: the RK register a level ahead instead of up front, in the
-    // instances whose 128 VGPRs it would overflow (source at N = 8, 22^3:
-    // 351 -> 310 us; at N = 9 the up-front loads are the faster ones, 24^3:
-    // 535 against 554)
-    constexpr bool KLATE = (N1 >= 7 && FEAT >= 2) || (N1 == 9 && FEAT == 1);
+    // KLATE: the RK register level by level instead of up front, in the
+    // instances whose 128 VGPRs it would overflow: a level ahead with a source
+    // or a dispersive region at N = 8 (22^3: 351 -> 310 us; at N = 9 the
+    // up-front loads are the faster ones, 24^3: 535 against 554), at the level
+    // (KHERE) with a PML or an incident wave, where the level ahead would spill
+    // (PML, N = 6 at 24^3 297 -> 264 us, N = 8 at 20^3 327 -> 318, N = 9 at 16^3
+    // 328 -> 300)
+    constexpr bool KHERE = FEAT >= 2 && N1 >= 7;
+    constexpr bool KLATE = KHERE || (N1 == 9 && FEAT == 1);
     double kp[3][KLATE ? 1 : KL];
     const bool rdk = RK && (a.kflags & 1);
     const double *kb = a.kbuf + 3 * grp * fs + eo;
@@ -298,7 +302,7 @@ box_kernel(StageArgs a) {
     for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int kk = 0; kk < (KLATE ? 1 : KL); ++kk) kp[c][kk] = 0.0;
-    if (rdk) {
+    if (rdk && !KHERE) {
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -544,10 +548,32 @@ box_kernel(StageArgs a) {
         if (!run_has(kk)) break;
         const int k = k0 + kk;
         const unsigned vloc = (unsigned)(k * N2 + q);
+        if (KHERE && rdk) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) kp[c][0] = ld_stream<NTK>(at(kb + c * fs, node0, 8 * kk * N2));
+        }
         const double ko[3] = {kp[0][KLATE ? 0 : kk], kp[1][KLATE ? 0 : kk], kp[2][KLATE ? 0 : kk]};
-        if (KLATE && rdk && kk + 1 < kn) {
+        if (KLATE && !KHERE && rdk && kk + 1 < kn) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) kp[c][0] = ld_stream<NTK>(at(kb + c * fs, node0, 8 * (kk + 1) * N2));
+        }
+        [[maybe_unused]] double pl[3], pk[3], sig[3];
+        auto load_aux = [&] {
+            const double *sb = a.psig + (int64_t)po * 3 * N3, *pb = a.pP + (int64_t)po * 6 * N3 + 3 * grp * N3;
+            const double *qb = a.pkP + (int64_t)po * 6 * N3 + 3 * grp * N3;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                sig[c] = *at(sb, node0, 8 * (c * N3 + kk * N2));
+                pl[c] = *at(pb, node0, 8 * (c * N3 + kk * N2));
+                pk[c] = RK ? *at(qb, node0, 8 * (c * N3 + kk * N2)) : 0.0;
+            }
+        };
+        // requested before the level's derivatives where the registers hold
+        // them (PML, N = 5 at 20^3 107 -> 102 us, N = 7 at 16^3 110 -> 108; at N =
+        // 8 they spill, 12^3 69 -> 81)
+        constexpr bool PEARLY = FEAT >= 2 && (N1 == 6 || N1 == 8);
+        if constexpr (PEARLY) {
+            if (po >= 0) load_aux();
         }
         double S1_r = 0, S2_r = 0, S0_s = 0, S2_s = 0;
 #pragma unroll
@@ -570,22 +596,22 @@ box_kernel(StageArgs a) {
             // next and last axis, the auxiliary field P (B for H, D for E)
             //   resP = res - sb P,  res += (sa - sb) P - sd mu H  (H)
             //                       res += (sa - sb) P - sigma_d E (E)
-            const int64_t sb = (int64_t)po * 3 * N3 + vloc, pb = (int64_t)po * 6 * N3 + 3 * grp * N3 + vloc;
-            const double sig[3] = {a.psig[sb], a.psig[sb + N3], a.psig[sb + 2 * N3]};
+            if constexpr (!PEARLY) load_aux();
+            const int64_t pb = (int64_t)po * 6 * N3 + 3 * grp * N3 + vloc;
             const double iep = grp ? mi : (MAT == MAT_NODE) ? (a.ieps + eo)[vloc] : a.ieps[e];
             const double mu = grp ? 0.0 : 1.0 / mi;
             const double sp[3] = {sig[0] * iep, sig[1] * iep, sig[2] * iep};
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const int cb = (c + 1) % 3, cd = (c + 2) % 3;
-                const double P = a.pP[pb + c * N3];
+                const double P = pl[c];
                 const double rP = r[c] - sp[cb] * P;
                 const double drive = grp ? sig[cd] * uo[c * N3] : sp[cd] * mu * uo[c * N3];
                 r[c] += -sp[cb] * P + sp[c] * P - drive;
                 if (!RK) {
                     a.presP[pb + c * N3] = rP;
                 } else {
-                    const double kq = a.rka * a.pkP[pb + c * N3] + dt * rP;
+                    const double kq = a.rka * pk[c] + dt * rP;
                     a.pkP[pb + c * N3] = kq;
                     a.pP[pb + c * N3] = P + a.rkb * kq;
                 }
