@@ -27,8 +27,8 @@
 //   3  the sums through the element's place in LDS back to the lanes that
 //      hold lambda and the gradient, and out in whole lines.
 //
-// What bounds it: HBM.  With the gradients at N = 7, 16^3, a stage moves 0.90
-// GB (151 us at the card's four-stream rate) for 0.67 GB of algorithmic
+// What bounds it: HBM.  With the gradients at N = 7, 16^3, a stage moves 0.83
+// GB (140 us at the card's four-stream rate) for 0.67 GB of algorithmic
 // bytes: the x-face reads of the stage state touch one node per 64-byte row
 // and so every line of the element and of its x-neighbours.  Whole-line stores from the lanes that loaded, tangential
 // traces, a split of the levels as the stage's and equal-work ranges under a
@@ -372,8 +372,8 @@ adjoint_kernel(AdjArgs a) {
         const double vo[4] = {s1[0], s2[0], s1[3 * N3], s2[3 * N3]};
         double adj[4], dq = 0.0;
         // admittance and impedance of both sides from 1/mu and 1/eps (a table
-        // of the pairs read here cost 40 MB of a stage's 0.9 GB at 16^3, N =
-        // 7: 172-182 us against 162-169)
+        // of the pairs read here: 0.90 GB a stage at 16^3, N = 7, instead of
+        // 0.83, 172-182 us against 162-169)
         const double Yo = sqrt(fm[n][0] / fm[n][1]), Zo = sqrt(fm[n][1] / fm[n][0]);
         const double Yn = sqrt(fi[n][0] / fi[n][1]), Zn = sqrt(fi[n][1] / fi[n][0]);
         adj_face<GM>(f & 1 ? 1.0 : -1.0, ftype[n], vo, vn[n], fd[n], fL[n][0], fL[n][1], a.C0, Yo, Zo, Yn, Zn, adj, dq);
