@@ -209,6 +209,7 @@ adjoint_kernel(AdjArgs a) {
     }
     const int j = q / N1, i = q - j * N1;
     constexpr int BASE = N1 / S::KS, REM = N1 % S::KS;
+    static_assert(S::PAD || REM == 0, "a short run's last slot would read a row of D past the table");
     const int k0 = part * BASE + (part < REM ? part : REM);
     const int kn = BASE + (part < REM ? 1 : 0);
     auto run_has = [&](int kk) { return REM == 0 || kk < kn; };

@@ -43,12 +43,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "level_runs.hpp"
 #include "stage_args.hpp"
 
 namespace nkc {
-
-// Runs a workgroup splits a group's levels into.
-constexpr int level_runs(int n1) { return n1 <= 5 ? n1 : (n1 % 3 == 0 ? 3 : 2); }
 
 // Launch shape and LDS layout for polynomial order N1 - 1.
 //   A group's levels are split into KS runs of (N+1)^2 lanes: padded to
@@ -459,7 +457,7 @@ box_kernel(StageArgs a) {
             const double v0 = S0[S::idx(i, j, l)], v1 = S1[S::idx(i, j, l)];
 #pragma unroll
             for (int kk = 0; kk < KL; ++kk) {
-                const double d = S::PAD ? bcast_lane(dk[S::PAD ? kk : 0], l) : s_D[k0 + kk + N1 * l];
+                const double d = S::PAD ? bcast_lane(dk[S::PAD ? kk : 0], l) : s_D[slot_level(N1, RUNS, k0, kn, kk) + N1 * l];
                 R0[kk] += d * v1;
                 R1[kk] += d * v0;
             }

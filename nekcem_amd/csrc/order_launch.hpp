@@ -19,12 +19,6 @@ namespace nkc {
 // addresses take a register each).
 constexpr int box_waves(int n1, int feat) { return n1 < 7 ? 0 : (n1 == 8 && feat >= 2) ? 3 : 4; }
 
-// Slab counts with an instance: those that shorten a lane's run of levels.
-constexpr int run_length(int n1, int sl) { return (n1 + level_runs(n1) * sl - 1) / (level_runs(n1) * sl); }
-constexpr bool slabs_built(int n1, int sl) {
-    return sl > 1 && level_runs(n1) * sl <= n1 && run_length(n1, sl) < run_length(n1, sl - 1);
-}
-
 // nt: k and the outputs past the caches (see stage_nt)
 #define NKC_DECL_ORDER(n)                                                                          \
     void launch_stage_n##n(const StageArgs &a, int mat, int mode, bool nt, int sl, int grid, hipStream_t s); \
