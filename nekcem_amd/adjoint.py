@@ -130,14 +130,28 @@ if torch is not None:
             E0 = torch.as_tensor(np.asarray(problem.E0), dtype=torch.float64, device=dev).reshape(3, n).contiguous()
             pr = torch.as_tensor(np.asarray(problem.probes), dtype=torch.long, device=dev)
             extra = {}
-            if pr.dim() == 1 and len(pr) and 0 <= int(pr.min()) and int(pr.max()) < n:
-                # each probe node once, and where it stands in that list
-                extra["nodes"], extra["which"] = torch.unique(pr, return_inverse=True)
             if isinstance(problem, DrudeProbeProblem):
                 extra["owner"] = torch.as_tensor(np.asarray(problem.owner), dtype=torch.long, device=dev)
                 extra["dindex"] = np.ascontiguousarray(np.asarray(problem.dindex) + 1, dtype=np.int32)
             problem._dev[key] = (H0, E0, pr, extra)
         return problem._dev[key]
+
+    def _probe_list(problem, dev):
+        """The probes as the library takes them, (list, each node once, where
+        each stands in that): contiguous copies on dev.  None for a list that
+        only torch's indexing rules cover.  On the host the problem's tensor
+        may be the caller's own array, strided and open to edits, so the
+        copies are made afresh there; a device's are made once."""
+        _, _, pr, extra = _problem_tensors(problem, dev)
+        if "list" not in extra:
+            made = None
+            if pr.dim() == 1 and len(pr) and 0 <= int(pr.min()) and int(pr.max()) < problem.solver.npts:
+                own = pr.clone(memory_format=torch.contiguous_format)
+                made = (own, *torch.unique(own, return_inverse=True))
+            if not pr.is_cuda:
+                return made
+            extra["list"] = made
+        return extra["list"]
 
     def _start(problem, dev):
         """Time and state to the problem's start (device to device)."""
@@ -152,13 +166,15 @@ if torch is not None:
         tensor on dev, gathered on the device."""
         s = problem.solver
         n = s.npts
-        _, _, pr, extra = _problem_tensors(problem, dev)
-        if "nodes" in extra:
-            out = torch.empty((6, len(pr)), dtype=torch.float64, device=dev)
+        listed = _probe_list(problem, dev)
+        if listed is not None:
+            nodes = listed[0]           # held until the call has read it
+            out = torch.empty((6, len(nodes)), dtype=torch.float64, device=dev)
             _ready(out)
-            _lib.check(s._L.nkc_get_state_at(s._h, len(pr), _iptr(pr.contiguous()), _ptr(out)))
+            _lib.check(s._L.nkc_get_state_at(s._h, len(nodes), _iptr(nodes), _ptr(out)))
             return out
         # torch's own indexing rules for every other list of probes
+        pr = _problem_tensors(problem, dev)[2]
         H = torch.empty((3, n), dtype=torch.float64, device=dev)
         E = torch.empty((3, n), dtype=torch.float64, device=dev)
         _ready(H)
@@ -171,16 +187,17 @@ if torch is not None:
         s = problem.solver
         n = s.npts
         dev = grad_out.device
-        _, _, pr, extra = _problem_tensors(problem, dev)
         g = grad_out.detach().to(torch.float64)
         ge = torch.empty(n, dtype=torch.float64, device=dev) if want_material else None
         gm = torch.empty(n, dtype=torch.float64, device=dev) if want_material else None
-        if "nodes" in extra:
-            nodes = extra["nodes"]
-            seeds = torch.zeros((6, len(nodes)), dtype=torch.float64, device=dev).index_add_(1, extra["which"], g)
+        listed = _probe_list(problem, dev)
+        if listed is not None:
+            _, nodes, which = listed
+            seeds = torch.zeros((6, len(nodes)), dtype=torch.float64, device=dev).index_add_(1, which, g)
             _ready(seeds)
             _lib.check(s._L.nkc_adjoint_backward_at(s._h, len(nodes), _iptr(nodes), _ptr(seeds), _ptr(ge), _ptr(gm)))
             return ge, gm
+        pr = _problem_tensors(problem, dev)[2]
         lamH = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[:3])
         lamE = torch.zeros((3, n), dtype=torch.float64, device=dev).index_add_(1, pr, g[3:])
         _ready(lamH)
