@@ -1016,30 +1016,36 @@ int32_t make_handle(const HostMesh &hm, double C0, nkc_handle **out) {
     return NKC_OK;
 }
 
-// Whether both arrays are memory of the current device.
-bool on_device(const double *p, const double *q) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    for (const double *x : {p, q}) {
-        hipPointerAttribute_t at{};
-        if (hipPointerGetAttributes(&at, x) != hipSuccess) {
-            (void)hipGetLastError();   // plain host memory
-            return false;
-        }
-        if (at.type != hipMemoryTypeDevice || at.device != dev) return false;
+// Whether x lies in memory of device dev and, for bytes > 0, that much of it.
+bool on_device(const void *x, int dev, size_t bytes) {
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base{};
+    size_t len = 0;
+    if (hipPointerGetAttributes(&at, x) != hipSuccess ||
+        (bytes && hipMemGetAddressRange(&base, &len, (hipDeviceptr_t)x) != hipSuccess)) {
+        (void)hipGetLastError();   // plain host memory
+        return false;
     }
-    return true;
+    return at.type == hipMemoryTypeDevice && at.device == dev &&
+           bytes <= len - (size_t)((const char *)x - (const char *)base);
 }
 
 // Copy 6 fields between the caller's arrays (3 + 3 components at stride ld,
 // in host or device memory) and the library's device blocks.  Device arrays
 // go in one launch on the null stream, where it follows the caller's work as
-// a hipMemcpy would; anything else by hipMemcpyDefault.  A copy between
-// device arrays, like a memset, returns before it is done, and the handle's
-// stream does not wait for the null stream: finished here.
+// a hipMemcpy would, if a kernel of the current device reaches all of both
+// sides; anything else, arrays on another device or too short for their
+// stride among them, goes to hipMemcpyDefault, which copies between devices
+// and refuses what leaves an allocation.  A copy between device arrays, like
+// a memset, returns before it is done, and the handle's stream does not wait
+// for the null stream: finished here.
 template <bool IN>
 int32_t copy_fields(double *blk, int64_t fs, double *hn, double *en, int64_t n, int64_t ld) {
-    if (on_device(hn, en)) {
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    const bool fits = ld < INT64_MAX / 32;
+    const size_t span = fits ? sizeof(double) * (size_t)(2 * ld + n) : 0;
+    if (fits && on_device(blk, dev, 0) && on_device(hn, dev, span) && on_device(en, dev, span)) {
         const int nb = (int)std::min<int64_t>(2048, (n + 255) / 256);
         hipLaunchKernelGGL(copy_fields_kernel<IN>, dim3(nb, 6), dim3(256), 0, nullptr, hn, en, ld, blk, fs, n);
         HIPCHK(hipGetLastError());
