@@ -130,9 +130,10 @@ int32_t nkc_get_state(nkc_handle *h, double *hn, double *en, double *khn,
 int32_t nkc_get_state_at(nkc_handle *h, int64_t n, const int64_t *nodes, double *out);
 
 /* nsteps calls of cem_maxwell_op_rk (src/cem_maxwell.F:327-345): 5-stage
- * low-storage RK per step, each stage one fused kernel.  *time += nsteps*dt (time_advancing_pde,
- * src/cem_drive.F:639).  Asynchronous on the handle's stream; the next
- * get_state or nkc_sync waits for it. */
+ * low-storage RK per step, each stage one fused kernel.  *time += nsteps*dt
+ * (time_advancing_pde, src/cem_drive.F:639); after a failed launch *time and
+ * the state are those of the steps queued whole.  Asynchronous on the handle's
+ * stream; the next get_state or nkc_sync waits for it. */
 int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps);
 
 /* The RK register khn/ken as rk4_upd leaves it (src/cem_common.F:18-76).

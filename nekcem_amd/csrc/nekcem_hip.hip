@@ -1172,11 +1172,13 @@ namespace {
 int32_t queue_batch(nkc_batch *b, int64_t nsteps) {
     HIPCHK(hipEventRecord(b->ev[0], b->main));
     for (hipStream_t s : b->streams) HIPCHK(hipStreamWaitEvent(s, b->ev[0], 0));
-    for (int64_t step = 0; step < nsteps; ++step)
-        for (size_t l = 0; l < b->lanes.size(); ++l)
-            for (int bin : b->lanes[l]) {
-                const DevMesh &dm = b->bins[bin];
-                for (int s = 0; s < 5; ++s) {
+    int32_t rc = NKC_OK;
+    int64_t step = 0;
+    for (; step < nsteps && !rc; ++step)
+        for (size_t l = 0; l < b->lanes.size() && !rc; ++l)
+            for (size_t i = 0; i < b->lanes[l].size() && !rc; ++i) {
+                const DevMesh &dm = b->bins[b->lanes[l][i]];
+                for (int s = 0; s < 5 && !rc; ++s) {
                     StageArgs a = mesh_args(dm);
                     const int src = (b->cur + (int)(step & 1) + s) & 1;
                     a.uin = dm.u[src];
@@ -1186,16 +1188,19 @@ int32_t queue_batch(nkc_batch *b, int64_t nsteps) {
                     a.kflags = stage_kflags(s);
                     a.rkb = RK4B[s];
                     a.dt = 0.0;              // per element from dt_e
-                    const int32_t rc = launch_stage(dm, a, MODE_RK, b->streams[l]);
-                    if (rc) return rc;
+                    rc = launch_stage(dm, a, MODE_RK, b->streams[l]);
                 }
             }
-    for (size_t l = 0; l < b->streams.size(); ++l) {
-        HIPCHK(hipEventRecord(b->ev[1 + l], b->streams[l]));
-        HIPCHK(hipStreamWaitEvent(b->main, b->ev[1 + l], 0));
-    }
-    b->cur = (b->cur + (int)(nsteps & 1)) & 1;
-    return NKC_OK;
+    // after a launch that failed too: what is queued by then is ordered before
+    // whatever follows on the batch's stream
+    if (rc) --step;
+    for (size_t l = 0; l < b->streams.size(); ++l)
+        if ((hipEventRecord(b->ev[1 + l], b->streams[l]) != hipSuccess ||
+             hipStreamWaitEvent(b->main, b->ev[1 + l], 0) != hipSuccess) &&
+            hipStreamSynchronize(b->streams[l]) != hipSuccess && !rc)
+            rc = fail(NKC_ERR_HIP, "join of the batch's streams: %s", hipGetErrorString(hipGetLastError()));
+    b->cur = (b->cur + (int)(step & 1)) & 1;
+    return rc;
 }
 
 // The bins' streams: largest first, each to the stream with the least work.
@@ -1363,14 +1368,18 @@ int32_t nkc_step(nkc_handle *h, double *time, double dt, int64_t nsteps) {
     if (rt) return rt;
     // direct launches: a captured step replayed took 3 us longer at every size
     // (4^3: N = 5 28.0 / 24.5 us, N = 7 41.4 / 38.3; 3^3, N = 9 60.8 / 57.5)
+    int32_t rc = NKC_OK;
     for (int64_t s = 0; s < nsteps; ++s) {
-        const int32_t rc = queue_step(h, h->cur, dt);
-        if (rc) return rc;
+        rc = queue_step(h, h->cur, dt);
+        if (rc) {
+            h->tdev_ok = false;     // the device's time may be a step ahead
+            break;
+        }
         h->cur ^= 1;
+        time_passed(h, dt);         // same sums as the device
     }
-    for (int64_t s = 0; s < nsteps; ++s) time_passed(h, dt);   // same sums as the device
     if (time) *time = h->t_host;
-    return NKC_OK;
+    return rc;
 }
 
 int32_t nkc_residual(nkc_handle *h, double rktime, double *reshn, double *resen, int64_t ld) {
@@ -2445,7 +2454,10 @@ int32_t store_window(nkc_handle *h, int64_t seg, int64_t q) {
     const int64_t n = win_steps(h, seg, q);
     if ((rc = current_time(h))) return rc;
     for (int64_t s = 0; s < n; ++s) {
-        if ((rc = queue_step_store(h, h->adj.dt, s))) return rc;
+        if ((rc = queue_step_store(h, h->adj.dt, s))) {
+            h->tdev_ok = false;     // the device's time may be a step ahead
+            return rc;
+        }
         time_passed(h, h->adj.dt);
     }
     h->adj.slot_id[h->adj.cur_slot] = seg * h->adj.nsub_max + q;

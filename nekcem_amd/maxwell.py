@@ -316,8 +316,9 @@ class MaxwellSolver:
 
     def step(self, dt, nsteps=1):
         t = C.c_double(self.time)
-        _lib.check(self._L.nkc_step(self._h, C.byref(t), float(dt), int(nsteps)))
-        self.time = t.value
+        rc = self._L.nkc_step(self._h, C.byref(t), float(dt), int(nsteps))
+        self.time = t.value        # of the steps queued whole, after a failure too
+        _lib.check(rc)
         self.istep += int(nsteps)
 
     def set_source(self, amp, direction=(0.0, 0.0, 1.0), t0=0.0, tw=1.0, omega=None, phase=0.0):
