@@ -305,16 +305,22 @@ int32_t nkc_adjoint_get_drude(nkc_handle *h, double *ga, double *gb);
  * nkc_adjoint_forward until nkc_adjoint_release, the next forward, a
  * set_* call or nkc_destroy; a cap (max_steps > 0) holds it to the
  * checkpoints plus one window of 5 max_steps stages.
- * Between a set_* call (materials, source, Drude region) or the next forward
- * and that handle's next nkc_adjoint_forward, at most a quarter of the
- * device's memory may wait allocated for reuse; nkc_adjoint_release and
- * nkc_destroy free it, and so does any allocation of this library that
- * would otherwise fail.
  * nkc_adjoint_info: out[5] = {every, segments, S, K, device bytes held}. */
 int32_t nkc_adjoint_set_store(nkc_handle *h, int64_t max_steps);
 /* Free everything the adjoint holds (checkpoints, stage store, adjoint
  * state, gradients); a backward sweep then needs a new forward. */
 int32_t nkc_adjoint_release(nkc_handle *h);
+/* keep = 1: from here to the next call with keep = 0 the buffers of a
+ * trajectory that nkc_set_materials, nkc_set_source(_time) or nkc_set_drude
+ * discards are not freed but wait for this handle's next nkc_adjoint_forward,
+ * which would otherwise allocate the same again (tens of GB, 50 to 400 ms).
+ * Put it around the set_* calls and the forward of a pass, with keep = 0 right
+ * after them: what still waits then is freed, so that no other allocator of
+ * the process runs short because of it.  At most a quarter of the device's
+ * memory waits; nkc_adjoint_release, nkc_destroy and any allocation of this
+ * library that would otherwise fail free it too.  0 (default): a discarded
+ * trajectory is freed at once. */
+int32_t nkc_adjoint_keep(nkc_handle *h, int32_t keep);
 /* material = 1 (default): the backward sweep returns dL/deps and dL/dmu; 0:
  * it skips them (zeros are returned), which drops the stage residual from
  * the store (half its size: larger windows) and from the adjoint stage;

@@ -62,10 +62,11 @@ def _run_forward(problem: ProbeProblem, eps: np.ndarray, mu: np.ndarray):
     """The probe fields for host arrays eps, mu (numpy; finite differences)."""
     s = problem.solver
     s.adjoint_set_grads(True)
-    s.set_materials(eps, mu)
-    s.time = problem.t0
-    s.set_state(problem.H0, problem.E0)
-    s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
+    with s.adjoint_buffers_kept():
+        s.set_materials(eps, mu)
+        s.time = problem.t0
+        s.set_state(problem.H0, problem.E0)
+        s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
     H, E = s.get_state()
     return np.concatenate([H[:, problem.probes], E[:, problem.probes]])
 
@@ -92,10 +93,11 @@ def _run_forward_drude(problem: DrudeProbeProblem, gamma: np.ndarray, wp: np.nda
     """The probe fields for host arrays gamma, wp (numpy; finite differences)."""
     s = problem.solver
     s.adjoint_set_grads(False)      # only the Drude gradients are asked for
-    s.set_drude(problem.dindex, gamma[problem.owner], (wp * wp)[problem.owner])
-    s.time = problem.t0
-    s.set_state(problem.H0, problem.E0)
-    s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
+    with s.adjoint_buffers_kept():
+        s.set_drude(problem.dindex, gamma[problem.owner], (wp * wp)[problem.owner])
+        s.time = problem.t0
+        s.set_state(problem.H0, problem.E0)
+        s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
     H, E = s.get_state()
     return np.concatenate([H[:, problem.probes], E[:, problem.probes]])
 
@@ -215,9 +217,10 @@ if torch is not None:
             m = mu.detach().to(device=dev, dtype=torch.float64).contiguous()
             s.adjoint_set_grads(True)
             _ready(e, m)
-            _lib.check(s._L.nkc_set_materials(s._h, _ptr(e), _ptr(m)))
-            _start(problem, dev)
-            s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
+            with s.adjoint_buffers_kept():
+                _lib.check(s._L.nkc_set_materials(s._h, _ptr(e), _ptr(m)))
+                _start(problem, dev)
+                s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
             ctx.problem = problem
             return _probe_fields(problem, dev)
 
@@ -242,11 +245,12 @@ if torch is not None:
             par = torch.stack([g[owner], (w * w)[owner]], dim=1).contiguous()   # (a, b) per listed node
             s.adjoint_set_grads(False)      # only the Drude gradients are asked for
             _ready(par)
-            _lib.check(s._L.nkc_set_drude(s._h, len(di), di.ctypes.data_as(C.POINTER(C.c_int32)), _ptr(par),
-                                          None, None))
-            s.ndrude = len(di)
-            _start(problem, dev)
-            s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
+            with s.adjoint_buffers_kept():
+                _lib.check(s._L.nkc_set_drude(s._h, len(di), di.ctypes.data_as(C.POINTER(C.c_int32)), _ptr(par),
+                                              None, None))
+                s.ndrude = len(di)
+                _start(problem, dev)
+                s.adjoint_forward(problem.dt, problem.nsteps, problem.every)
             ctx.problem = problem
             ctx.wp = w
             ctx.ne = g.shape[0]

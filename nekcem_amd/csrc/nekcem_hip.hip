@@ -78,12 +78,14 @@ bool supported_n1_general(int n1) { return n1 >= GEO_MIN_N1 && n1 <= GEO_MAX_N1;
 
 // Adjoint buffers between two passes.  An adjoint pass holds tens of GB and
 // every pass frees and allocates the same sizes: mapping 40 GB took 50 to
-// 400 ms, as much as the pass itself (16^3, N = 7, 40 steps).  When a set_*
-// call or the next forward drops a handle's adjoint, its buffers wait here
-// for that handle's next nkc_adjoint_forward, which takes those whose size
-// it needs and frees the rest.  At most a quarter of a device's memory
-// waits; nkc_adjoint_release and nkc_destroy give a handle's buffers back,
-// and an allocation that finds the device full takes back all of them.
+// 400 ms, as much as the pass itself (16^3, N = 7, 40 steps).  When the next
+// forward, or under nkc_adjoint_keep a set_* call, drops a handle's adjoint,
+// its buffers wait here for that handle's next nkc_adjoint_forward, which
+// takes those whose size it needs and frees the rest.  Nothing waits outside
+// those calls and that scope, so other allocators of the process find the
+// memory free; at most a quarter of a device's memory waits; the end of the
+// scope, nkc_adjoint_release and nkc_destroy give a handle's buffers back, and
+// an allocation that finds the device full takes back all of them.
 struct IdleBlock {
     const void *owner;
     int device;
@@ -651,6 +653,7 @@ struct nkc_handle {
     bool hm_stale = false;                // hm.ieps/imu are older than the device's tables
     double *list = nullptr;               // node_list: room for `listed` nodes and their values
     int64_t listed = 0;
+    bool adj_keep = false;                // nkc_adjoint_keep
     int64_t adj_store_cap = 0;            // cap on the adjoint's stage-store window (0: from free memory)
     int32_t adj_grads = 3;                // bit 0: eps/mu gradients, bit 1: Drude gradients
     double tune_us[NLAYOUT] = {NAN, NAN, NAN, NAN, NAN, NAN, NAN, NAN};   // tuner's stage times per layout
@@ -1440,7 +1443,7 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     if (!h) return fail(NKC_ERR_ARG, "null handle");
     if (h->m.general && (amp != nullptr)) return general_refuses(h, "a source");
     HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h, true);                 // the stored trajectory has the old source
+    free_adjoint(h, h->adj_keep);         // the stored trajectory has the old source
     h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->src_off); h->src_off = nullptr;
     (void)hipFree(h->src_amp); h->src_amp = nullptr;
@@ -1482,7 +1485,7 @@ int32_t nkc_set_source_time(nkc_handle *h, int32_t kind, double omega, double ph
     if (kind != 0 && kind != 1) return fail(NKC_ERR_ARG, "source time kind %d not 0 or 1", kind);
     if (!std::isfinite(omega) || !std::isfinite(phase)) return fail(NKC_ERR_ARG, "source omega/phase not finite");
     HIPCHK(hipStreamSynchronize(h->stream));
-    free_adjoint(h, true);                 // the stored trajectory has the old source
+    free_adjoint(h, h->adj_keep);         // the stored trajectory has the old source
     h->src_kind = kind;
     h->src_om = omega;
     h->src_ph = phase;
@@ -1513,7 +1516,7 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     (void)hipFree(h->dkJ); h->dkJ = nullptr;
     (void)hipFree(h->dpar); h->dpar = nullptr;
     (void)hipFree(h->dresJ); h->dresJ = nullptr;
-    free_adjoint(h, true);                 // the stored trajectory has the old region
+    free_adjoint(h, h->adj_keep);         // the stored trajectory has the old region
     h->m.layout = -1;                     // the step's kernel instance may change
     h->ndrude = 0;
     h->ndelem = 0;
@@ -2287,7 +2290,7 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps, const double *mu) {
         return give_all_back(fail(NKC_ERR_HIP, "material check"));
     const unsigned long long bad = *std::min_element(h->red, h->red + nb);
     if (bad != ~0ull) return give_all_back(bad_node((int64_t)bad));
-    free_adjoint(h, true);                 // the stored trajectory has the old materials
+    free_adjoint(h, h->adj_keep);         // the stored trajectory has the old materials
     const int64_t nface = m.nelt * 6 * m.n1 * m.n1;
     hipLaunchKernelGGL(face_coefs, item_grid(nface), dim3(256), 0, h->stream, (const double *)ieps,
                        (const double *)imu, (const int32_t *)m.nbr, m.n1, m.nelt, (int)HOST_FACE_PEC, h->C0, fco);
@@ -2328,11 +2331,11 @@ int32_t dev_alloc_counted(nkc_handle *h, double **p, size_t n) {
 }
 
 // Free device memory as the adjoint's layout counts it: what is free and
-// what waits for this handle.
+// what waits, for this handle or for another (an allocation takes that back).
 int32_t adjoint_room(const nkc_handle *h, size_t *fr) {
     size_t tot = 0;
     HIPCHK(hipMemGetInfo(fr, &tot));
-    *fr += idle_bytes(h, h->device);
+    *fr += idle_bytes(nullptr, h->device);
     return NKC_OK;
 }
 
@@ -2551,6 +2554,13 @@ int32_t nkc_adjoint_release(nkc_handle *h) {
     return NKC_OK;
 }
 
+int32_t nkc_adjoint_keep(nkc_handle *h, int32_t keep) {
+    if (!h) return fail(NKC_ERR_ARG, "null handle");
+    h->adj_keep = keep != 0;
+    if (!h->adj_keep) idle_drop([&](const IdleBlock &b) { return b.owner == h; });
+    return NKC_OK;
+}
+
 int32_t nkc_adjoint_set_grads(nkc_handle *h, int32_t material) {
     if (!h) return fail(NKC_ERR_ARG, "null handle");
     h->adj_grads = (material ? 1 : 0) | 2;
@@ -2564,7 +2574,7 @@ int32_t nkc_adjoint_info(nkc_handle *h, int64_t *out) {
     out[1] = A.nseg;
     out[2] = A.S;
     out[3] = A.K;
-    out[4] = (int64_t)A.bytes;
+    out[4] = (int64_t)(A.bytes + idle_bytes(h, h->device));
     return NKC_OK;
 }
 

@@ -22,6 +22,7 @@ operator.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 
 import numpy as np
@@ -575,6 +576,19 @@ class MaxwellSolver:
     def adjoint_release(self):
         """Free the adjoint's checkpoints, stage store and gradients."""
         _lib.check(self._L.nkc_adjoint_release(self._h))
+
+    @contextlib.contextmanager
+    def adjoint_buffers_kept(self):
+        """Around the set_* calls and the adjoint_forward of a pass: the
+        forward takes the buffers of the trajectory those calls discard
+        instead of freeing and allocating them; whatever it has not taken is
+        freed at the end."""
+        _lib.check(self._L.nkc_adjoint_keep(self._h, 1))
+        try:
+            yield
+        finally:
+            if self._h:          # not closed meanwhile
+                _lib.check(self._L.nkc_adjoint_keep(self._h, 0))
 
     def adjoint_set_grads(self, material=True):
         """Whether the backward sweep computes dL/deps, dL/dmu (default) or
