@@ -311,18 +311,28 @@ box_kernel(StageArgs a) {
     const double sgn = grp ? 1.0 : -1.0;
     const double gx = sgn * geo[0], gy = sgn * geo[1], gz = sgn * geo[2];
     const double dt = a.dt_e ? a.dt_e[e] : a.dt;
-    double minv[MAT == MAT_NODE ? KL : 1];
+    // N = 9 in whole elements, whose 8-wave workgroups live on 128 VGPRs with
+    // five levels a lane: what a level alone needs is loaded at the level
+    // instead of held from here (MHERE 1/m of per-node materials, SHERE the
+    // source's amplitude beside a PML, an incident wave or a sheet), and DRREG
+    // the row of D stays in LDS there.  Held, they spilled 20 to 84 B a lane: us
+    // per stage, per-node materials at 9.9e5 nodes 44.3 -> 40.1 (2.9e6: 131 ->
+    // 123), with a Drude region 55.0 -> 50.3, with a PML 89.8 -> 68.1 (per
+    // element 70.0 -> 62.7; 2.9e6: 218 -> 188).
+    constexpr bool MHERE = MAT == MAT_NODE && N1 == 10 && SL == 1;
+    double minv[MAT == MAT_NODE && !MHERE ? KL : 1];
     const double *mp = (grp ? a.ieps : a.imu) + eo;
     if (MAT == MAT_ELEM) {
         minv[0] = grp ? a.ieps[e] : a.imu[e];
-    } else {
+    } else if (!MHERE) {
 #pragma unroll
         for (int kk = 0; kk < KL; ++kk) minv[kk] = run_has(kk) ? *at(mp, node0, 8 * kk * N2) : 0.0;
     }
     const int so = (FEAT >= 1 && grp == 1 && a.src_off) ? a.src_off[e] : -1;
-    [[maybe_unused]] double samp[KL];
+    constexpr bool SHERE = FEAT >= 2 && N1 == 10 && SL == 1;
+    [[maybe_unused]] double samp[SHERE ? 1 : KL];
     [[maybe_unused]] const double *sp = a.src_amp + (int64_t)so * N3;
-    if constexpr (FEAT >= 1) {
+    if constexpr (FEAT >= 1 && !SHERE) {
 #pragma unroll
         for (int kk = 0; kk < KL; ++kk) samp[kk] = 0.0;
         if (so >= 0) {
@@ -508,7 +518,7 @@ box_kernel(StageArgs a) {
         if (FEAT == 1 && so >= 0) {
 #pragma unroll
             for (int kk = 0; kk < KL; ++kk) {
-                const double am = samp[kk] * sgt;
+                const double am = samp[SHERE ? 0 : kk] * sgt;
                 R0[kk] += am * a.src_dir[0];
                 R1[kk] += am * a.src_dir[1];
                 R2[kk] += am * a.src_dir[2];
@@ -534,9 +544,12 @@ box_kernel(StageArgs a) {
     // D rows of the lane's column; at N = 9 the s row stays in LDS (its 20
     // VGPRs would spill at two 8-wave workgroups per CU)
     constexpr bool DSREG = N1 < 9 || (N1 == 9 && FEAT <= 1);
-    double Dr[N1], Ds[DSREG ? N1 : 1];
+    constexpr bool DRREG = !(N1 == 10 && FEAT >= 2 && SL == 1);
+    double Dr[DRREG ? N1 : 1], Ds[DSREG ? N1 : 1];
+    if constexpr (DRREG) {
 #pragma unroll
-    for (int l = 0; l < N1; ++l) Dr[l] = s_D[i + N1 * l];
+        for (int l = 0; l < N1; ++l) Dr[l] = s_D[i + N1 * l];
+    }
     if constexpr (DSREG) {
 #pragma unroll
         for (int l = 0; l < N1; ++l) Ds[l] = s_D[j + N1 * l];
@@ -578,8 +591,9 @@ box_kernel(StageArgs a) {
         for (int l = 0; l < N1; ++l) {
             const int pr = S::idx(l, j, k), ps = S::idx(i, l, k);
             const double dsl = DSREG ? Ds[DSREG ? l : 0] : s_D[j + N1 * l];
-            S1_r += Dr[l] * S1[pr];
-            S2_r += Dr[l] * S2[pr];
+            const double drl = DRREG ? Dr[DRREG ? l : 0] : s_D[i + N1 * l];
+            S1_r += drl * S1[pr];
+            S2_r += drl * S2[pr];
             S0_s += dsl * S0[ps];
             S2_s += dsl * S2[ps];
         }
@@ -587,7 +601,7 @@ box_kernel(StageArgs a) {
         r[0] = R0[kk] + gy * S2_s;
         r[1] = R1[kk] - gx * S2_r;
         r[2] = R2[kk] + (gx * S1_r - gy * S0_s);
-        const double mi = minv[MAT == MAT_NODE ? kk : 0];
+        const double mi = MHERE ? *at(mp, node0, 8 * kk * N2) : minv[MAT == MAT_NODE && !MHERE ? kk : 0];
         [[maybe_unused]] const double *uo = own + S::idx(i, j, k);   // the group's own fields at this node
         if (FEAT >= 2 && po >= 0) {
             // pml_step: with sa, sb, sd = sigma/eps of the component's own,
@@ -617,7 +631,7 @@ box_kernel(StageArgs a) {
         }
         if (FEAT >= 2) {
             if (so >= 0) {
-                const double am = samp[kk] * sgt;
+                const double am = (SHERE ? *at(sp, node0, 8 * kk * N2) : samp[SHERE ? 0 : kk]) * sgt;
 #pragma unroll
                 for (int c = 0; c < 3; ++c) r[c] += am * a.src_dir[c];
             }
