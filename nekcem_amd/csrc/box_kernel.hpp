@@ -253,15 +253,34 @@ box_kernel(StageArgs a) {
         for (int n = 0; n < S::NLD; ++n) ld[c][n] = *at(ug + c * fs, ldo[n]);
     // neighbour traces (a wall reads the element itself, unused), flux
     // coefficients and lift factors of this wave's face chunks
-    double up[S::NF][4], cf[S::NF][4], fL[S::NF];
-    int fown[S::NF], ftype[S::NF];
-    [[maybe_unused]] int64_t fnb[S::NF];
-#pragma unroll
-    for (int n = 0; n < S::NF; ++n) {
+    // PACKF: face nodes back to back over the workgroup's lanes (96 of 128 at N
+    // = 3) instead of a face a wave pass (three passes of 16 of 64 lanes, with
+    // three sets of traces and coefficients held: 81 VGPRs against 63 with
+    // per-node materials; us per stage 3.1e6 nodes 154 -> 142, 1e7 510 -> 474;
+    // per element 1e7 396 -> 387, 1e5 7.3 -> 6.8).  From N = 4 on a face fills
+    // the better part of a wave and the face stays uniform across it.
+    // (An instance with a sheet keeps the uniform faces: 33 -> 38 us at 3.9e5.)
+    constexpr bool PACKF = N1 == 4 && FEAT <= 2;
+    constexpr int NF = PACKF ? 1 : S::NF;
+    // face and in-face node of the wave's chunk n
+    auto face_at = [&](int n, int &fq) {
+        if (PACKF) {
+            const int x = min(t, 6 * N2 - 1), f = x / N2;
+            fq = x - f * N2;
+            return f;
+        }
         const int id = min(w + 2 * WG * n, 6 * S::FC - 1), f = id / S::FC;
-        const int ax = f >> 1, side = f & 1;
-        int fq = (id - f * S::FC) * 64 + lane;
+        fq = (id - f * S::FC) * 64 + lane;
         if (N2 % 64 != 0) fq = min(fq, N2 - 1);
+        return f;
+    };
+    double up[NF][4], cf[NF][4], fL[NF];
+    int fown[NF], ftype[NF];
+    [[maybe_unused]] int64_t fnb[NF];
+#pragma unroll
+    for (int n = 0; n < NF; ++n) {
+        int fq;
+        const int f = face_at(n, fq), ax = f >> 1, side = f & 1;
         const int fb = fq / N1, fa = fq - fb * N1;
         ftype[n] = a.nbr[e * 6 + f];
         const int M = side ? N1 - 1 : 0;
@@ -363,12 +382,10 @@ box_kernel(StageArgs a) {
 
     // ---- phase 1: each wave takes whole faces (or halves of one) ----
 #pragma unroll
-    for (int n = 0; n < S::NF; ++n) {
-        const int id = w + 2 * WG * n, f = id / S::FC;
-        if (6 * S::FC % (2 * WG) != 0 && id >= 6 * S::FC) break;
-        const int ax = f >> 1, side = f & 1;
-        int fq = (id - f * S::FC) * 64 + lane;
-        if (N2 % 64 != 0) fq = min(fq, N2 - 1);
+    for (int n = 0; n < NF; ++n) {
+        if (PACKF ? 64 * w >= 6 * N2 : 6 * S::FC % (2 * WG) != 0 && w + 2 * WG * n >= 6 * S::FC) break;
+        int fq;
+        const int f = face_at(n, fq), ax = f >> 1, side = f & 1;
         const int t1 = pick3(ax, 1, 2, 0), t2 = pick3(ax, 2, 0, 1);
         const double *s1 = s_u + t1 * N3 + fown[n], *s2 = s_u + t2 * N3 + fown[n];
         double um[4] = {s1[0], s2[0], s1[3 * N3], s2[3 * N3]};
