@@ -259,8 +259,7 @@ box_kernel(StageArgs a) {
     // per-node materials; us per stage 3.1e6 nodes 154 -> 142, 1e7 510 -> 474;
     // per element 1e7 396 -> 387, 1e5 7.3 -> 6.8).  From N = 4 on a face fills
     // the better part of a wave and the face stays uniform across it.
-    // (An instance with a sheet keeps the uniform faces: 33 -> 38 us at 3.9e5.)
-    constexpr bool PACKF = N1 == 4 && FEAT <= 2;
+    constexpr bool PACKF = N1 == 4;
     constexpr int NF = PACKF ? 1 : S::NF;
     // face and in-face node of the wave's chunk n
     auto face_at = [&](int n, int &fq) {
@@ -277,6 +276,10 @@ box_kernel(StageArgs a) {
     double up[NF][4], cf[NF][4], fL[NF];
     int fown[NF], ftype[NF];
     [[maybe_unused]] int64_t fnb[NF];
+    // sheet blocks on the own and on the far side, asked for with the traces:
+    // at the flux they were another round trip of every element (N = 3, 3.1e6
+    // nodes 213 -> 204 us per stage)
+    [[maybe_unused]] int sho[NF], shn[NF];
 #pragma unroll
     for (int n = 0; n < NF; ++n) {
         int fq;
@@ -298,6 +301,10 @@ box_kernel(StageArgs a) {
         up[n][2] = *at(p1 + 3 * fs, 8u * (unsigned)opp);
         up[n][3] = *at(p2 + 3 * fs, 8u * (unsigned)opp);
         load_coef<N1, MAT>(a, e, f, fq, cf[n]);
+        if (FEAT == 3) {
+            sho[n] = a.gr_off ? a.gr_off[e * 6 + f] : -1;
+            shn[n] = a.gr_off && ftype[n] >= 0 ? a.gr_off[ftype[n] * 6 + (f ^ 1)] : -1;
+        }
         fL[n] = a.geo[(int64_t)e * 9 + 3 + f];
     }
     // this lane's nodes: RK register, inverse materials, source amplitude
@@ -435,12 +442,12 @@ box_kernel(StageArgs a) {
             // own side's state advances
             double g[3] = {0.0, 0.0, 0.0}, J[3];
             if (a.gr_off) {
-                const int b = a.gr_off[e * 6 + f];
+                const int b = sho[n];
                 if (b >= 0) {
                     sheet_current<N2>(a, b, fq, ax, t1, t2, sg, um, RK, dt, J);
                     g[0] -= J[0]; g[1] -= J[1]; g[2] -= J[2];
                 }
-                const int bn = ftype[n] >= 0 ? a.gr_off[ftype[n] * 6 + (f ^ 1)] : -1;
+                const int bn = shn[n];
                 if (bn >= 0) {
                     sheet_current<N2>(a, bn, fq, ax, t1, t2, -sg, up[n], false, dt, J);
                     g[0] -= J[0]; g[1] -= J[1]; g[2] -= J[2];

@@ -19,6 +19,7 @@
 #include <array>
 #include <functional>
 #include <mutex>
+#include <queue>
 
 #include "../../include/nekcem_hip.h"
 #include "adjoint_kernel.hpp"
@@ -272,6 +273,12 @@ constexpr double DRUDE_WORK = 1.6;
 // per stage: 358 us with equal counts, 339 at 1.4, 330 at 1.7, 324 at 2, 328
 // at 2.4; N = 7, 16^3: 118, 111, 114, 116, 118.
 constexpr double PML_WORK = 1.7;
+// What a sheet face adds to its element's stage (both sides' currents and the
+// own side's state at each face node), relative to a plain element's N + 1
+// levels; at N = 3 the other faces packed into the sheet's wave wait for it.
+// N = 3 at 9.9e5 nodes, one z plane, 4 / 6 / 10: 60.1 / 56.5 / 48.8 us per stage;
+// N = 4 at 1.0e6 52.6 / 49.8 / 52.4; N = 5 at 9.9e5 49.9 / 45.4 / 51.0.
+constexpr double sheet_work(int n1) { return (n1 == 4 ? 10.0 : 6.0) / n1; }
 
 // Whether a layout number names a kernel at this order.
 bool layout_built(int n1, int layout) {
@@ -829,6 +836,25 @@ int32_t queue_step(nkc_handle *h, int from, double dt) {
     return NKC_OK;
 }
 
+// The longest of the XCDs' times when each takes its elements in order, `slots`
+// workgroups at a time.
+double longest_xcd(const std::vector<double> &work, const std::vector<int32_t> &lo, int slots) {
+    double longest = 0.0;
+    for (int x = 0; x < 8; ++x) {
+        std::priority_queue<double, std::vector<double>, std::greater<double>> ends;
+        for (int32_t e = lo[x]; e < lo[x + 1]; ++e) {
+            double start = 0.0;
+            if ((int)ends.size() == slots) {
+                start = ends.top();
+                ends.pop();
+            }
+            ends.push(start + work[e]);
+            longest = std::max(longest, start + work[e]);
+        }
+    }
+    return longest;
+}
+
 // Element bounds of 8 contiguous ranges of equal work, one per XCD, when
 // Drude and PML elements cost more than the others (elements in order, so
 // each XCD still takes a compact run of the mesh).  A PML fills the first and
@@ -838,16 +864,25 @@ int32_t queue_step(nkc_handle *h, int from, double dt) {
 // N = 9 at 12^3 87.6 / 84.1).  Only when the chip's resident workgroups (16
 // waves a CU) do not hold the mesh at once: there a longer range is a second
 // round on its XCD (PML, N = 9 at 8^3, one round: 40 / 51; N = 7 at 8^3 20.6 /
-// 22.5; Drude, N = 9 at 8^3 30.9 / 31.8).
+// 22.5; Drude, N = 9 at 8^3 30.9 / 31.8).  A sheet across z is a plane or two
+// of the element order, all of it on one or two XCDs, and costs more than
+// twice a plain element at low orders: there the ranges are those whose longest
+// XCD, played through with the sheet instance's workgroups, is the shorter (equal
+// counts / chosen, one z plane: N = 3 at 3.9e5 nodes 33.3 / 29.0, 3.1e6 204 /
+// 154; N = 5 at 2.1e5 24.5 / 17.7, 3.0e6 169 / 143; N = 7 at 9.6e5 47.2 / 40.0;
+// N = 9 at 9.9e5 51.7 / 48.7, 2.9e6 154 / 138; slower only N = 8 at 1.8e5, 16.3 /
+// 17.4).
 void balance_xcds(nkc_handle *h) {
     h->m.xcd_lo.clear();
     const int64_t n = h->m.nelt;
-    if (h->drude_elems.empty() && h->pml_elems.empty()) return;
-    if (n * stage_block(h->m.n1) <= (int64_t)256 * 16 * 64) return;
+    const bool sheet = !h->gr_face.empty();
+    if (h->drude_elems.empty() && h->pml_elems.empty() && !sheet) return;
+    if (!sheet && n * stage_block(h->m.n1) <= (int64_t)256 * 16 * 64) return;
     std::vector<double> work(n, 1.0);
     double total = (double)n;
     for (int64_t e : h->drude_elems) { work[e] += DRUDE_WORK - 1.0; total += DRUDE_WORK - 1.0; }
     for (int64_t e : h->pml_elems) { work[e] += PML_WORK - 1.0; total += PML_WORK - 1.0; }
+    for (int64_t f : h->gr_face) { work[f / 6] += sheet_work(h->m.n1); total += sheet_work(h->m.n1); }
     std::vector<int32_t> lo(9, (int32_t)n);
     lo[0] = 0;
     double acc = 0.0;
@@ -855,6 +890,12 @@ void balance_xcds(nkc_handle *h) {
     for (int64_t e = 0; e < n && x < 8; ++e) {
         acc += work[e];
         while (x < 8 && acc >= total * x / 8.0) lo[x++] = (int32_t)(e + 1);
+    }
+    if (sheet) {
+        std::vector<int32_t> even(9);
+        for (int i = 0; i < 9; ++i) even[i] = (int32_t)std::min<int64_t>(n, (n + 7) / 8 * i);
+        const int slots = 32 * sheet_waves(h->m.n1) * 256 / stage_block(h->m.n1);
+        if (longest_xcd(work, even, slots) < longest_xcd(work, lo, slots)) return;
     }
     h->m.xcd_lo = lo;
 }
@@ -1967,6 +2008,7 @@ void free_sheet(nkc_handle *h) {
     (void)hipFree(h->gA[1]); h->gA[1] = nullptr;
     (void)hipFree(h->gK); h->gK = nullptr;
     h->gr_face.clear();
+    balance_xcds(h);
     h->gr_list.clear();
     h->ngraph = 0;
 }
@@ -2043,6 +2085,7 @@ int32_t nkc_set_graphene(nkc_handle *h, int64_t ngraph, const int32_t *graphinde
     }
     h->gr_list = std::move(list);
     h->ngraph = ngraph;
+    balance_xcds(h);
     return NKC_OK;
 }
 

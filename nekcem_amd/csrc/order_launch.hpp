@@ -19,6 +19,10 @@ namespace nkc {
 // addresses take a register each).
 constexpr int box_waves(int n1, int feat) { return n1 < 7 ? 0 : (n1 == 8 && feat >= 2) ? 3 : 4; }
 
+// Waves per SIMD of the instances with a sheet, as built: 129 and 152 VGPRs at
+// N = 5, 161 and 167 at N = 7, below 128 at the other orders.
+constexpr int sheet_waves(int n1) { return n1 == 6 || n1 == 8 ? 3 : 4; }
+
 // nt: k and the outputs past the caches (see stage_nt)
 #define NKC_DECL_ORDER(n)                                                                          \
     void launch_stage_n##n(const StageArgs &a, int mat, int mode, bool nt, int sl, int grid, hipStream_t s); \
