@@ -337,15 +337,16 @@ box_kernel(StageArgs a) {
     const double sgn = grp ? 1.0 : -1.0;
     const double gx = sgn * geo[0], gy = sgn * geo[1], gz = sgn * geo[2];
     const double dt = a.dt_e ? a.dt_e[e] : a.dt;
-    // N = 9 in whole elements, whose 8-wave workgroups live on 128 VGPRs with
-    // five levels a lane: what a level alone needs is loaded at the level
+    // N = 8 and 9 in whole elements, whose 8-wave workgroups live on 128 VGPRs
+    // with three and five levels a lane: what a level alone needs is loaded at the level
     // instead of held from here (MHERE 1/m of per-node materials, SHERE the
     // source's amplitude beside a PML, an incident wave or a sheet), and DRREG
     // the row of D stays in LDS there.  Held, they spilled 20 to 84 B a lane: us
     // per stage, per-node materials at 9.9e5 nodes 44.3 -> 40.1 (2.9e6: 131 ->
     // 123), with a Drude region 55.0 -> 50.3, with a PML 89.8 -> 68.1 (per
-    // element 70.0 -> 62.7; 2.9e6: 218 -> 188).
-    constexpr bool MHERE = MAT == MAT_NODE && N1 == 10 && SL == 1;
+    // element 70.0 -> 62.7; 2.9e6: 218 -> 188); N = 8 with a dispersive region and
+    // per-node materials, 28 B: 1.25e6 64.8 -> 57.5, 3.0e6 171 -> 156.
+    constexpr bool MHERE = MAT == MAT_NODE && (N1 == 10 || (N1 == 9 && FEAT == 1)) && SL == 1;
     double minv[MAT == MAT_NODE && !MHERE ? KL : 1];
     const double *mp = (grp ? a.ieps : a.imu) + eo;
     if (MAT == MAT_ELEM) {

@@ -1,8 +1,8 @@
-"""Scratch of the N = 9 stage instances, from the compiler's resource report
+"""Scratch of the N = 8 and 9 stage instances, from the compiler's resource report
 (nekcem_amd/build.py's flags, device code only; nothing is run).  Its 8-wave
 workgroups sit at 128 VGPRs, and what spilled there cost more than the kernel
 before had gained: per-node materials 44 us against 41 at 9.9e5 nodes, with a
-PML 90 against 68."""
+PML 90 against 68 (N = 9); with a dispersive region 65 against 62 (N = 8)."""
 import os
 import re
 import subprocess
@@ -12,19 +12,19 @@ import pytest
 from nekcem_amd import build as B
 
 
-def _report(tmp_path):
+def _report(tmp_path, n1):
     try:
         cc = B.hipcc()
     except RuntimeError:
         pytest.skip("needs hipcc")
     r = subprocess.run([cc] + B.HIPCC_FLAGS + ["-I", os.path.join(B.ROOT, "include"), "--cuda-device-only",
                                                "-Rpass-analysis=kernel-resource-usage", "-c", "-o",
-                                               str(tmp_path / "o"), os.path.join(B.CSRC, "order_n10.hip")],
+                                               str(tmp_path / "o"), os.path.join(B.CSRC, f"order_n{n1}.hip")],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
     out, key = {}, None
     for line in r.stderr.splitlines():
-        m = re.search(r"Function Name: _ZN3nkc10box_kernelILi10ELi(\d)ELi(\d)ELi(\d)ELb(\d)ELi4ELi(\d)E", line)
+        m = re.search(rf"Function Name: _ZN3nkc10box_kernelILi{n1}ELi(\d)ELi(\d)ELi(\d)ELb(\d)ELi4ELi(\d)E", line)
         if "Function Name:" in line:
             key = tuple(map(int, m.groups())) if m else None
         m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", line)
@@ -34,7 +34,7 @@ def _report(tmp_path):
 
 
 def test_scratch_at_n9(tmp_path):
-    scratch = _report(tmp_path)        # (materials, mode, features, non-temporal, slabs) -> bytes a lane
+    scratch = _report(tmp_path, 10)    # (materials, mode, features, non-temporal, slabs) -> bytes a lane
     assert len(scratch) >= 20
     for nt in (0, 1):
         assert scratch[1, 0, 0, nt, 1] == 0          # per-node materials
@@ -42,3 +42,12 @@ def test_scratch_at_n9(tmp_path):
         for mat in (0, 1):
             assert scratch[mat, 0, 2, nt, 1] <= 32   # with a PML or an incident wave
             assert scratch[mat, 0, 3, nt, 1] <= 32   # with a sheet
+
+
+def test_scratch_at_n8(tmp_path):
+    scratch = _report(tmp_path, 9)
+    assert len(scratch) >= 16
+    for mat in (0, 1):
+        for nt in (0, 1):
+            for feat in (0, 1, 2):
+                assert scratch[mat, 0, feat, nt, 1] == 0
