@@ -185,12 +185,26 @@ struct DevMesh {
 };
 
 // Whether a stage streams k and its outputs past the caches (non-temporal):
-// once u, k and the output no longer fit the 256 MB Infinity Cache together.
-// Per stage, plain / non-temporal: N = 5 at 18^3 (181 MB) 39.1 / 47.2 us, at
-// 25^3 (486 MB) 137.7 / 121.6; N = 7 at 12^3 (127 MB) 32.2 / 33.8, at 18^3
-// (430 MB) 109.4 / 103.4; N = 8 at 12^3 (181 MB) 45.2 / 49.9, at 16^3 (430
-// MB) 116.9 / 110.0.
-bool stage_nt(int64_t npts) { return 18.0 * sizeof(double) * (double)npts > 256.0 * 1024 * 1024; }
+// once what a stage touches no longer fits the 256 MB Infinity Cache together:
+// u, k and the output (18 doubles a node), with per-node materials the inverse
+// materials and four coefficients a face node, a source's amplitudes, and the
+// dispersive currents with their register and parameters.  Per stage, plain /
+// non-temporal: N = 5 at 18^3 (181 MB) 39.1 / 47.2 us, at 25^3 (486 MB) 137.7 /
+// 121.6; N = 7 at 12^3 (127 MB) 32.2 / 33.8, at 18^3 (430 MB) 109.4 / 103.4; N =
+// 8 at 12^3 (181 MB) 45.2 / 49.9, at 16^3 (430 MB) 116.9 / 110.0; per-node
+// materials, N = 3 at 233 MB 42.1 / 48.8, at 291 67.2 / 60.6; N = 7 at 257 48.9 /
+// 54.4, at 317 69.2 / 65.8; N = 8 at 227 47.2 / 52.0, at 289 71.4 / 67.0; source
+// and Drude region, N = 7 per node at 260 59 / 62, at 280 71 / 64, per element at
+// 234 51 / 59, at 275 70.7 / 68.2; Lorentz, N = 8 per node at 255 63 / 69, N = 9
+// at 294 87.9 / 80.6.  The PML's fields, which a part of the elements touch, do
+// not count: N = 8 at 12^3, 180 MB and 113 MB of them, 65 / 77.
+bool stage_nt(double doubles) { return sizeof(double) * doubles > 256.0 * 1024 * 1024; }
+
+// Doubles a stage touches of a mesh without regions or sources.  (General
+// meshes stream by the 18 alone: at N = 7 as geo_block's figures.)
+double mesh_doubles(const DevMesh &dm) {
+    return (double)dm.npts * (18.0 + (!dm.general && dm.mat == MAT_NODE ? 2.0 + 24.0 / dm.n1 : 0.0));
+}
 
 // Whether a reversed stage streams its outputs and the residual past the
 // caches: once lambda and kappa, in and out, and the stage's state (30 doubles
@@ -225,7 +239,8 @@ int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     dm.nelt = m.nelt;
     dm.npts = m.nelt * m.n1 * m.n1 * m.n1;
     dm.fs = (dm.npts + 31) / 32 * 32;
-    dm.nt = stage_nt(dm.npts);
+    dm.general = m.general;
+    dm.nt = stage_nt(mesh_doubles(dm));
     dm.jac = m.jac;
     dm.w = m.w;
     const size_t ub = sizeof(double) * 6 * (size_t)dm.fs;
@@ -242,7 +257,6 @@ int32_t dev_mesh_upload(const HostMesh &m, DevMesh &dm) {
     if ((rc = upload(&dm.fco, m.fco))) return rc;
     if ((rc = upload(&dm.ieps, m.ieps))) return rc;
     if ((rc = upload(&dm.imu, m.imu))) return rc;
-    dm.general = m.general;
     if (m.general) {
         if ((rc = upload(&dm.gmet, m.gmet))) return rc;
         if ((rc = upload(&dm.fgeo, m.fgeo))) return rc;
@@ -622,6 +636,7 @@ struct nkc_handle {
     double t_host = 0.0;
     // source
     int32_t *src_off = nullptr;
+    int64_t nsrc = 0;                     // elements with a source
     double *src_amp = nullptr;
     double src_dir[3] = {0, 0, 0}, src_t0 = 0, src_tw = 1;
     int32_t src_kind = 0;                 // 0 Gaussian pulse, 1 sin(src_om t + src_ph)
@@ -781,6 +796,13 @@ StageArgs base_args(nkc_handle *h) {
 // writes the register too, so khn/ken after a step are rk4_upd's.
 int32_t handle_kflags(const nkc_handle *h, int s) {
     return stage_kflags(s) | ((h->keep_k && s == 4) ? 2 : 0);
+}
+
+// Whether the handle's stages stream, after its materials, source or regions
+// changed.
+void set_streaming(nkc_handle *h) {
+    const double n3 = (double)h->m.n1 * h->m.n1 * h->m.n1;
+    h->m.nt = stage_nt(mesh_doubles(h->m) + n3 * ((double)h->nsrc + 8.0 * (double)h->ndelem + 15.0 * (double)h->nlelem));
 }
 
 // Whether the stages read the time.
@@ -1488,6 +1510,8 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     h->m.layout = -1;                     // the step's kernel instance may change
     (void)hipFree(h->src_off); h->src_off = nullptr;
     (void)hipFree(h->src_amp); h->src_amp = nullptr;
+    h->nsrc = 0;
+    set_streaming(h);
     int32_t rc = NKC_OK;
     if (!amp) return rc;
     if (!dir || !(tw != 0.0) || !std::isfinite(t0) || !std::isfinite(tw)) return fail(NKC_ERR_ARG, "bad source direction/time");
@@ -1514,6 +1538,8 @@ int32_t nkc_set_source(nkc_handle *h, const double *amp, const double dir[3], do
     // failed upload leaves the source off rather than half set
     if ((rc = upload(&h->src_amp, vals))) return rc;
     if ((rc = upload(&h->src_off, off))) return rc;
+    h->nsrc = (int64_t)(vals.size() / n3);
+    set_streaming(h);
     for (int c = 0; c < 3; ++c) h->src_dir[c] = dir[c];
     h->src_t0 = t0;
     h->src_tw = tw;
@@ -1564,6 +1590,7 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     h->drude_slot.clear();
     h->drude_elems.clear();
     balance_xcds(h);
+    set_streaming(h);
     int32_t rc = NKC_OK;
     if (ndrude == 0) return rc;
     if (ndrude < 0 || !dindex || !params) return fail(NKC_ERR_ARG, "bad Drude node list");
@@ -1600,6 +1627,7 @@ int32_t nkc_set_drude(nkc_handle *h, int64_t ndrude, const int32_t *dindex_in, c
     for (int64_t e = 0; e < m.nelt; ++e)
         if (off[e] >= 0) h->drude_elems.push_back(e);
     balance_xcds(h);
+    set_streaming(h);
     return NKC_OK;
 }
 
@@ -1784,6 +1812,7 @@ int32_t nkc_set_lorentz(nkc_handle *h, int64_t nlor, const int32_t *lindex, cons
     h->nlor = 0;
     h->nlelem = 0;
     h->lor_slot.clear();
+    set_streaming(h);
     int32_t rc = NKC_OK;
     if (nlor == 0) return rc;
     if (nlor < 0 || !lindex || !params) return fail(NKC_ERR_ARG, "bad Lorentz node list");
@@ -1816,6 +1845,7 @@ int32_t nkc_set_lorentz(nkc_handle *h, int64_t nlor, const int32_t *lindex, cons
     if ((rc = upload(&h->lor_off, off))) return rc;     // last: switches the term on
     h->nlor = nlor;
     h->nlelem = nle;
+    set_streaming(h);
     return NKC_OK;
 }
 
@@ -2349,6 +2379,7 @@ int32_t nkc_set_materials(nkc_handle *h, const double *eps, const double *mu) {
     m.mat = MAT_NODE;
     h->hm.mat = 1;
     h->hm_stale = true;
+    set_streaming(h);
     if (h->ngraph) {
         // the sheet's Yfac and yconduc follow the materials
         const size_t n2 = (size_t)m.n1 * m.n1;
@@ -2905,9 +2936,9 @@ int32_t nkc_batch_create(int32_t ncav, const nkc_box_desc *d, nkc_batch **out) {
         }
     }
     // the orders step side by side: one working set
-    int64_t npts = 0;
-    for (const auto &dm : b->bins) npts += dm.npts;
-    for (auto &dm : b->bins) dm.nt = stage_nt(npts);
+    double doubles = 0.0;
+    for (const auto &dm : b->bins) doubles += mesh_doubles(dm);
+    for (auto &dm : b->bins) dm.nt = stage_nt(doubles);
     if (!rc) {
         plan_streams(b);
         for (size_t l = 0; l < b->lanes.size(); ++l) {
