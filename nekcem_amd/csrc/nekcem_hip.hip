@@ -226,10 +226,16 @@ bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 25
 // (5), at 5^3 12.7 / 10.1 (2), at 6^3 13.6 / 14.5 (2); with a Drude region N =
 // 7 at 4^3 10.8 / 7.3, N = 9 at 4^3 17.3 / 11.1; with a PML N = 9 at 5^3 27.4 /
 // 16.9.  N = 7's 4-wave workgroups gain from two slabs up to two per CU: 6^3
-// 8.6 / 7.9, 8^3 12.5 / 12.1.
-int stage_slabs(int n1, int64_t nelt) {
+// 8.6 / 7.9, 8^3 12.5 / 12.1.  So do the two 8-wave ones of N = 9 with a
+// dispersive region, whose currents' update follows the levels: whole elements
+// of the 129 to 448 it helps were up to 7 per cent slower than the kernel before,
+// which had it in the levels (150 elements 18.0 / 16.7 in two / 14.5 in three,
+// 180 18.4 / 17.3 / 16.6, 200 19.2 / 18.5 / 17.5, 210 19.7 / 18.8 / 19.5, 252
+// 20.7 / 19.2 / 21.5, 392 27.1 / 25.8, 448 28.1 / 26.8, 504 28.8 / 32.6).
+int stage_slabs(int n1, int64_t nelt, bool dispersive) {
     for (int sl = 5; sl > 1; --sl)
         if (slabs_built(n1, sl) && nelt * sl <= 256) return sl;
+    if (n1 == 10 && dispersive) return nelt <= 200 ? 3 : nelt <= 448 ? 2 : 1;
     return n1 == 8 && nelt <= 512 ? 2 : 1;
 }
 
@@ -396,7 +402,7 @@ int32_t launch_stage(const DevMesh &dm, const StageArgs &a, int mode, hipStream_
     }
     const bool nt = a.st_r || a.st_J ? adjoint_nt(dm.npts) : dm.nt;
     const bool whole = mode != MODE_RK || nt || a.gr_off || a.st_r || a.st_J || b.xcd_bal;
-    const int sl = whole ? 1 : stage_slabs(dm.n1, dm.nelt);
+    const int sl = whole ? 1 : stage_slabs(dm.n1, dm.nelt, a.drude_off || a.lor_off);
     switch (dm.n1) {
     case 4: launch_stage_n4(b, dm.mat, mode, nt, sl, grid, s); break;
     case 5: launch_stage_n5(b, dm.mat, mode, nt, sl, grid, s); break;
