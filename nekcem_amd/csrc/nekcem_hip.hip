@@ -228,14 +228,16 @@ bool adjoint_nt(int64_t npts) { return 30.0 * sizeof(double) * (double)npts > 25
 // 16.9.  N = 7's 4-wave workgroups gain from two slabs up to two per CU: 6^3
 // 8.6 / 7.9, 8^3 12.5 / 12.1.  So do the two 8-wave ones of N = 9 with a
 // dispersive region, whose currents' update follows the levels: whole elements
-// of the 129 to 448 it helps were up to 7 per cent slower than the kernel before,
+// of the 129 to 352 it helps were up to 7 per cent slower than the kernel before,
 // which had it in the levels (150 elements 18.0 / 16.7 in two / 14.5 in three,
 // 180 18.4 / 17.3 / 16.6, 200 19.2 / 18.5 / 17.5, 210 19.7 / 18.8 / 19.5, 252
-// 20.7 / 19.2 / 21.5, 392 27.1 / 25.8, 448 28.1 / 26.8, 504 28.8 / 32.6).
+// 20.7 / 19.2 / 21.5; a driven cavity with its middle half a Drude region, per
+// step: 343 139 / 131 us, 392 as 7 7 8 143 / 139, as 8 7 7 144 / 156, 432 146 /
+// 161).
 int stage_slabs(int n1, int64_t nelt, bool dispersive) {
     for (int sl = 5; sl > 1; --sl)
         if (slabs_built(n1, sl) && nelt * sl <= 256) return sl;
-    if (n1 == 10 && dispersive) return nelt <= 200 ? 3 : nelt <= 448 ? 2 : 1;
+    if (n1 == 10 && dispersive) return nelt <= 200 ? 3 : nelt <= 352 ? 2 : 1;
     return n1 == 8 && nelt <= 512 ? 2 : 1;
 }
 

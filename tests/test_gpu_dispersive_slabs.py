@@ -8,6 +8,6 @@ from tests.test_gpu_stage_slabs import test_slabs_equal_whole_elements as _slabs
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("small", [(3, 1, 43), (5, 5, 8), (3, 1, 67), (8, 8, 7), (449, 1, 1)])
+@pytest.mark.parametrize("small", [(3, 1, 43), (5, 5, 8), (3, 1, 67), (8, 4, 11), (353, 1, 1)])
 def test_many_slabs_equal_whole_elements(small):
     _slabs_equal_whole_elements(9, small, "dispersive")

@@ -14,8 +14,8 @@ def slabs(s):
     sl = int(l.split("box_kernel<")[1].split(">")[0].split(", ")[6])
     assert int(l.split("grid ")[1].split()[0]) == sl * 8 * ((s.mesh.nelt + 7) // 8), l
     return sl
-for nelt, plain, dispersive in ((51, 5, 5), (85, 3, 3), (128, 2, 2), (129, 1, 3), (200, 1, 3), (201, 1, 2), (448, 1, 2),
-                                (449, 1, 1), (512, 1, 1)):
+for nelt, plain, dispersive in ((51, 5, 5), (85, 3, 3), (128, 2, 2), (129, 1, 3), (200, 1, 3), (201, 1, 2), (352, 1, 2),
+                                (353, 1, 1), (512, 1, 1)):
     s = MaxwellSolver.from_box((nelt, 1, 1), 9)
     assert slabs(s) == plain, nelt
     s.set_source(np.full(s.npts, 1e-3), (0, 0, 1.), 1.0, 0.5)
