@@ -18,23 +18,24 @@
 //   0  the element (64-node chunks), the tangential neighbour traces, the
 //      lane's RK register and per-node data: every load up front, one HBM
 //      round trip; the element into LDS;
-//   1  each wave forms the flux of whole faces (four tangential components;
-//      a face's flux has none along its normal) into LDS;
+//   1  each wave forms the flux of whole faces (at N = 3 of face nodes packed
+//      over the lanes) into LDS: four tangential components, a face's flux has
+//      none along its normal;
 //   2  t derivatives of all the lane's levels from one read of its column,
 //      lifts, then per level the r and s derivatives, physics, k update;
 //   3  k and then u back into the element's place in LDS and out in the
 //      order of memory, whole 128-byte lines.
 //
-// What bounds it: HBM, about 28.8 B per node and field (DESIGN keeps the
-// table); what used to cost more at every order but N = 7 is how the bytes
-// left: a level's (N+1)^2 doubles straddle cache lines, and a store that
-// covers part of a line costs about a whole one (the N = 7 kernel with its
-// arrays shifted by 8 bytes: 555 -> 719 us at 32^3; only the stores matter,
-// shifted element loads 547 -> 555).  Phase 3's line-aligned stores, the
-// 32-bit addressing and the single column read took, per stage, N = 3 (44^3)
-// 246 -> 222 us, N = 4 (40^3) 411 -> 345, N = 5 (36^3) 480 -> 378, N = 6
-// (32^3) 514 -> 424, N = 7 (32^3) 587 -> 555, N = 8 (22^3) 361 -> 281, N = 9
-// (24^3) 603 -> 507.
+// What bounds it: HBM, about 28.8 B per node and field; what used to cost
+// more at every order but N = 7 is how the bytes left: a level's (N+1)^2
+// doubles straddle cache lines, and a store that covers part of a line costs
+// about a whole one (the N = 7 kernel with its arrays shifted by 8 bytes: 555 -> 719 us at 32^3; only the stores matter,
+// shifted element loads 547 -> 555).  With phase 3's line-aligned stores, the
+// 32-bit addressing and the single column read a stage takes, against the
+// kernel before on the same card, N = 3 (44^3) 241 -> 208 us (per-node
+// materials 282 -> 256), N = 4 (40^3) 408 -> 343, N = 5 (36^3) 474 -> 378, N = 6
+// (32^3) 509 -> 412, N = 7 (32^3) 577 -> 544, N = 8 (22^3) 354 -> 279, N = 9
+// (24^3) 600 -> 507 (per-node materials, 20^3, 405 -> 346).
 //
 // Field order in HBM: 0 Hx, 1 Hy, 2 Hz, 3 Ex, 4 Ey, 5 Ez, each a contiguous
 // array of npts doubles at stride fs, volume index i + n1*j + n1^2*k +
@@ -315,8 +316,9 @@ box_kernel(StageArgs a) {
     // or a dispersive region at N = 8 (22^3: 351 -> 310 us; at N = 9 the
     // up-front loads are the faster ones, 24^3: 535 against 554), at the level
     // (KHERE) with a PML or an incident wave, where the level ahead would spill
-    // (PML, N = 6 at 24^3 297 -> 264 us, N = 8 at 20^3 327 -> 318, N = 9 at 16^3
-    // 328 -> 300)
+    // more (PML, N = 6 at 24^3 297 -> 264 us, N = 8 at 20^3 327 -> 318, N = 9 at
+    // 16^3 328 -> 300; what still spills: N = 6 12 B a lane, 44 with per-node
+    // materials, N = 9 28 and 20 B)
     constexpr bool KHERE = FEAT >= 2 && N1 >= 7;
     constexpr bool KLATE = KHERE || (N1 == 9 && FEAT == 1);
     double kp[3][KLATE ? 1 : KL];

@@ -23,8 +23,8 @@
 //      then the derivatives from LDS, the curl, the lifted fluxes of the
 //      faces the node lies on, inverse mass and the low-storage RK update.
 // Bound: on small meshes one workgroup's chain of phases (5 x 5 x 2 elements
-// at N = 11: 41 -> 13 us per stage), on large ones the bytes (10^3
-// elements at N = 7, in the Infinity Cache: 36 -> 32 us).
+// at N = 11: 41 -> 12.3 us per stage), on large ones the bytes (10^3
+// elements at N = 7, in the Infinity Cache: 36 -> 28 us).
 // Up to N = 11 (12^3 nodes: 125 KB of LDS, one workgroup per CU).  Materials
 // per node, flux coefficients per face node.
 #pragma once
@@ -59,9 +59,10 @@ struct GeoArgs {
     int32_t kflags;                    // bit 0 read k, bit 1 write k
 };
 
-// Lanes of a workgroup: 16 waves per CU at one (N = 11), two (N = 8..10) or
-// three to four workgroups per CU, what their LDS allows.  At N = 7 the three
-// 4-wave workgroups its LDS allows on a CU serve meshes whose stages stream
+// Lanes of a workgroup: 16 waves per CU at one (N = 11) or two (N = 8, 9)
+// workgroups per CU, 8 at N = 10, whose 100 KB of LDS leave one of 512 lanes,
+// and three to four workgroups of four waves below, what their LDS allows.  At
+// N = 7 the three 4-wave workgroups on a CU serve meshes whose stages stream
 // (nt), two of 8 waves with one face node a lane those in the caches: 6^3
 // 10.1 / 9.5 us, 8^3 18.4 / 16.7, 10^3 31.2 / 29.6, 12^3 48.4 / 47.2, 16^3
 // 134.9 / 141.5.
