@@ -29,9 +29,9 @@
 // What bounds it: HBM, about 28.8 B per node and field; what used to cost
 // more at every order but N = 7 is how the bytes left: a level's (N+1)^2
 // doubles straddle cache lines, and a store that covers part of a line costs
-// about a whole one (the N = 7 kernel with its arrays shifted by 8 bytes: 555 -> 719 us at 32^3; only the stores matter,
-// shifted element loads 547 -> 555).  With phase 3's line-aligned stores, the
-// 32-bit addressing and the single column read a stage takes, against the
+// about a whole one (the N = 7 kernel with its arrays shifted by 8 bytes: 555
+// -> 719 us at 32^3; only the stores matter, shifted element loads 547 -> 555).
+// With phase 3's line-aligned stores, the 32-bit addressing and the single column read a stage takes, against the
 // kernel before on the same card, N = 3 (44^3) 241 -> 208 us (per-node
 // materials 282 -> 256), N = 4 (40^3) 408 -> 343, N = 5 (36^3) 474 -> 378, N = 6
 // (32^3) 509 -> 412, N = 7 (32^3) 577 -> 544, N = 8 (22^3) 354 -> 279, N = 9
@@ -318,8 +318,14 @@ box_kernel(StageArgs a) {
     // (KHERE) with a PML or an incident wave, where the level ahead would spill
     // more (PML, N = 6 at 24^3 297 -> 264 us, N = 8 at 20^3 327 -> 318, N = 9 at
     // 16^3 328 -> 300; what still spills: N = 6 12 B a lane, 44 with per-node
-    // materials, N = 9 28 and 20 B)
-    constexpr bool KHERE = FEAT >= 2 && N1 >= 7;
+    // materials, N = 9 28 and 20 B), and in the stages kept for the adjoint at N =
+    // 7 and 9, whose stage residual's addresses come on top: up front they
+    // spilled 12 to 56 B and were up to 13 per cent slower than the kernel before
+    // (2e6 nodes, that kernel / up front / a level ahead / here: N = 7 per node
+    // 102 / 115 / 102 / 98, with a Drude region 108 / 116 / 94 / 93, N = 9 per node
+    // 156 / 146 / 132 / 126; 8e5: N = 9 per element with a Drude region 46.4 / 50.3
+    // / 43.3 / 42.0)
+    constexpr bool KHERE = (FEAT >= 2 && N1 >= 7) || (MODE == MODE_RK_STORE && (N1 == 8 || N1 == 10));
     constexpr bool KLATE = KHERE || (N1 == 9 && FEAT == 1);
     double kp[3][KLATE ? 1 : KL];
     const bool rdk = RK && (a.kflags & 1);

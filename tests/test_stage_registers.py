@@ -1,8 +1,9 @@
-"""Scratch of the N = 8 and 9 stage instances, from the compiler's resource report
-(nekcem_amd/build.py's flags, device code only; nothing is run).  Its 8-wave
-workgroups sit at 128 VGPRs, and what spilled there cost more than the kernel
+"""Scratch of the N = 7 to 9 stage instances, from the compiler's resource report
+(nekcem_amd/build.py's flags, device code only; nothing is run).  They
+sit at 128 VGPRs, and what spilled there cost more than the kernel
 before had gained: per-node materials 44 us against 41 at 9.9e5 nodes, with a
-PML 90 against 68 (N = 9); with a dispersive region 65 against 62 (N = 8)."""
+PML 90 against 68 (N = 9); with a dispersive region 65 against 62 (N = 8), the stages kept for the adjoint
+115 against 102 at 2e6 nodes (N = 7)."""
 import os
 import re
 import subprocess
@@ -42,6 +43,8 @@ def test_scratch_at_n9(tmp_path):
         for mat in (0, 1):
             assert scratch[mat, 0, 2, nt, 1] <= 32   # with a PML or an incident wave
             assert scratch[mat, 0, 3, nt, 1] <= 32   # with a sheet
+            assert scratch[mat, 2, 0, nt, 1] == 0    # kept for the adjoint
+            assert scratch[mat, 2, 1, nt, 1] <= 8
 
 
 def test_scratch_at_n8(tmp_path):
@@ -51,3 +54,11 @@ def test_scratch_at_n8(tmp_path):
         for nt in (0, 1):
             for feat in (0, 1, 2):
                 assert scratch[mat, 0, feat, nt, 1] == 0
+
+
+def test_scratch_of_kept_stages_at_n7(tmp_path):
+    scratch = _report(tmp_path, 8)
+    for mat in (0, 1):
+        for nt in (0, 1):
+            for feat in (0, 1):
+                assert scratch[mat, 2, feat, nt, 1] == 0
